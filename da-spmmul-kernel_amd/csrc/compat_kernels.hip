@@ -217,127 +217,205 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
 }
 
 // ===========================================================================
-// Nnz-balanced, sequential reduction, row-major (spmv_coo_scalar,
-// spmm_coo_scalar_row).  Each group of L lanes owns NE consecutive
-// nonzeros; the block's nonzeros (row, col, val) are staged in LDS (padded
-// so that groups reading their k-th element hit distinct banks).  A group
-// sums runs of equal row in order and atomically adds each finished run.
+// Nnz-balanced, row-major, nv > 1 (spmm_coo_scalar_row, spmm_coo_vector_row,
+// spmv_coo_vector with nv 2 or 4).  A wavefront owns G * NE consecutive
+// nonzeros, G = 64 / L, and stages their (row, col, val) in its own LDS
+// region with coalesced loads (one pad word per group, so that groups reading
+// their k-th element hit distinct banks).  A group of L lanes sums NE
+// consecutive ones in order, UNR gathers in flight, and adds every finished
+// run of equal row to C with atomics.  Runs that cross group borders are
+// joined first by a wave64 segmented scan over the groups' last runs, so that
+// a row costs one atomic addition per wavefront it lies in.
+//
+// What bounds it: the atomics, then the gathers.  L2 takes about 19 G
+// atomic accesses a second, one per 64-byte line that an instruction touches,
+// so a run is added with its columns contiguous over the lanes (through LDS
+// where a lane holds several columns), and runs are as long as the nonzeros
+// of a wavefront allow.  Both reference algorithms run this kernel: without
+// the join a row costs an atomic per group (64^3 27-point stencil, nv = 64:
+// 395 us against 279 with it, before the contiguous additions; 133 with both;
+// an atomic per eight nonzeros and four strided ones per float4 took 947 and
+// 1902 us).
 // ===========================================================================
 template <int VW, int L, int NE>
-__global__ __launch_bounds__(kBlock) void k_coo_scalar_rm(int nnz, int nv, int64_t ldb, int64_t ldc,
-                                                           const int *__restrict__ rowIdx,
-                                                           const int *__restrict__ colIdx,
-                                                           const float *__restrict__ values,
-                                                           const float *__restrict__ B,
-                                                           float *__restrict__ C, int slab_w) {
-    constexpr int GPB = kBlock / L;            // groups per block
-    constexpr int CH = GPB * NE;               // nonzeros per block
-    constexpr int PADN = CH + GPB;             // one pad word per group
-    __shared__ int s_row[PADN];
-    __shared__ int s_col[PADN];
-    __shared__ float s_val[PADN];
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int64_t base = (int64_t)b * CH;
+__global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc,
+                                                    const int *__restrict__ rowIdx,
+                                                    const int *__restrict__ colIdx,
+                                                    const float *__restrict__ values,
+                                                    const float *__restrict__ B,
+                                                    float *__restrict__ C, int slab_w) {
+    constexpr int G = kWave / L;               // groups per wavefront
+    constexpr int CH = G * NE;                 // nonzeros per wavefront
+    constexpr int PADN = CH + G;
+    constexpr int WPB = kBlock / kWave;
+    constexpr int UNR = NE < 8 ? NE : 8;
+    __shared__ int s_row[WPB][PADN];
+    __shared__ int s_col[WPB][PADN];
+    __shared__ float s_val[WPB][PADN];
+    __shared__ __align__(16) float s_flush[WPB][VW > 1 ? kWave * VW : 1];
+    const int wv = (int)threadIdx.x / kWave, ln = lane_id();
+    const int64_t base = ((int64_t)xcd_remap(blockIdx.x, gridDim.x) * WPB + wv) * CH;
+    if (base >= nnz) return;                   // the whole wavefront leaves; no barrier follows
     const int cnt = (int)min<int64_t>(CH, (int64_t)nnz - base);
-    for (int i = threadIdx.x; i < cnt; i += kBlock) {
+    // Non-temporal where the gathered rows of B want the caches (64^3 stencil,
+    // nv = 64: 132 us, plain loads 142); plain where the sparse operand is most
+    // of the traffic and may be resident (nv = 4: 34.8 us, 39.6).
+    constexpr bool NT = L >= 16;
+    for (int i = ln; i < cnt; i += kWave) {
         const int j = i + i / NE;
-        s_row[j] = ld_stream(rowIdx + base + i);
-        s_col[j] = ld_stream(colIdx + base + i);
-        s_val[j] = ld_stream(values + base + i);
+        const int64_t p = base + i;
+        s_row[wv][j] = NT ? ld_stream(rowIdx + p) : rowIdx[p];
+        s_col[wv][j] = NT ? ld_stream(colIdx + p) : colIdx[p];
+        s_val[wv][j] = NT ? ld_stream(values + p) : values[p];
     }
-    __syncthreads();
-    const int grp = threadIdx.x / L;
-    const int col0 = blockIdx.y * slab_w + ((int)threadIdx.x % L) * VW;
-    const int e0 = grp * NE, e1 = min(e0 + NE, cnt);
-    if (e0 >= e1 || col0 >= nv) return;
-    const int j0 = grp * (NE + 1);
-    int cur = s_row[j0];
-    float acc[VW];
-    {
-        float bv[VW];
-        load_vec<VW>(bv, B + (int64_t)s_col[j0] * ldb + col0);
-        const float a = s_val[j0];
+    wave_lds_sync();
+    const int g = ln / L;
+    const int col0 = blockIdx.y * slab_w + (ln % L) * VW;
+    const bool colok = col0 < nv;
+    const int n = max(0, min(NE, cnt - g * NE));   // nonzeros of this group
+    const int *sr = s_row[wv] + g * (NE + 1), *sc = s_col[wv] + g * (NE + 1);
+    const float *sv = s_val[wv] + g * (NE + 1);
+    const float *__restrict__ Bc = B + (colok ? col0 : 0);
+    // Adds v to row r of C.  An atomic instruction costs one L2 access per
+    // 64-byte line it touches, so the group's lanes trade their VW consecutive
+    // columns for columns L apart (through LDS) and each instruction covers L
+    // consecutive floats.
+    auto flush = [&](int r, const float (&v)[VW]) {
+        float *c = C + (int64_t)r * ldc + blockIdx.y * slab_w;
+        const int l = ln % L;
+        if constexpr (VW == 1) {
+            if (colok) unsafeAtomicAdd(c + l, v[0]);
+        } else {
+            float *f = s_flush[wv] + (ln - l) * VW;
+            wave_lds_sync();                   // the group's previous flush has been read
+            store_vec<VW>(f + l * VW, v);
+            wave_lds_sync();
+            const int ncol = nv - (int)blockIdx.y * slab_w;
 #pragma unroll
-        for (int k = 0; k < VW; k++) acc[k] = a * bv[k];
-    }
-    constexpr int UNR = 4;
-    int e = e0 + 1;
-    for (; e < e1; e += UNR) {
+            for (int k = 0; k < VW; k++)
+                if (k * L + l < ncol) unsafeAtomicAdd(c + k * L + l, f[k * L + l]);
+        }
+    };
+    int cur = INT_MAX, first = INT_MAX;        // rows of the running and of the first run
+    bool one = true;                           // a single run so far
+    float acc[VW], head[VW];
+#pragma unroll
+    for (int k = 0; k < VW; k++) acc[k] = head[k] = 0.f;
+    if (n > 0) cur = first = sr[0];
+    for (int e = 0; e < n; e += UNR) {
         float bv[UNR][VW];
 #pragma unroll
-        for (int u = 0; u < UNR; u++) {
-            const int j = j0 + (e + u - e0);
-            if (e + u < e1) load_vec<VW>(bv[u], B + (int64_t)s_col[j] * ldb + col0);
-        }
+        for (int u = 0; u < UNR; u++)          // padded with the last entry: no branch around loads
+            load_vec<VW>(bv[u], Bc + (int64_t)sc[min(e + u, n - 1)] * ldb);
+        // summed per block of UNR, the blocks' sums then in order: a run of 32
+        // rounds no worse than the scan over eight lanes that it replaces
+        float part[VW];
+#pragma unroll
+        for (int k = 0; k < VW; k++) part[k] = 0.f;
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
-            if (e + u < e1) {
-                const int j = j0 + (e + u - e0);
-                const int rr = s_row[j];
-                const float a = s_val[j];
-                if (rr != cur) {
-                    atomic_add_vec<VW>(C + (int64_t)cur * ldc + col0, acc);
+            if (e + u < n) {
+                const int r = sr[e + u];
+                const float a = sv[e + u];
+                if (r != cur) {
 #pragma unroll
-                    for (int k = 0; k < VW; k++) acc[k] = a * bv[u][k];
-                    cur = rr;
-                } else {
+                    for (int k = 0; k < VW; k++) acc[k] += part[k];
+                    if (one) {                 // the first run may continue the previous group's
 #pragma unroll
-                    for (int k = 0; k < VW; k++) acc[k] = acc[k] + a * bv[u][k];
+                        for (int k = 0; k < VW; k++) head[k] = acc[k];
+                        one = false;
+                    } else {
+                        flush(cur, acc);
+                    }
+                    cur = r;
+#pragma unroll
+                    for (int k = 0; k < VW; k++) acc[k] = part[k] = 0.f;
                 }
+#pragma unroll
+                for (int k = 0; k < VW; k++) part[k] = __builtin_fmaf(a, bv[u][k], part[k]);
             }
         }
+#pragma unroll
+        for (int k = 0; k < VW; k++) acc[k] += part[k];
     }
-    atomic_add_vec<VW>(C + (int64_t)cur * ldc + col0, acc);
+    if constexpr (L == kWave) {
+        if (n > 0) {
+            if (!one) flush(first, head);
+            flush(cur, acc);
+        }
+    } else {
+        // acc becomes the sum of the row's last runs up to this group: rows are
+        // sorted, so equal last rows mean that the groups between hold nothing else
+        segmented_scan<L, VW>(acc, cur);
+        const int prow = __shfl_up(cur, L);
+        const bool joins = ln >= L && prow == first;
+#pragma unroll
+        for (int k = 0; k < VW; k++) {
+            const float p = __shfl_up(acc[k], L);
+            if (joins && !one) head[k] += p;
+        }
+        if (n > 0 && !one) flush(first, head);
+        // the last group of a row's runs adds it (the next group's head takes it otherwise)
+        const int nfirst = __shfl_down(first, L);
+        const bool ends = ln >= kWave - L || nfirst != cur;
+        if (n > 0 && ends) flush(cur, acc);
+    }
 }
 
 // ===========================================================================
-// Nnz-balanced, parallel reduction, row-major (spmv_coo_vector,
-// spmm_coo_vector_row).  A wavefront takes G = 64/L consecutive nonzeros
-// per step, one per group; products are combined by row with a wave64
-// segmented scan (or a plain butterfly when the whole step is one row) and
-// the last group of each row segment adds it atomically.  Grid-strided.
+// Nnz-balanced, nv = 1 (spmv_coo_scalar, spmv_coo_vector).  A wavefront owns U
+// chunks of 64 consecutive nonzeros, one per lane: all U * 64 gathers of x are
+// issued, then each chunk is combined by row with the wave64 segmented scan
+// (or a butterfly when it is one row), the sum of a row that goes on in the
+// next chunk enters that chunk's first lane, and the last lane of each row
+// adds it to y.  Rows are adjacent in y, so one instruction's additions fall
+// in few lines.
 // ===========================================================================
-template <int VW, int L>
-__global__ __launch_bounds__(kBlock) void k_coo_vector_rm(int nnz, int nv, int64_t ldb, int64_t ldc,
-                                                           const int *__restrict__ rowIdx,
-                                                           const int *__restrict__ colIdx,
-                                                           const float *__restrict__ values,
-                                                           const float *__restrict__ B,
-                                                           float *__restrict__ C, int slab_w) {
-    constexpr int G = kWave / L;
+template <int U>
+__global__ __launch_bounds__(kBlock) void k_coo_spmv(int nnz, const int *__restrict__ rowIdx,
+                                                      const int *__restrict__ colIdx,
+                                                      const float *__restrict__ values,
+                                                      const float *__restrict__ x, int64_t ldx,
+                                                      float *__restrict__ y, int64_t ldy) {
     const int ln = lane_id();
-    const int g = ln / L;
-    const int wave = (xcd_remap(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) / kWave;
-    const int64_t nwaves = (int64_t)gridDim.x * (kBlock / kWave);
-    const int col0 = blockIdx.y * slab_w + (ln % L) * VW;
-    const bool colok = col0 < nv;
-    for (int64_t base = (int64_t)wave * G; base < nnz; base += nwaves * G) {
-        const int64_t p = base + g;
-        const bool valid = p < nnz;
-        int key = INT_MAX;
-        float v[VW];
+    const int64_t wave = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * (kBlock / kWave) +
+                         (int)threadIdx.x / kWave;
+    const int64_t base = wave * (U * kWave);   // plain loads below: non-temporal ones cost 4 us
+    if (base >= nnz) return;                   // the whole wavefront leaves
+    int key[U], c[U];
+    float v[U];
 #pragma unroll
-        for (int k = 0; k < VW; k++) v[k] = 0.f;
-        if (valid) {
-            key = rowIdx[p];
-            if (colok) {
-                const float a = values[p];
-                float bv[VW];
-                load_vec<VW>(bv, B + (int64_t)colIdx[p] * ldb + col0);
-#pragma unroll
-                for (int k = 0; k < VW; k++) v[k] = a * bv[k];
-            }
+    for (int u = 0; u < U; u++) {
+        const int64_t p = base + u * kWave + ln;
+        key[u] = INT_MAX;
+        c[u] = 0;
+        v[u] = 0.f;
+        if (p < nnz) {
+            key[u] = rowIdx[p];
+            c[u] = colIdx[p];
+            v[u] = values[p];
         }
-        const int kfirst = read_lane(key, 0), klast = read_lane(key, kWave - 1);
-        if (kfirst == klast) {
+    }
 #pragma unroll
-            for (int k = 0; k < VW; k++) v[k] = butterfly_sum<L, kWave>(v[k]);
-            if (g == 0 && colok) atomic_add_vec<VW>(C + (int64_t)key * ldc + col0, v);
-        } else {
-            segmented_scan<L, VW>(v, key);
-            const bool tail = valid && (g == G - 1 || p + 1 >= nnz || rowIdx[p + 1] != key);
-            if (tail && colok) atomic_add_vec<VW>(C + (int64_t)key * ldc + col0, v);
+    for (int u = 0; u < U; u++)
+        if (key[u] != INT_MAX) v[u] *= x[(int64_t)c[u] * ldx];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int kfirst = read_lane(key[u], 0), klast = read_lane(key[u], kWave - 1);
+        float s[1] = {v[u]};
+        if (kfirst == klast) s[0] = butterfly_sum<1, kWave>(s[0]);
+        else segmented_scan<1, 1>(s, key[u]);
+        int next = __shfl_down(key[u], 1);
+        if (ln == kWave - 1) next = INT_MAX;
+        if (u + 1 < U) {                       // a row that goes on: its sum joins the next chunk
+            const int nk = read_lane(key[u + 1 < U ? u + 1 : u], 0);
+            const float t = __shfl(s[0], kWave - 1);
+            if (nk == klast && ln == 0) v[u + 1 < U ? u + 1 : u] += t;
+            if (ln == kWave - 1) next = nk;
         }
+        if (key[u] != INT_MAX && next != key[u] &&
+            !(kfirst == klast && ln != kWave - 1))
+            unsafeAtomicAdd(y + (int64_t)key[u] * ldy, s[0]);
     }
 }
 
@@ -649,33 +727,65 @@ dspmm_status_t csr_vector_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
     return launch_status();
 }
 
-dspmm_status_t coo_scalar_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
-                             const int *colIdx, const float *values, const float *B, float *C,
-                             hipStream_t st) {
-    const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, 4));
-    with_vw(s.vw, [&](auto vw_c) {
-        with_lanes(s.lanes, [&](auto l_c) {
-            constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-            constexpr int CH = (kBlock / L_) * kCooNE;
-            dim3 grid(div_up(nnz, CH), s.count);
-            hipLaunchKernelGGL((k_coo_scalar_rm<VW_, L_, kCooNE>), grid, dim3(kBlock), 0, st, nnz,
-                               nv, ldb, ldc, rowIdx, colIdx, values, B, C, s.width);
-        });
-    });
+// Nonzeros per group of k_coo_rm (chunks per wavefront of k_coo_spmv): as many
+// as leave the launch at least kCooWaves wavefronts, 32 per CU, since fewer
+// runs are then cut; at most kCooPairs per wavefront, which its LDS holds.
+constexpr int64_t kCooWaves = 8192;
+constexpr int kCooPairs = 512;
+
+template <int VW, int L, int NE>
+void launch_coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx, const int *colIdx,
+                   const float *values, const float *B, float *C, hipStream_t st, const Slab &s) {
+    if constexpr (NE * (kWave / L) <= kCooPairs) {
+        dim3 grid(div_up(nnz, (int64_t)(kBlock / L) * NE), s.count);
+        hipLaunchKernelGGL((k_coo_rm<VW, L, NE>), grid, dim3(kBlock), 0, st, nnz, nv, ldb, ldc,
+                           rowIdx, colIdx, values, B, C, s.width);
+    }
+}
+
+template <int U>
+void launch_coo_spmv(int nnz, const int *rowIdx, const int *colIdx, const float *values,
+                     const float *x, int64_t ldx, float *y, int64_t ldy, hipStream_t st) {
+    hipLaunchKernelGGL((k_coo_spmv<U>), dim3(div_up(nnz, kBlock * U)), dim3(kBlock), 0, st, nnz,
+                       rowIdx, colIdx, values, x, ldx, y, ldy);
+}
+
+dspmm_status_t coo_spmv(int nnz, int64_t ldx, int64_t ldy, const int *rowIdx, const int *colIdx,
+                        const float *values, const float *x, float *y, hipStream_t st) {
+    // two chunks where that leaves kCooWaves wavefronts (power law, 3.2 M
+    // nonzeros: one 20.9, two 20.8, four 22.0 us; stencil, 6.9 M: 26.4, 22.9, 24.3)
+    if (nnz >= kCooWaves * kWave * 2)
+        launch_coo_spmv<2>(nnz, rowIdx, colIdx, values, x, ldx, y, ldy, st);
+    else
+        launch_coo_spmv<1>(nnz, rowIdx, colIdx, values, x, ldx, y, ldy, st);
     return launch_status();
 }
 
-dspmm_status_t coo_vector_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
-                             const int *colIdx, const float *values, const float *B, float *C,
-                             hipStream_t st) {
-    const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, 4));
+// ALG_COO_SCALAR and ALG_COO_VECTOR, row-major.
+dspmm_status_t coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
+                      const int *colIdx, const float *values, const float *B, float *C,
+                      hipStream_t st) {
+    if (nv == 1) return coo_spmv(nnz, ldb, ldc, rowIdx, colIdx, values, B, C, st);
+    // The widest vectors that leave a group 16 lanes, a 64-byte line of C per
+    // atomic instruction: at nv = 32 two floats (stencil 64^3 90 us, power law
+    // 75 us; four floats 93 and 88, one 128 and 78), at nv = 64 four
+    // (stencil 133 us; two 157, one 243).
+    const int widest = nv >= 64 ? 4 : nv >= 32 ? 2 : 1;
+    const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, widest));
+    int ne = 32;
+    while (ne > 8 && (ne * (kWave / s.lanes) > kCooPairs ||
+                      (int64_t)nnz * s.lanes * s.count < kCooWaves * kWave * ne))
+        ne /= 2;
     with_vw(s.vw, [&](auto vw_c) {
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-            constexpr int G = kWave / L_;
-            dim3 grid(grid_for_waves(((int64_t)nnz + G - 1) / G), s.count);
-            hipLaunchKernelGGL((k_coo_vector_rm<VW_, L_>), grid, dim3(kBlock), 0, st, nnz, nv, ldb,
-                               ldc, rowIdx, colIdx, values, B, C, s.width);
+            if constexpr (L_ >= (VW_ > 1 ? 16 : 2)) {
+                switch (ne) {
+                case 32: launch_coo_rm<VW_, L_, 32>(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st, s); break;
+                case 16: launch_coo_rm<VW_, L_, 16>(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st, s); break;
+                default: launch_coo_rm<VW_, L_, 8>(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st, s); break;
+                }
+            }
         });
     });
     return launch_status();
@@ -757,10 +867,9 @@ dspmm_status_t launch_compat(int which, int nr, int nc, int nnz, int nv, int64_t
         return csr_vector_rm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st, hint);
     case K_SPMV_COO_SCALAR:
     case K_SPMM_COO_SCALAR_ROW:
-        return coo_scalar_rm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
     case K_SPMV_COO_VECTOR:
     case K_SPMM_COO_VECTOR_ROW:
-        return coo_vector_rm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
+        return coo_rm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
     case K_SPMM_CSR_SCALAR_COL:
         return csr_scalar_cm(nr, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
     case K_SPMM_CSR_VECTOR_COL:

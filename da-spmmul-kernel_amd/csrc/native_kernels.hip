@@ -43,16 +43,6 @@ __host__ __device__ inline int wave_lds_ints(int G, int S) {
     return 2 * skew_h(G * S) + G * S + 1;
 }
 
-// Wavefront-level LDS ordering: every wavefront stages into and reads from
-// its own LDS region only, so a workgroup barrier is not needed between
-// staging and use -- the wavefront's LDS writes are made complete and
-// ordered before its reads.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 struct WaveStage {
     int P0, R0;
     int *s_col;

@@ -158,4 +158,14 @@ __device__ __forceinline__ int read_lane(int v, int src) {
     return __builtin_amdgcn_readlane(v, src);
 }
 
+// Wavefront-level LDS ordering: every wavefront stages into and reads from
+// its own LDS region only, so a workgroup barrier is not needed between
+// staging and use -- the wavefront's LDS writes are made complete and
+// ordered before its reads.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 }  // namespace dspmm
