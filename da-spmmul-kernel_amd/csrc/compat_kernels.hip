@@ -47,12 +47,19 @@ __device__ __forceinline__ void seq_accumulate(float (&acc)[VW], int p0, int p1,
             for (int k = 0; k < VW; k++) acc[k] = acc[k] + a * b[u][k];
         }
     }
-    for (; p < p1; p++) {
-        float b[VW];
-        load_b<TB, VW>(b, B + (int64_t)s_col[p - w] * ldb + col0);
-        const float a = s_val[p - w];
+    if (p < p1) {                               // the rest, loaded together
+        float b[UNR - 1][VW];
 #pragma unroll
-        for (int k = 0; k < VW; k++) acc[k] = acc[k] + a * b[k];
+        for (int u = 0; u < UNR - 1; u++)
+            if (p + u < p1) load_b<TB, VW>(b[u], B + (int64_t)s_col[p + u - w] * ldb + col0);
+#pragma unroll
+        for (int u = 0; u < UNR - 1; u++) {
+            if (p + u < p1) {
+                const float a = s_val[p + u - w];
+#pragma unroll
+                for (int k = 0; k < VW; k++) acc[k] = acc[k] + a * b[u][k];
+            }
+        }
     }
 }
 
@@ -60,17 +67,260 @@ __device__ __forceinline__ void seq_accumulate(float (&acc)[VW], int p0, int p1,
 __device__ __forceinline__ void stage_window(int *s_col, float *s_val, const int *__restrict__ colIdx,
                                              const float *__restrict__ values, int w, int cnt) {
     for (int i = threadIdx.x; i < cnt; i += kBlock) {
-        s_col[i] = ld_stream(colIdx + w + i);
-        s_val[i] = ld_stream(values + w + i);
+        s_col[i] = colIdx[w + i];
+        s_val[i] = values[w + i];
     }
 }
 
+// Rows that a block of k_csr_scalar_rm sums together, all its groups
+// gathering: at least kLongRow nonzeros and twice the block's mean row, so
+// that the row's own group would otherwise work on alone.
+constexpr int kLongRow = 96;
+// The longest rows (kScoutRow nonzeros or more) are found and summed by the
+// first blocks of the launch, each of which looks at kScoutRows rows and sums
+// kScoutCols of their columns: begun last, or with the gathers of one block
+// only, one of them would set the kernel's time.  On a power-law matrix
+// (262144 rows, the longest 4900, nv = 64): 32 columns 160 us, 16
+// (64-byte gathers) 192, without these blocks 203, with a lane group alone on
+// each row 660.
+constexpr int kScoutRow = 1024;
+constexpr int kScoutRows = 512;
+constexpr int kScoutCols = 32;
+__device__ __forceinline__ bool is_long_row(int len, int block_nnz, int block_rows) {
+    return len >= kLongRow && (int64_t)len * block_rows >= 2 * (int64_t)block_nnz;
+}
+
+// One row [p0, p1) summed by the whole block in nonzero order.  Per step the
+// groups multiply P nonzeros into LDS (P products of L * VW columns, two
+// steps' gathers in flight) and thread t < L * VW adds column t's products in
+// order; the (column, value) pairs go through LDS in chunks, loaded a chunk
+// ahead.  Returns column t's sum.  Every thread calls it (barriers
+// inside).
+template <int VW, int L, int U>
+struct LongRow {
+    static constexpr int W = L * VW;
+    static constexpr int P = kBlock / L * U;
+    static constexpr int PPT = P > kBlock / 4 ? 4 * P / kBlock : 1;   // pairs per thread and chunk
+    static constexpr int CHK = PPT * kBlock;                // pairs per chunk
+    static constexpr int kFloats = P * W + 4 * CHK;         // products, two chunks of pairs
+    static constexpr int S = CHK / P;                       // steps per chunk
+    static_assert(U >= 1 && S >= 4 && P % 16 == 0, "steps of 16 products, four to a chunk");
+
+    static __device__ __forceinline__ float sum(int p0, int p1, const int *__restrict__ colIdx,
+                                                const float *__restrict__ values,
+                                                const float *__restrict__ B, int64_t ldb, int col0,
+                                                bool colok, float *mem) {
+        const int t = threadIdx.x, g = t / L, l = t % L;
+        float *prod = mem;
+        int *s_c = reinterpret_cast<int *>(mem + P * W);
+        float *s_v = mem + P * W + 2 * CHK;
+        const float *__restrict__ Bc = B + (colok ? col0 : 0);
+        const int n = p1 - p0;
+        const int steps = (n + 2 * P - 1) / (2 * P) * 2;    // even: two register sets in turn
+        int nc[PPT];                                        // this thread's pairs of the next chunk
+        float nv[PPT];
+        auto load_pairs = [&](int j) {
+#pragma unroll
+            for (int x = 0; x < PPT; x++) {
+                const int q = p0 + min(j * CHK + x * kBlock + t, n - 1);
+                nc[x] = colIdx[q];
+                nv[x] = values[q];
+            }
+        };
+        auto put_pairs = [&](int j) {
+#pragma unroll
+            for (int x = 0; x < PPT; x++) {
+                s_c[(j & 1) * CHK + x * kBlock + t] = nc[x];
+                s_v[(j & 1) * CHK + x * kBlock + t] = nv[x];
+            }
+        };
+        float b[2][U][VW];
+        auto gather = [&](int k, float (&d)[U][VW]) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                load_vec<VW>(d[u], Bc + (int64_t)s_c[(k * P + g * U + u) % (2 * CHK)] * ldb);
+        };
+        float sum = 0.f;
+        auto step = [&](int k, float (&d)[U][VW]) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = k * P + g * U + u;
+                const float v = s_v[i % (2 * CHK)];
+                float m[VW];
+#pragma unroll
+                for (int q = 0; q < VW; q++)   // +0 past the end: a sum that began at +0 keeps its bits
+                    m[q] = i < n ? v * d[u][q] : 0.f;
+                store_vec<VW>(prod + (g * U + u) * W + l * VW, m);
+            }
+            gather(k + 2, d);
+            if ((k + 3) % S == 0) {            // the chunk that step k + 3 begins, read from step k + 1 on
+                put_pairs((k + 3) / S);
+                load_pairs((k + 3) / S + 1);
+            }
+            __syncthreads();
+            const int m = min(P, n - k * P);
+            if (t < W) {                       // H products read ahead of the H being added
+                                constexpr int H = 8;
+                const float *pr = prod + t;
+                float x[H], y[H];
+#pragma unroll
+                for (int j = 0; j < H; j++) x[j] = pr[j * W];
+                for (int i = 0; i < m; i += 2 * H) {
+#pragma unroll
+                    for (int j = 0; j < H; j++) y[j] = pr[(i + H + j) * W];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 0; j < H; j++) sum = sum + x[j];
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int nx = min(i + 2 * H, P - H);
+#pragma unroll
+                    for (int j = 0; j < H; j++) x[j] = pr[(nx + j) * W];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 0; j < H; j++) sum = sum + y[j];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __syncthreads();
+        };
+        load_pairs(0);
+        __syncthreads();                       // `mem` is free
+        put_pairs(0);
+        load_pairs(1);
+        __syncthreads();
+        gather(0, b[0]);
+        gather(1, b[1]);
+        for (int k = 0; k < steps; k += 2) {
+            step(k, b[0]);
+            step(k + 1, b[1]);
+        }
+        return sum;
+    }
+};
+
 // ===========================================================================
-// Row-balanced, sequential reduction, row-major (spmv_csr_scalar for nv=1,
-// spmm_csr_scalar_row for nv>1).  A group of L lanes owns one row; each lane
+// Row-balanced, sequential reduction, row-major, for few columns
+// (spmv_csr_scalar; spmm_csr_scalar_row with L * VW <= 8).  A wavefront owns
+// G consecutive rows, at most 64 / (L * VW).  In windows of PW of their pairs,
+// every lane gathers B for its share of the window at once, the next window's
+// while this one is added, and the products go to the wavefront's LDS region,
+// one column after another; then lane (row, column) adds its row's products
+// in nonzero order.  However long a row is, all 64 lanes gather for it.
+//
+// What bounds it: gather latency for short rows, the chain of additions for
+// long ones.  nv = 1, lanes that gathered their own rows before and now:
+// stencil 64^3 28.7 -> 15.9 us, 20000 rows of 100 82 -> 12 us, power law
+// (262144 rows, the longest 4900) 320 -> 61 us.
+// ===========================================================================
+// Pairs per window at W columns.
+constexpr int stream_pairs(int W) { return W == 1 ? 512 : W == 8 ? 128 : 256; }
+template <int VW, int L>
+__global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_t ldb, int64_t ldc,
+                                                           const int *__restrict__ rowPtr,
+                                                           const int *__restrict__ colIdx,
+                                                           const float *__restrict__ values,
+                                                           const float *__restrict__ B,
+                                                           float *__restrict__ C, int G) {
+    constexpr int W = L * VW, WPB = kBlock / kWave;
+    constexpr int PW = stream_pairs(W);
+    constexpr int E = PW * L / kWave;                             // gathers per lane and window
+    constexpr int LD = PW + 8;                                    // floats per column of products
+    __shared__ float s_prod[WPB][W * LD];
+    const int ln = lane_id(), wv = (int)threadIdx.x / kWave;
+    const int64_t rw = ((int64_t)xcd_remap(blockIdx.x, gridDim.x) * WPB + wv) * G;
+    if (rw >= nr) return;                      // the whole wavefront leaves; no barrier follows
+    const int c = ln % W;
+    const bool mine = ln / W < G && rw + ln / W < nr;
+    const int r = (int)min(rw + ln / W, (int64_t)nr);
+    const int start = rowPtr[r], end = mine ? rowPtr[r + 1] : start;
+    const int e0 = rowPtr[rw], e1 = rowPtr[min(rw + G, (int64_t)nr)];
+    const int gl = (ln % L) * VW;              // first column that this lane gathers
+    const float *__restrict__ Bc = B + (gl < nv ? gl : 0);
+    float *sp = s_prod[wv];
+    int cc[E];
+    float vv[E], b[E][VW];
+    auto gather = [&](int w) {
+#pragma unroll
+        for (int k = 0; k < E; k++) {
+            const int p = min(w + ln / L + k * (kWave / L), e1 - 1);
+            cc[k] = colIdx[p];
+            vv[k] = values[p];
+        }
+#pragma unroll
+        for (int k = 0; k < E; k++) load_vec<VW>(b[k], Bc + (int64_t)cc[k] * ldb);
+    };
+    float acc = 0.f;
+    if (e0 < e1) gather(e0);
+    for (int w = e0; w < e1; w += PW) {
+        wave_lds_sync();                       // the last window's products have been read
+#pragma unroll
+        for (int k = 0; k < E; k++) {
+            const int i = ln / L + k * (kWave / L);
+#pragma unroll
+            for (int q = 0; q < VW; q++)       // +0 past the end: a sum that began at +0 keeps its bits
+                sp[(gl + q) * LD + i] = w + i < e1 ? vv[k] * b[k][q] : 0.f;
+        }
+        if (w + PW < e1) gather(w + PW);
+        wave_lds_sync();
+        const int p0 = max(start, w) - w;
+        int n = min(end, w + PW) - w - p0;
+        // Long rows (of this window): 64 products at a time in the lanes of one
+        // register per column, and each lane adds its product to the sum that
+        // its lower neighbour hands up: 63 steps put the row's sum in order in
+        // lane 63.  (A lane that reads one product after the other from LDS
+        // took 66 cycles each.)
+        uint64_t longs = __ballot(c == 0 && n >= kWave);
+        if (__popcll(longs) > 4) longs = 0;    // as many lanes add their rows side by side
+        for (; longs; longs &= longs - 1) {
+            const int o = __builtin_ctzll(longs);          // the row's lane of column 0
+            const int q0 = read_lane(p0, o), qn = read_lane(n, o);
+            float sum[W];
+#pragma unroll
+            for (int q = 0; q < W; q++)
+                sum[q] = __int_as_float(read_lane(__float_as_int(acc), o + q));
+            for (int i = 0; i < qn; i += kWave) {
+                float x[W], y[W];
+#pragma unroll
+                for (int q = 0; q < W; q++) {
+                    const float v = sp[q * LD + min(q0 + i + ln, PW)];
+                    x[q] = i + ln < qn ? v : 0.f;
+                    if (ln == 0) x[q] = sum[q] + x[q];
+                    y[q] = x[q];
+                }
+#pragma unroll 9
+                for (int k = 0; k < kWave - 1; k++) {
+#pragma unroll
+                    for (int q = 0; q < W; q++) y[q] = dpp0_f<kDppWaveShr1>(y[q]) + x[q];
+                }
+#pragma unroll
+                for (int q = 0; q < W; q++)
+                    sum[q] = __int_as_float(read_lane(__float_as_int(y[q]), kWave - 1));
+            }
+#pragma unroll
+            for (int q = 0; q < W; q++)
+                if (ln == o + q) acc = sum[q];
+            if (ln / W == o / W) n = 0;
+        }
+        const float *pr = sp + c * LD + p0;
+        for (; n > 0; n -= 8, pr += 8) {       // reads past the row stay in the window's LDS
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = pr[u];
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc = acc + (u < n ? x[u] : 0.f);
+        }
+    }
+    if (mine && c < nv) __builtin_nontemporal_store(acc, C + (int64_t)r * ldc + c);
+}
+
+// ===========================================================================
+// Row-balanced, sequential reduction, row-major (spmm_csr_scalar_row with more
+// than 8 columns).  A group of L lanes owns one row; each lane
 // owns VW consecutive columns of the slab.  The block's rows' nonzeros are
 // staged through LDS in windows; every lane reads its row's (col, val) as an
 // LDS broadcast within its group.  Overwrites every row (empty rows -> 0).
+// Rows far longer than the block's others are summed by the whole block, the
+// longest ones by blocks of their own at the front of the grid (LongRow).
 // SLICED: a block whose rows overflow one window, and one of whose rows is
 // at least 4 shares of a window long (kWin / rows per block), splits each
 // window into one slice per row that still has nonzeros (kWin / n for n
@@ -85,13 +335,43 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
                                                            const int *__restrict__ colIdx,
                                                            const float *__restrict__ values,
                                                            const float *__restrict__ B,
-                                                           float *__restrict__ C, int slab_w) {
+                                                           float *__restrict__ C, int slab_w,
+                                                           int scouts) {
     constexpr int RPB = kBlock / L;
     constexpr int NW = kBlock / kWave;
-    __shared__ int s_col[kWin];
-    __shared__ float s_val[kWin];
+    using Long = LongRow<VW, L, (L >= 32 ? 4 : L >= 16 ? 2 : 1)>;
+    constexpr int SW = L * VW < kScoutCols ? L * VW : kScoutCols;
+    constexpr int SL = SW / VW;                // lanes of a scout's group
+    using Scout = LongRow<VW, SL, (SL >= 8 ? SL / 4 : SL / 2)>;
+    constexpr int kLds = Long::kFloats > 2 * kWin ? Long::kFloats : 2 * kWin;
+    static_assert(Scout::kFloats <= kLds, "LDS");
+    __shared__ __align__(16) float s_mem[kLds];
+    int *s_col = reinterpret_cast<int *>(s_mem);
+    float *s_val = s_mem + kWin;
+    __shared__ int s_long[RPB];                // rows that the block sums together
+    __shared__ uint16_t s_scout[kScoutRows];
+    __shared__ int s_nlong;
     __shared__ int s_tab[SLICED ? 2 * RPB + NW : 1];   // slice start, count per rank; per-wave counts
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    if ((int)blockIdx.x < scouts) {            // the longest rows first
+        const int parts = (min(slab_w, nv - (int)blockIdx.y * slab_w) + SW - 1) / SW;
+        const int q0 = (int)blockIdx.x / parts * kScoutRows, q1 = min(q0 + kScoutRows, nr);
+        if (threadIdx.x == 0) s_nlong = 0;
+        __syncthreads();
+        for (int q = q0 + (int)threadIdx.x; q < q1; q += kBlock)
+            if (rowPtr[q + 1] - rowPtr[q] >= kScoutRow) s_scout[atomicAdd(&s_nlong, 1)] = (uint16_t)(q - q0);
+        __syncthreads();
+        const int cb = blockIdx.y * slab_w + (int)blockIdx.x % parts * SW;
+        const int c0 = cb + ((int)threadIdx.x % SL) * VW;
+        for (int i = 0; i < s_nlong; i++) {
+            const int q = q0 + s_scout[i];
+            const float sum = Scout::sum(rowPtr[q], rowPtr[q + 1], colIdx, values, B, ldb, c0,
+                                         c0 < nv, s_mem);
+            if ((int)threadIdx.x < SW && cb + (int)threadIdx.x < nv)
+                C[(int64_t)q * ldc + cb + (int)threadIdx.x] = sum;
+        }
+        return;
+    }
+    const int b = xcd_remap(blockIdx.x - scouts, gridDim.x - scouts);
     const int r0 = b * RPB;
     const int r = r0 + (int)threadIdx.x / L;
     const int col0 = blockIdx.y * slab_w + ((int)threadIdx.x % L) * VW;
@@ -103,6 +383,28 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
     float acc[VW];
 #pragma unroll
     for (int k = 0; k < VW; k++) acc[k] = 0.f;
+    // Rows that this block's groups sum together, or the scouts do.
+    auto apart = [&](int len) {
+        return is_long_row(len, be - bs, rlast - r0) || len >= kScoutRow;
+    };
+    int nlong = 0;
+    if (be - bs >= kLongRow) {                 // the same in every thread
+        if (threadIdx.x == 0) s_nlong = 0;
+        __syncthreads();
+        if (threadIdx.x % L == 0 && apart(end - start)) s_long[atomicAdd(&s_nlong, 1)] = r;
+        __syncthreads();
+        nlong = s_nlong;
+        for (int i = 0; i < nlong; i++) {
+            const int q = s_long[i], p0 = rowPtr[q], p1 = rowPtr[q + 1];
+            if (p1 - p0 >= kScoutRow) continue;
+            const float sum = Long::sum(p0, p1, colIdx, values, B, ldb, col0, colok, s_mem);
+            const int c = blockIdx.y * slab_w + (int)threadIdx.x;
+            if ((int)threadIdx.x < L * VW && c < nv)
+                __builtin_nontemporal_store(sum, C + (int64_t)q * ldc + c);
+        }
+    }
+    const bool mine = nlong == 0 || !apart(end - start);
+    if (!mine) end = start;                    // done
     bool slice = false;
     if constexpr (SLICED) {
         // slices pay where a row is long against its share of a window (kWin /
@@ -121,6 +423,11 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
     }
     if (!slice) {
         for (int w = bs; w < be; w += kWin) {
+            for (int i = 0; i < nlong; i++) {  // no window starts inside a row that is done
+                const int q = s_long[i];
+                if (w >= rowPtr[q] && w < rowPtr[q + 1]) { w = rowPtr[q + 1]; i = -1; }
+            }
+            if (w >= be) break;
             const int cnt = min(kWin, be - w);
             __syncthreads();
             stage_window(s_col, s_val, colIdx, values, w, cnt);
@@ -160,8 +467,8 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
             for (int i = threadIdx.x; i < (nact << lsl); i += kBlock) {
                 const int q = i >> lsl, o = i & ((1 << lsl) - 1);
                 if (o < tab_c[q]) {
-                    s_col[i] = ld_stream(colIdx + tab_s[q] + o);
-                    s_val[i] = ld_stream(values + tab_s[q] + o);
+                    s_col[i] = colIdx[tab_s[q] + o];
+                    s_val[i] = values[tab_s[q] + o];
                 }
             }
             __syncthreads();
@@ -172,7 +479,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
             __syncthreads();                              // before the next window's tables
         }
     }
-    if (r < nr && colok) store_vec_nt<VW>(C + (int64_t)r * ldc + col0, acc);
+    if (r < nr && colok && mine) store_vec_nt<VW>(C + (int64_t)r * ldc + col0, acc);
 }
 
 // ===========================================================================
@@ -673,10 +980,33 @@ void with_vw(int vw, F &&f) {
     }
 }
 
+// Rows per wavefront of k_csr_stream_rm: most of a window of pairs, at most one
+// row per lane and column.  Fewer pairs leave gathers unused (64^3 stencil,
+// nv = 4: half a window 26.6 us, 3/4 18.6, one 16.1), more make a long row's
+// wavefront later (power law, nv = 1: 60, 61, 83).
+int stream_rows(int W, int nnz, int nr) {
+    const double mean = std::max(1.0, (double)nnz / nr);
+    return std::max(1, std::min(kWave / W, (int)(0.75 * stream_pairs(W) / mean)));
+}
+
 dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st) {
     const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, 4));
+    if (s.width <= 8) {
+        with_vw(s.vw, [&](auto vw_c) {
+            with_lanes(s.lanes, [&](auto l_c) {
+                constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
+                if constexpr (VW_ * L_ <= 8) {
+                    const int g = stream_rows(VW_ * L_, nnz, nr);
+                    hipLaunchKernelGGL((k_csr_stream_rm<VW_, L_>), dim3(div_up(nr, (int64_t)g * (kBlock / kWave))),
+                                       dim3(kBlock), 0, st, nr, nv, ldb, ldc, rowPtr, colIdx, values,
+                                       B, C, g);
+                }
+            });
+        });
+        return launch_status();
+    }
     // sliced windows where a block's rows typically fill more than half a
     // window (the mean row length decides; a block that fits one window
     // runs the same code in both forms)
@@ -684,13 +1014,19 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
     with_vw(s.vw, [&](auto vw_c) {
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-            dim3 grid(div_up(nr, kBlock / L_), s.count);
-            if (sliced)
-                hipLaunchKernelGGL((k_csr_scalar_rm<VW_, L_, true>), grid, dim3(kBlock), 0, st, nr,
-                                   nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width);
-            else
-                hipLaunchKernelGGL((k_csr_scalar_rm<VW_, L_, false>), grid, dim3(kBlock), 0, st, nr,
-                                   nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width);
+            if constexpr (VW_ * L_ > 8) {
+                // scouts: one per kScoutRows rows and kScoutCols columns; a whole
+                // number per XCD, which leaves xcd_remap its meaning
+                const int parts = div_up(std::min(nv, s.width), std::min(s.width, kScoutCols));
+                const int scouts = div_up((int64_t)div_up(nr, kScoutRows) * parts, kNumXcd) * kNumXcd;
+                dim3 grid(scouts + div_up(nr, kBlock / L_), s.count);
+                if (sliced)
+                    hipLaunchKernelGGL((k_csr_scalar_rm<VW_, L_, true>), grid, dim3(kBlock), 0, st, nr,
+                                       nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width, scouts);
+                else
+                    hipLaunchKernelGGL((k_csr_scalar_rm<VW_, L_, false>), grid, dim3(kBlock), 0, st, nr,
+                                       nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width, scouts);
+            }
         });
     });
     return launch_status();

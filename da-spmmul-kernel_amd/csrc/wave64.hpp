@@ -27,6 +27,7 @@ constexpr int kDppQuadXor2 = 0x4E;   // quad_perm:[2,3,0,1]  -> lane ^ 2
 constexpr int kDppRowRor8 = 0x128;   // row_ror:8            -> lane ^ 8 within a row
 constexpr int dpp_row_shr(int n) { return 0x110 + n; }   // row_shr:n (1..15)
 
+constexpr int kDppWaveShr1 = 0x138;  // wave_shr:1           -> lane - 1
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int old, int v) {
     return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xF, 0xF, false);
@@ -35,6 +36,12 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_f(float old, float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v),
                                                       CTRL, 0xF, 0xF, false));
+}
+
+// The same with 0 in the lanes that have no source (foldable into the add).
+template <int CTRL>
+__device__ __forceinline__ float dpp0_f(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
 // ds_swizzle in bitmask mode: within each 32-lane half, lane i reads lane

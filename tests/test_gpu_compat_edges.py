@@ -64,3 +64,44 @@ def test_coo_row_major_large():
     c = int_case("large", lens, 5000, 64)
     for nv in (1, 2, 32, 64):
         check(c, "spmm_coo_vector_row", nv)
+
+
+def float_case(name, lens, nc, maxnv, seed=6):
+    rng = np.random.default_rng(seed)
+    rp = np.concatenate([[0], np.cumsum(np.asarray(lens, np.int64))])
+    n = int(rp[-1])
+    return Case(name, len(lens), nc, rp, rng.integers(0, nc, n),
+                rng.standard_normal(n).astype(np.float32), maxnv,
+                B=rng.uniform(-1, 1, nc * maxnv).astype(np.float32))
+
+
+def row_lengths(kind):
+    rng = np.random.default_rng(11)
+    if kind == "uniform_100":          # every row long against a window, none against the others
+        return np.full(700, 100)
+    if kind == "tiny":
+        return np.array([1, 0, 70, 0, 2])
+    lens = rng.integers(0, 12, 1300)   # three scouts' worth of rows
+    if kind == "one_long":
+        lens[5] = 5003
+    elif kind == "many_long":
+        at = rng.choice(1300, 40, replace=False)
+        lens[at] = np.resize([95, 96, 97, 191, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 1279,
+                              1281, 2048, 63, 64, 65, 128], 40)
+        lens[[0, 511, 512, 1299]] = 1100
+    return lens
+
+
+@pytest.mark.parametrize("kind", ["tiny", "uniform_100", "one_long", "many_long"])
+def test_csr_scalar_long_rows_bit_exact(kind):
+    """Rows summed by a lane, a group, a whole block and a scout equal the host
+    loop bit for bit, whatever the number of columns."""
+    c = float_case(kind, row_lengths(kind), 3000, 260)
+    for nv in (1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 48, 64, 100, 128, 256, 260):
+        name = "spmm_csr_scalar_row"
+        note(f"{kind} {name} nv={nv}")
+        c.fill_output(np.nan)
+        st = D.launch(name, c.nr, c.nc, c.nnz, nv, c.d_rp, c.d_ri, c.d_ci, c.d_v, c.d_B, c.d_C)
+        assert st == 0, D.status_string(st)
+        D.synchronize()
+        assert_bitwise(c.output(nv), c.ref(D.DENSE_ROW_MAJOR, nv)[0], f"{kind} nv={nv}")
