@@ -50,6 +50,18 @@ struct RingPlan {
     bool usable = false;     // false: a tile needs more B rows than the ring holds
 };
 
+// A diagonal-slice plan (k_spmv_diag) on the device.
+struct DiagPlan {
+    void *d_mem = nullptr;           // the one allocation that the arrays lie in
+    int *d_off = nullptr, *d_diags = nullptr;
+    float4 *d_vals = nullptr;
+    uint32_t *d_didx = nullptr;
+    int nslices = 0;
+    size_t bytes = 0;
+    bool known = false;              // the matrix has been looked at
+    bool usable = false;
+};
+
 // LDS budget of one nnz-tiled workgroup (keeps two workgroups per CU).
 constexpr size_t kMaxTileLds = 64 * 1024;
 
@@ -59,6 +71,9 @@ void build_tiles(const std::vector<int> &rp, int nr, int S, std::vector<int4> &t
 // long; a longer row gets its own tile(s) of <= T nonzeros.
 void build_spmv_tiles(const std::vector<int> &rp, int nr, int T, int row_max,
                       std::vector<int4> &tiles, std::vector<int4> &splits, int &nslots);
+
+bool build_diag_slices(const std::vector<int> &rp, const std::vector<int> &ci, int nr,
+                       std::vector<int> &diags, std::vector<int> &off);
 
 // Column-cached plan: tiles of whole rows with at most umax distinct columns,
 // at most smax nonzeros and kCachedRowsMax rows; a row that does not fit alone
@@ -102,6 +117,7 @@ struct dspmm_matrix_s {
     int rb_stride2 = -1;     // the best distance below it that divides it (1: none)
     // ring plans by (w, h, tiles per stream)
     std::map<std::tuple<int, int, int>, dspmm::RingPlan> ring_plans;
+    dspmm::DiagPlan diag;
     // tiles per stream chosen for tile shape (w, h) when the config leaves it to the library
     std::map<std::pair<int, int>, int> ring_auto;
     std::map<std::tuple<int, int, int>, dspmm_config> tuned;       // (layout, nv, btype)
@@ -112,7 +128,7 @@ struct dspmm_matrix_s {
     size_t tbuf_bytes = 0;
 
     size_t hbm_bytes() {
-        size_t b = base_bytes + carry_bytes + tbuf_bytes;
+        size_t b = base_bytes + carry_bytes + tbuf_bytes + diag.bytes;
         if (rowIdx) b += sizeof(int) * (size_t)nnz;
         for (auto &kv : plans) b += kv.second.bytes;
         for (auto &kv : ring_plans) b += kv.second.bytes;
@@ -143,6 +159,10 @@ int shared_row_stride2(dspmm_matrix_s *A);
 // on first use (build == false: DSPMM_STATUS_NOT_PREPARED if missing).
 dspmm_status_t get_ring_plan(dspmm_matrix_s *A, int w, int h, int zchunk, RingPlan **out,
                              bool build = true);
+// The matrix's diagonal-slice plan, looked for and built on first use
+// (build == false: DSPMM_STATUS_NOT_PREPARED if it was not); *out is NULL for
+// a matrix that has none.
+dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build = true);
 // The plan's shape for tile w x h (one row distance: w * h consecutive rows
 // per tile, walked along that distance).  Reads the sampled row distances.
 RingShape ring_shape(dspmm_matrix_s *A, int w, int h, int zchunk);

@@ -129,6 +129,32 @@ dspmm_status_t launch_nnz_tiled_batched(const BatchLaunch &a, hipStream_t st);
 // SpMV (nv == 1) tiles: item.S is the tile size T, item.tiles a plan made
 // by build_spmv_tiles.
 dspmm_status_t launch_spmv_tiled(const NbLaunch &a, hipStream_t st);
+// SpMV of a matrix whose nonzeros lie on at most kDiagMax diagonals (grid
+// stencils, banded matrices).  Rows are cut in slices of kDiagRows; a slice
+// stores its rows side by side, padded to its longest row rounded up to four:
+// group g of slice s (off[s] <= g < off[s + 1]) holds four nonzeros of each
+// row, vals[g * kDiagRows + lane] and, one byte each, their diagonals'
+// positions in `diags` (column minus row, ascending), didx[g * kDiagRows + lane].
+struct SpmvDiagLaunch {
+    const int *off = nullptr;
+    const float4 *vals = nullptr;
+    const uint32_t *didx = nullptr;
+    const int *diags = nullptr;        // kDiagMax entries
+    const int *rowPtr = nullptr;
+    const void *x = nullptr;
+    float *y = nullptr;
+    int64_t ldx = 1, ldy = 1;
+    int nr = 0, nslices = 0;
+    bool bf16 = false;
+};
+constexpr int kDiagRows = 64;      // a wavefront's lanes
+constexpr int kDiagMax = 256;
+constexpr double kDiagPad = 1.25;
+dspmm_status_t launch_spmv_diag(const SpmvDiagLaunch &a, hipStream_t st);
+// Fills vals and didx of the slices from the device CSR arrays.
+dspmm_status_t launch_diag_fill(const int *off, const int *diags, int ndiags, const int *rowPtr,
+                                const int *colIdx, const float *values, int nr, int nslices,
+                                float4 *vals, uint32_t *didx, hipStream_t st);
 constexpr int kSpmvRowMax = 256;   // longest row of a multi-row SpMV tile
 constexpr int kSpmvThreadRow = 16; // longest row summed by one thread
 constexpr int kSpmvLongTiles = 16; // rows up to 16 T nonzeros get one workgroup

@@ -384,8 +384,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
             c[k] = 0;
             a[k] = 0.f;
             if (i < n) {
-                c[k] = ld_stream(ci + i);
-                a[k] = ld_stream(va + i);
+                c[k] = ci[i];
+                a[k] = va[i];
             }
         }
 #pragma unroll
@@ -425,8 +425,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
         float a[4], xv[4][1];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            c[k] = ld_stream(ci + i + k * kBlock);
-            a[k] = ld_stream(va + i + k * kBlock);
+            c[k] = ci[i + k * kBlock];
+            a[k] = va[i + k * kBlock];
         }
 #pragma unroll
         for (int k = 0; k < 4; k++) load_b<TB, 1>(xv[k], x + (int64_t)c[k] * d.ldb);
@@ -435,8 +435,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
     }
     for (; i < n; i += kBlock) {
         float xv[1];
-        load_b<TB, 1>(xv, x + (int64_t)ld_stream(ci + i) * d.ldb);
-        s = s + ld_stream(va + i) * xv[0];
+        load_b<TB, 1>(xv, x + (int64_t)ci[i] * d.ldb);
+        s = s + va[i] * xv[0];
     }
     red[t] = s;
     __syncthreads();
@@ -447,6 +447,105 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
     if (t == 0) {
         if (tile.y < 0) d.carry[(int64_t)(-1 - tile.y) * d.ldcarry] = red[0];
         else d.C[(int64_t)tile.x * d.ldc] = red[0];
+    }
+}
+
+// ---- SpMV on diagonal slices ------------------------------------------------
+// One wavefront per slice, lane = row (layout: SpmvDiagLaunch).  The CSR kernel
+// reads 8 bytes per nonzero and gathers x from scattered lines; here a
+// nonzero takes 5 bytes, read 16 + 4 per lane and group, and the lanes'
+// x are neighbours, since neighbouring rows share their diagonals.  Rows of at
+// most kSpmvThreadRow nonzeros are summed in order with a rounded multiply and
+// add -- the host loop's bits -- and longer ones in four interleaved FMA sums,
+// whose rounding is no worse than the 64-lane tree's.
+// What bounds it: reading the slices.
+template <typename TB, bool UNIT>
+__global__ __launch_bounds__(kBlock) void k_spmv_diag(SpmvDiagLaunch a) {
+    __shared__ int s_diag[kDiagMax];
+    for (int i = threadIdx.x; i < kDiagMax; i += kBlock) s_diag[i] = a.diags[i];
+    __syncthreads();
+    const int ln = lane_id();
+    const int s = xcd_remap(blockIdx.x, gridDim.x) * (kBlock / kWave) + (int)threadIdx.x / kWave;
+    if (s >= a.nslices) return;                  // whole wavefronts leave; no barrier follows
+    const int r = s * kDiagRows + ln;
+    int len = 0;
+    if (r < a.nr) len = a.rowPtr[r + 1] - a.rowPtr[r];
+    const int g0 = a.off[s], g1 = a.off[s + 1];
+    const TB *__restrict__ x = reinterpret_cast<const TB *>(a.x);
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    float seq = 0.f;
+    const bool any_short = __ballot(len <= kSpmvThreadRow) != 0;
+    auto group = [&](int g, bool first) {        // first: within the first kSpmvThreadRow nonzeros
+        const uint32_t d = a.didx[(int64_t)g * kDiagRows + ln];
+        const float4 v4 = a.vals[(int64_t)g * kDiagRows + ln];
+        const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+        float xv[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const bool has = 4 * (g - g0) + k < len;
+            const int c = has ? r + s_diag[(d >> (8 * k)) & 255u] : 0;
+            float t[1];
+            load_b<TB, 1>(t, UNIT ? x + c : x + (int64_t)c * a.ldx);
+            xv[k] = has ? t[0] : 0.f;            // padding adds +0, whatever x holds
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[k] = __builtin_fmaf(v[k], xv[k], acc[k]);
+        if (first) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) seq = seq + v[k] * xv[k];
+        }
+    };
+    int g = g0;
+    if (any_short) {
+        const int ge = min(g1, g0 + kSpmvThreadRow / 4);
+        for (; g < ge; g++) group(g, true);
+    }
+#pragma unroll 4
+    for (; g < g1; g++) group(g, false);
+    if (r < a.nr)
+        a.y[UNIT ? (int64_t)r : (int64_t)r * a.ldy] =
+            len <= kSpmvThreadRow ? seq : (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
+
+// One wavefront per slice, lane = row; a nonzero's diagonal by binary search.
+__global__ __launch_bounds__(kBlock) void k_diag_fill(const int *__restrict__ off,
+                                                      const int *__restrict__ diags, int ndiags,
+                                                      const int *__restrict__ rowPtr,
+                                                      const int *__restrict__ colIdx,
+                                                      const float *__restrict__ values, int nr,
+                                                      int nslices, float4 *__restrict__ vals,
+                                                      uint32_t *__restrict__ didx) {
+    __shared__ int s_diag[kDiagMax];
+    for (int i = threadIdx.x; i < kDiagMax; i += kBlock) s_diag[i] = diags[i];
+    __syncthreads();
+    const int ln = lane_id();
+    const int s = (int)blockIdx.x * (kBlock / kWave) + (int)threadIdx.x / kWave;
+    if (s >= nslices) return;
+    const int r = s * kDiagRows + ln;
+    int p0 = 0, len = 0;
+    if (r < nr) {
+        p0 = rowPtr[r];
+        len = rowPtr[r + 1] - p0;
+    }
+    for (int g = off[s]; g < off[s + 1]; g++) {
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+        uint32_t d = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int q = 4 * (g - off[s]) + k;
+            if (q < len) {
+                const int dist = colIdx[p0 + q] - r;
+                v[k] = values[p0 + q];
+                int lo = 0, hi = ndiags - 1;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (s_diag[mid] < dist) lo = mid + 1; else hi = mid;
+                }
+                d |= (uint32_t)lo << (8 * k);
+            }
+        }
+        vals[(int64_t)g * kDiagRows + ln] = make_float4(v[0], v[1], v[2], v[3]);
+        didx[(int64_t)g * kDiagRows + ln] = d;
     }
 }
 
@@ -857,6 +956,29 @@ dspmm_status_t launch_spmv_e(const NbLaunch &a, hipStream_t st) {
     return launch_status();
 }
 }  // namespace
+
+dspmm_status_t launch_spmv_diag(const SpmvDiagLaunch &a, hipStream_t st) {
+    if (a.nslices == 0) return DSPMM_STATUS_SUCCESS;
+    const dim3 g(div_up(a.nslices, kBlock / kWave)), b(kBlock);
+    const bool unit = a.ldx == 1 && a.ldy == 1;
+    if (a.bf16) {
+        if (unit) hipLaunchKernelGGL((k_spmv_diag<uint16_t, true>), g, b, 0, st, a);
+        else hipLaunchKernelGGL((k_spmv_diag<uint16_t, false>), g, b, 0, st, a);
+    } else {
+        if (unit) hipLaunchKernelGGL((k_spmv_diag<float, true>), g, b, 0, st, a);
+        else hipLaunchKernelGGL((k_spmv_diag<float, false>), g, b, 0, st, a);
+    }
+    return launch_status();
+}
+
+dspmm_status_t launch_diag_fill(const int *off, const int *diags, int ndiags, const int *rowPtr,
+                                const int *colIdx, const float *values, int nr, int nslices,
+                                float4 *vals, uint32_t *didx, hipStream_t st) {
+    if (nslices == 0) return DSPMM_STATUS_SUCCESS;
+    hipLaunchKernelGGL(k_diag_fill, dim3(div_up(nslices, kBlock / kWave)), dim3(kBlock), 0, st, off,
+                       diags, ndiags, rowPtr, colIdx, values, nr, nslices, vals, didx);
+    return launch_status();
+}
 
 size_t nnz_cached_lds_bytes(int umax, int smax, int nv, int vw, bool bf16) {
     const size_t ls = (size_t)cached_stride(nv, vw);

@@ -1,6 +1,6 @@
 // tile_plans.cpp -- host-side plans of the native kernels (no device code,
 // no runtime calls): nnz tiles with split rows (k_nnz_tiled), SpMV tiles
-// (k_spmv_tiled), column-cached tiles (k_nnz_cached) and strided row blocks
+// (k_spmv_tiled) and diagonal slices (k_spmv_diag), column-cached tiles (k_nnz_cached) and strided row blocks
 // (k_row_blocked).  api_native.cpp uploads them.
 #include <hip/hip_runtime.h>
 
@@ -184,6 +184,54 @@ bool build_row_blocks(const std::vector<int> &rp, const std::vector<int> &ci,
             list.push_back(make_int2(c, mask));
         }
         boff[(size_t)b + 1] = (int)list.size();
+    }
+    return true;
+}
+
+// The distinct column-minus-row distances, ascending, and the slices' offsets
+// (see SpmvDiagLaunch); false if there are more than kDiagMax, or if padding
+// the slices would store more than kDiagPad times the nonzeros.
+bool build_diag_slices(const std::vector<int> &rp, const std::vector<int> &ci, int nr,
+                       std::vector<int> &diags, std::vector<int> &off) {
+    diags.clear();
+    const int nslices = (int)(((int64_t)nr + kDiagRows - 1) / kDiagRows);
+    off.assign((size_t)nslices + 1, 0);
+    int64_t groups = 0;
+    for (int s = 0; s < nslices; s++) {
+        int longest = 0;
+        const int r1 = (int)std::min<int64_t>(nr, ((int64_t)s + 1) * kDiagRows);
+        for (int r = s * kDiagRows; r < r1; r++)
+            longest = std::max(longest, rp[(size_t)r + 1] - rp[(size_t)r]);
+        groups += (longest + 3) / 4;
+        if (groups * (4 * kDiagRows) > INT_MAX) return false;
+        off[(size_t)s + 1] = (int)groups;
+    }
+    const int64_t nnz = rp[(size_t)nr];
+    if (nnz == 0 || (double)groups * (4 * kDiagRows) > kDiagPad * (double)nnz + 4 * kDiagRows)
+        return false;
+    // most rows of such a matrix repeat the distances of the row before
+    const int *prev = nullptr;
+    int64_t prev_shift = 0;
+    int prev_len = -1;
+    for (int r = 0; r < nr; r++) {
+        const int *c = ci.data() + rp[(size_t)r];
+        const int len = rp[(size_t)r + 1] - rp[(size_t)r];
+        if (len == prev_len) {
+            const int shift = (int)(r - prev_shift);
+            int differ = 0;
+            for (int k = 0; k < len; k++) differ |= (c[k] - shift) ^ prev[k];
+            if (!differ) continue;
+        }
+        prev = c;
+        prev_shift = r;
+        prev_len = len;
+        for (int k = 0; k < len; k++) {
+            const int d = c[k] - r;
+            const auto it = std::lower_bound(diags.begin(), diags.end(), d);
+            if (it != diags.end() && *it == d) continue;
+            if ((int)diags.size() == kDiagMax) return false;
+            diags.insert(it, d);
+        }
     }
     return true;
 }

@@ -263,7 +263,12 @@ typedef enum dspmm_variant {
     DSPMM_VARIANT_COO_VECTOR = 5,
     DSPMM_VARIANT_SPMV_TILED = 6,/* nv == 1 only: workgroup per nnz tile, products
                                     in LDS, per-row sums (row-exact), tree for
-                                    long rows; tile_nnz = tile size */
+                                    long rows; tile_nnz = tile size.  A matrix
+                                    whose nonzeros lie on at most 256 diagonals
+                                    is stored as slices of 64 rows instead
+                                    (5 bytes a nonzero); rows of at most 16
+                                    nonzeros are summed like the host loop in
+                                    both */
     DSPMM_VARIANT_NNZ_CACHED = 7,/* row-major, lanes * vec >= nv: tiles of whole
                                     rows whose distinct columns' B rows are
                                     staged in LDS once per tile (matrices whose
