@@ -26,7 +26,7 @@ dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc
     // the batch slower, not faster.
     dspmm_config c{};
     c.variant = DSPMM_VARIANT_NNZ_TILED;
-    complete_nb(c, nv, ldb, ldc, B, C, bf16);
+    complete_nb(c, nv, bf16);
     if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) {
         c.tile_nnz = 16;
         if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) return DSPMM_STATUS_NOT_SUPPORTED;
@@ -101,6 +101,7 @@ struct dspmm_batch_s {
     float *carry = nullptr;
     size_t carry_bytes = 0;
     size_t table_bytes = 0;
+    std::vector<int> align_vw;       // per item: floats that its operands' alignment was a multiple of
     int nblocks = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -189,6 +190,10 @@ dspmm_status_t dspmm_batch_create(dspmm_batch_t *out, const dspmm_batch_item *it
         free_batch(b);
         return st;
     }
+    for (const dspmm_batch_item &it : b->items)
+        b->align_vw.push_back(choose_vw(it.nv, it.ldb, it.ldc, it.B, it.C,
+                                        btype == DSPMM_R_16BF ? 2 : 4,
+                                        btype == DSPMM_R_16BF ? 8 : 4));
     b->nblocks = schedule_blocks(b->sch, blocks_per_cu);
     if (b->sch.carry_floats > 0) {
         b->carry_bytes = sizeof(float) * (size_t)b->sch.carry_floats;
@@ -276,9 +281,8 @@ dspmm_status_t dspmm_batch_set_operands(dspmm_batch_t b, int index, const void *
     if (!b || index < 0 || index >= b->count) return DSPMM_STATUS_INVALID_VALUE;
     dspmm_batch_item &it = b->items[(size_t)index];
     if ((it.A->nnz > 0 && !B) || (it.A->nr > 0 && !C)) return DSPMM_STATUS_INVALID_VALUE;
-    const dspmm_config &c = b->sch.cfg[(size_t)index];
-    const int eb = b->btype == DSPMM_R_16BF ? 2 : 4;
-    if (!aligned(B, c.vec * eb) || !aligned(C, c.vec * 4)) return DSPMM_STATUS_NOT_SUPPORTED;
+    const int eb = b->btype == DSPMM_R_16BF ? 2 : 4, vw = b->align_vw[(size_t)index];
+    if (!aligned(B, vw * eb) || !aligned(C, vw * 4)) return DSPMM_STATUS_NOT_SUPPORTED;
     it.B = B;
     it.C = C;
     ItemDesc &d = b->sch.items[(size_t)index];

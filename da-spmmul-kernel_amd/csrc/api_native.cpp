@@ -447,17 +447,24 @@ int64_t carry_ld(int nv) { return ((int64_t)nv + 7) / 8 * 8; }
 
 int default_tile(int lanes) { return std::max(16, std::min(256, 16 * lanes)); }
 
-// Fills unset fields of an NNZ_TILED config for these operands.
-void complete_nb(dspmm_config &c, int nv, int64_t ldb, int64_t ldc, const void *B, const void *C,
-                 bool bf16) {
-    const int eb = bf16 ? 2 : 4;
-    const int maxvw = bf16 ? 8 : 4;
-    const int auto_vw = choose_vw(nv, ldb, ldc, B, C, eb, maxvw);
+// Unset fields of a configuration whose vectors may be auto_vw wide.
+static void complete_vw(dspmm_config &c, int nv, int auto_vw) {
     if (c.vec <= 0 || c.vec > auto_vw || (auto_vw % c.vec) != 0) c.vec = auto_vw;
     const int need = pow2_ceil(div_up(nv, c.vec));
     if (c.lanes <= 0 || c.lanes > 64 || (c.lanes & (c.lanes - 1)) != 0) c.lanes = std::min(64, need);
     if (c.tile_nnz <= 0) c.tile_nnz = default_tile(c.lanes);
     if (c.unroll <= 0) c.unroll = 8;
+}
+
+// Fills unset fields of an NNZ_TILED config for these operands.
+void complete_nb(dspmm_config &c, int nv, bool bf16) {
+    complete_vw(c, nv, choose_vw_any(nv, bf16 ? 8 : 4));
+}
+
+// The same for the kernels that stage B in LDS and need whole, aligned vectors.
+void complete_aligned(dspmm_config &c, int nv, int64_t ldb, int64_t ldc, const void *B,
+                      const void *C, bool bf16) {
+    complete_vw(c, nv, choose_vw(nv, ldb, ldc, B, C, bf16 ? 2 : 4, bf16 ? 8 : 4));
 }
 
 constexpr int kSpmvTile = 1024;
@@ -625,7 +632,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
     case DSPMM_VARIANT_NNZ_TILED: {
         if (layout != DENSE_ROW_MAJOR) return DSPMM_STATUS_NOT_SUPPORTED;
         dspmm_config c = cfg;
-        complete_nb(c, nv, ldb, ldc, B, C, bf16);
+        complete_nb(c, nv, bf16);
         if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) return DSPMM_STATUS_NOT_SUPPORTED;
         NbPlan *plan = nullptr;
         dspmm_status_t s = get_plan(A, c.tile_nnz, &plan, kPlanNnzTiled, 1, build);
@@ -669,7 +676,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         if (layout != DENSE_ROW_MAJOR) return DSPMM_STATUS_NOT_SUPPORTED;
         dspmm_config c = cfg;
         const int umax = c.tile_nnz > 0 ? c.tile_nnz : kCachedUmaxDefault;
-        complete_nb(c, nv, ldb, ldc, B, C, bf16);
+        complete_aligned(c, nv, ldb, ldc, B, C, bf16);
         if (c.lanes * c.vec < nv) return DSPMM_STATUS_NOT_SUPPORTED;     // one slab only
         if (umax < 8 || umax > 4096 || umax % 8) return DSPMM_STATUS_NOT_SUPPORTED;
         const int smax = cached_smax(umax);
@@ -717,7 +724,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         if (R != 2 && R != 4 && R != 8) return DSPMM_STATUS_NOT_SUPPORTED;
         dspmm_config c = cfg;
         c.tile_nnz = 0;
-        complete_nb(c, nv, ldb, ldc, B, C, bf16);
+        complete_nb(c, nv, bf16);
         if (cfg.row_stride < -1 || cfg.row_stride > std::max(1, A->nr))
             return DSPMM_STATUS_INVALID_VALUE;
         if (cfg.row_stride < 0 && A->rb_stride < 1 && !build) return DSPMM_STATUS_NOT_PREPARED;
@@ -761,7 +768,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         dspmm_config c = cfg;
         c.tile_nnz = 0;
         c.unroll = 0;
-        complete_nb(c, nv, ldb, ldc, B, C, bf16);
+        complete_aligned(c, nv, ldb, ldc, B, C, bf16);
         const Slab sl = make_slab(nv, c.vec);
         if (sl.count != 1) return DSPMM_STATUS_NOT_SUPPORTED;          // one slab only
         if (A->rb_stride < 1 && !build) return DSPMM_STATUS_NOT_PREPARED;
@@ -861,7 +868,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
             c.unroll = cfg.unroll > 0 ? cfg.unroll : 4;
             if (!row_seq_unroll_ok(c.unroll)) return DSPMM_STATUS_NOT_SUPPORTED;
             if (!launch) return DSPMM_STATUS_SUCCESS;
-            complete_nb(c, nv, ldb, ldc, B, C, bf16);
+            complete_nb(c, nv, bf16);
             const Slab sl = make_slab(nv, c.vec);
             RowSeqLaunch a;
             a.rowPtr = A->rowPtr;
@@ -976,9 +983,7 @@ dspmm_status_t ex_workspace_bytes(dspmm_matrix_s *A, DenseLayout layout, int nv,
         return DSPMM_STATUS_SUCCESS;
     }
     if (c.variant != DSPMM_VARIANT_NNZ_TILED) return DSPMM_STATUS_SUCCESS;
-    // Tile size does not depend on pointers; use aligned placeholders.
-    complete_nb(c, nv, nv, nv, reinterpret_cast<const void *>(256), reinterpret_cast<const void *>(256),
-                btype == DSPMM_R_16BF);
+    complete_nb(c, nv, btype == DSPMM_R_16BF);
     NbPlan *plan = nullptr;
     dspmm_status_t st = get_plan(A, c.tile_nnz, &plan);
     if (st != DSPMM_STATUS_SUCCESS) return st;
@@ -1346,7 +1351,7 @@ std::vector<dspmm_config> autotune_candidates(dspmm_matrix_s *A, DenseLayout lay
     if (nv > 1) {
         dspmm_config base{};
         base.variant = DSPMM_VARIANT_NNZ_TILED;
-        complete_nb(base, nv, ldb, ldc, B, C, bf16);
+        complete_nb(base, nv, bf16);
         for (int l = base.lanes / 2; l >= 1 && l * 4 >= base.lanes; l /= 2) slab_lanes.push_back(l);
     }
     if (nv > 1) {
@@ -1402,7 +1407,7 @@ std::vector<dspmm_config> autotune_candidates(dspmm_matrix_s *A, DenseLayout lay
         if (reuse >= kCachedMinReuse) {
             dspmm_config base{};
             base.variant = DSPMM_VARIANT_NNZ_TILED;
-            complete_nb(base, nv, ldb, ldc, B, C, bf16);
+            complete_nb(base, nv, bf16);
             for (int vw = base.vec; vw >= 1 && vw * 2 >= base.vec; vw /= 2) {
                 for (int umax : {64, 128, 256, 512}) {
                     for (int nt : {64, 128, 256}) {
@@ -1420,12 +1425,12 @@ std::vector<dspmm_config> autotune_candidates(dspmm_matrix_s *A, DenseLayout lay
     {
         dspmm_config base{};
         base.variant = DSPMM_VARIANT_NNZ_TILED;
-        complete_nb(base, nv, ldb, ldc, B, C, bf16);
+        complete_nb(base, nv, bf16);
         for (int vw = base.vec; vw >= 1; vw /= 2) {
             dspmm_config c{};
             c.variant = DSPMM_VARIANT_NNZ_TILED;
             c.vec = vw;
-            complete_nb(c, nv, ldb, ldc, B, C, bf16);
+            complete_nb(c, nv, bf16);
             if (c.vec != vw) continue;
             const int s0 = default_tile(c.lanes);
             for (int S : {s0 / 8, s0 / 4, s0 / 2, s0, s0 * 2, s0 * 4}) {
@@ -1465,7 +1470,7 @@ std::vector<dspmm_config> autotune_candidates(dspmm_matrix_s *A, DenseLayout lay
             }
         dspmm_config base{};
         base.variant = DSPMM_VARIANT_NNZ_TILED;
-        complete_nb(base, nv, ldb, ldc, B, C, bf16);
+        complete_nb(base, nv, bf16);
         const int g = 64 / std::min(base.lanes, make_slab(nv, base.vec).lanes);   // rows per wavefront
         bool overflow = false;
         for (int rw = 0; rw < A->nr && !overflow; rw += g)

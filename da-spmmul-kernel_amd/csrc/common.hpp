@@ -113,6 +113,58 @@ __device__ __forceinline__ void load_b(float (&r)[VW], const TB *p) {
     else load_vec_bf16<VW>(r, reinterpret_cast<const uint16_t *>(p));
 }
 
+// The same on global memory at any element-aligned address.  Global loads and
+// stores of 4 to 16 bytes need no natural alignment on gfx950 (the compiler
+// emits one instruction either way), so row-major kernels use the widest
+// vectors for every nv and leading dimension; see slab_col.
+template <typename T, int N, int ALIGN>
+struct VecAt {
+    typedef T type __attribute__((ext_vector_type(N), aligned(ALIGN)));
+};
+template <typename TB, int VW>
+__device__ __forceinline__ void load_g(float (&r)[VW], const TB *p) {
+    if constexpr (VW == 1) {
+        load_b<TB, 1>(r, p);
+    } else if constexpr (sizeof(TB) == 4) {
+        static_assert(VW <= 4, "VW");
+        const auto t = *reinterpret_cast<const typename VecAt<float, VW, 4>::type *>(p);
+#pragma unroll
+        for (int k = 0; k < VW; k++) r[k] = t[k];
+    } else if constexpr (VW == 2) {
+        typedef uint32_t u32_at2 __attribute__((aligned(2)));
+        const uint32_t t = *reinterpret_cast<const u32_at2 *>(p);
+        r[0] = bf16_lo(t); r[1] = bf16_hi(t);
+    } else {
+        const auto t = *reinterpret_cast<const typename VecAt<uint32_t, VW / 2, 2>::type *>(p);
+#pragma unroll
+        for (int k = 0; k < VW / 2; k++) { r[2 * k] = bf16_lo(t[k]); r[2 * k + 1] = bf16_hi(t[k]); }
+    }
+}
+template <bool NT, int VW>
+__device__ __forceinline__ void store_g(float *p, const float (&r)[VW]) {
+    if constexpr (VW == 8) {
+        store_g<NT, 4>(p, reinterpret_cast<const float (&)[4]>(r[0]));
+        store_g<NT, 4>(p + 4, reinterpret_cast<const float (&)[4]>(r[4]));
+    } else if constexpr (VW == 1) {
+        if constexpr (NT) __builtin_nontemporal_store(r[0], p); else *p = r[0];
+    } else {
+        using V = typename VecAt<float, VW, 4>::type;
+        V t;
+#pragma unroll
+        for (int k = 0; k < VW; k++) t[k] = r[k];
+        if constexpr (NT) __builtin_nontemporal_store(t, reinterpret_cast<V *>(p));
+        else *reinterpret_cast<V *>(p) = t;
+    }
+}
+
+// First column of a lane's VW columns.  Where fewer than VW are left of the
+// row (nv >= VW), the last ones of the row: the lane shares columns with its
+// neighbour and both write the same values.
+template <int VW>
+__device__ __forceinline__ int slab_col(int col, int nv) {
+    return VW > 1 && col < nv && col + VW > nv ? nv - VW : col;
+}
+
 // Streaming (read-once) scalar loads for the sparse operand.
 template <typename T>
 __device__ __forceinline__ T ld_stream(const T *p) { return __builtin_nontemporal_load(p); }

@@ -39,7 +39,7 @@ __device__ __forceinline__ void seq_accumulate(float (&acc)[VW], int p0, int p1,
         float b[UNR][VW];
 #pragma unroll
         for (int u = 0; u < UNR; u++)
-            load_b<TB, VW>(b[u], B + (int64_t)s_col[p + u - w] * ldb + col0);
+            load_g<TB, VW>(b[u], B + (int64_t)s_col[p + u - w] * ldb + col0);
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
             const float a = s_val[p + u - w];
@@ -51,7 +51,7 @@ __device__ __forceinline__ void seq_accumulate(float (&acc)[VW], int p0, int p1,
         float b[UNR - 1][VW];
 #pragma unroll
         for (int u = 0; u < UNR - 1; u++)
-            if (p + u < p1) load_b<TB, VW>(b[u], B + (int64_t)s_col[p + u - w] * ldb + col0);
+            if (p + u < p1) load_g<TB, VW>(b[u], B + (int64_t)s_col[p + u - w] * ldb + col0);
 #pragma unroll
         for (int u = 0; u < UNR - 1; u++) {
             if (p + u < p1) {
@@ -94,7 +94,7 @@ __device__ __forceinline__ bool is_long_row(int len, int block_nnz, int block_ro
 // groups multiply P nonzeros into LDS (P products of L * VW columns, two
 // steps' gathers in flight) and thread t < L * VW adds column t's products in
 // order; the (column, value) pairs go through LDS in chunks, loaded a chunk
-// ahead.  Returns column t's sum.  Every thread calls it (barriers
+// ahead.  `base` is the first of the L * VW columns.  Returns column t's sum.  Every thread calls it (barriers
 // inside).
 template <int VW, int L, int U>
 struct LongRow {
@@ -108,9 +108,11 @@ struct LongRow {
 
     static __device__ __forceinline__ float sum(int p0, int p1, const int *__restrict__ colIdx,
                                                 const float *__restrict__ values,
-                                                const float *__restrict__ B, int64_t ldb, int col0,
-                                                bool colok, float *mem) {
+                                                const float *__restrict__ B, int64_t ldb, int base,
+                                                int nv_, float *mem) {
         const int t = threadIdx.x, g = t / L, l = t % L;
+        const int col0 = slab_col<VW>(base + l * VW, nv_), at = col0 - base;
+        const bool colok = col0 < nv_, whole = nv_ % VW == 0;
         float *prod = mem;
         int *s_c = reinterpret_cast<int *>(mem + P * W);
         float *s_v = mem + P * W + 2 * CHK;
@@ -138,7 +140,7 @@ struct LongRow {
         auto gather = [&](int k, float (&d)[U][VW]) {
 #pragma unroll
             for (int u = 0; u < U; u++)
-                load_vec<VW>(d[u], Bc + (int64_t)s_c[(k * P + g * U + u) % (2 * CHK)] * ldb);
+                load_g<float, VW>(d[u], Bc + (int64_t)s_c[(k * P + g * U + u) % (2 * CHK)] * ldb);
         };
         float sum = 0.f;
         auto step = [&](int k, float (&d)[U][VW]) {
@@ -150,7 +152,14 @@ struct LongRow {
 #pragma unroll
                 for (int q = 0; q < VW; q++)   // +0 past the end: a sum that began at +0 keeps its bits
                     m[q] = i < n ? v * d[u][q] : 0.f;
-                store_vec<VW>(prod + (g * U + u) * W + l * VW, m);
+                float *to = prod + (g * U + u) * W + at;
+                if (whole) {
+                    store_vec<VW>(to, m);
+                } else {                       // the row's last columns, some of them a neighbour's
+#pragma unroll
+                    for (int q = 0; q < VW; q++)
+                        if (at + q >= 0) to[q] = m[q];
+                }
             }
             gather(k + 2, d);
             if ((k + 3) % S == 0) {            // the chunk that step k + 3 begins, read from step k + 1 on
@@ -234,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_
     const int r = (int)min(rw + ln / W, (int64_t)nr);
     const int start = rowPtr[r], end = mine ? rowPtr[r + 1] : start;
     const int e0 = rowPtr[rw], e1 = rowPtr[min(rw + G, (int64_t)nr)];
-    const int gl = (ln % L) * VW;              // first column that this lane gathers
+    const int gl = slab_col<VW>((ln % L) * VW, nv);   // first column that this lane gathers
     const float *__restrict__ Bc = B + (gl < nv ? gl : 0);
     float *sp = s_prod[wv];
     int cc[E];
@@ -247,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_
             vv[k] = values[p];
         }
 #pragma unroll
-        for (int k = 0; k < E; k++) load_vec<VW>(b[k], Bc + (int64_t)cc[k] * ldb);
+        for (int k = 0; k < E; k++) load_g<float, VW>(b[k], Bc + (int64_t)cc[k] * ldb);
     };
     float acc = 0.f;
     if (e0 < e1) gather(e0);
@@ -361,11 +370,10 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
             if (rowPtr[q + 1] - rowPtr[q] >= kScoutRow) s_scout[atomicAdd(&s_nlong, 1)] = (uint16_t)(q - q0);
         __syncthreads();
         const int cb = blockIdx.y * slab_w + (int)blockIdx.x % parts * SW;
-        const int c0 = cb + ((int)threadIdx.x % SL) * VW;
         for (int i = 0; i < s_nlong; i++) {
             const int q = q0 + s_scout[i];
-            const float sum = Scout::sum(rowPtr[q], rowPtr[q + 1], colIdx, values, B, ldb, c0,
-                                         c0 < nv, s_mem);
+            const float sum = Scout::sum(rowPtr[q], rowPtr[q + 1], colIdx, values, B, ldb, cb,
+                                         nv, s_mem);
             if ((int)threadIdx.x < SW && cb + (int)threadIdx.x < nv)
                 C[(int64_t)q * ldc + cb + (int)threadIdx.x] = sum;
         }
@@ -374,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
     const int b = xcd_remap(blockIdx.x - scouts, gridDim.x - scouts);
     const int r0 = b * RPB;
     const int r = r0 + (int)threadIdx.x / L;
-    const int col0 = blockIdx.y * slab_w + ((int)threadIdx.x % L) * VW;
+    const int col0 = slab_col<VW>(blockIdx.y * slab_w + ((int)threadIdx.x % L) * VW, nv);
     const bool colok = col0 < nv;
     const int rlast = min(r0 + RPB, nr);
     const int bs = rowPtr[r0], be = rowPtr[rlast];
@@ -397,7 +405,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
         for (int i = 0; i < nlong; i++) {
             const int q = s_long[i], p0 = rowPtr[q], p1 = rowPtr[q + 1];
             if (p1 - p0 >= kScoutRow) continue;
-            const float sum = Long::sum(p0, p1, colIdx, values, B, ldb, col0, colok, s_mem);
+            const float sum = Long::sum(p0, p1, colIdx, values, B, ldb, blockIdx.y * slab_w, nv, s_mem);
             const int c = blockIdx.y * slab_w + (int)threadIdx.x;
             if ((int)threadIdx.x < L * VW && c < nv)
                 __builtin_nontemporal_store(sum, C + (int64_t)q * ldc + c);
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
             __syncthreads();                              // before the next window's tables
         }
     }
-    if (r < nr && colok && mine) store_vec_nt<VW>(C + (int64_t)r * ldc + col0, acc);
+    if (r < nr && colok && mine) store_g<true, VW>(C + (int64_t)r * ldc + col0, acc);
 }
 
 // ===========================================================================
@@ -502,7 +510,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
     const int t = threadIdx.x;
     const int r = b * RPB + t / T;
     const int g = (t % T) / L;
-    const int col0 = blockIdx.y * slab_w + (t % L) * VW;
+    const int col0 = slab_col<VW>(blockIdx.y * slab_w + (t % L) * VW, nv);
     const bool colok = col0 < nv;
     float acc[VW];
 #pragma unroll
@@ -513,14 +521,14 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
             const int c = colIdx[p];
             const float a = values[p];
             float bv[VW];
-            load_vec<VW>(bv, B + (int64_t)c * ldb + col0);
+            load_g<float, VW>(bv, B + (int64_t)c * ldb + col0);
 #pragma unroll
             for (int k = 0; k < VW; k++) acc[k] = __builtin_fmaf(a, bv[k], acc[k]);
         }
     }
 #pragma unroll
     for (int k = 0; k < VW; k++) acc[k] = butterfly_sum<L, T>(acc[k]);
-    if (r < nr && colok && g == 0) store_vec_nt<VW>(C + (int64_t)r * ldc + col0, acc);
+    if (r < nr && colok && g == 0) store_g<true, VW>(C + (int64_t)r * ldc + col0, acc);
 }
 
 // ===========================================================================
@@ -992,7 +1000,7 @@ int stream_rows(int W, int nnz, int nr) {
 dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st) {
-    const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, 4));
+    const Slab s = make_slab(nv, choose_vw_any(nv, 4));
     if (s.width <= 8) {
         with_vw(s.vw, [&](auto vw_c) {
             with_lanes(s.lanes, [&](auto l_c) {
@@ -1046,7 +1054,7 @@ void launch_csr_vector_rm(int nr, int nv, int64_t ldb, int64_t ldc, const int *r
 dspmm_status_t csr_vector_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st, int hint) {
-    const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, 4));
+    const Slab s = make_slab(nv, choose_vw_any(nv, 4));
     const double mean = nr ? (double)nnz / nr : 0.0;
     int gt = hint > 0 ? pow2_floor(hint) : lanes_for_mean(mean, 64);
     gt = std::max(1, std::min(gt, 64 / s.lanes));

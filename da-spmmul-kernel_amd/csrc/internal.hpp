@@ -33,6 +33,10 @@ inline int choose_vw(int nv, int64_t ldb, int64_t ldc, const void *B, const void
     return 1;
 }
 
+// The same for kernels whose lanes may start anywhere in a row (slab_col):
+// the widest that nv columns fill, whatever the alignment.
+inline int choose_vw_any(int nv, int max_vw) { return pow2_floor(nv < max_vw ? nv : max_vw); }
+
 // Lane-group shape covering nv columns with `vw` floats per lane: lanes is a
 // power of two <= 64, slab = lanes*vw columns per grid.y slice.
 struct Slab {

@@ -84,7 +84,7 @@ __device__ __forceinline__ void process_tiles(const ItemDesc &d, int t0, int tco
                                               const WaveStage &w) {
     const int ln = lane_id();
     const int g = ln / L;
-    const int col0 = slab * d.slab_w + (ln % L) * VW;
+    const int col0 = slab_col<VW>(slab * d.slab_w + (ln % L) * VW, d.nv);
     if (g >= tcount || col0 >= d.nv) return;
     const TB *__restrict__ B = reinterpret_cast<const TB *>(d.B);
     const int4 tile = d.tiles[t0 + g];
@@ -103,7 +103,7 @@ __device__ __forceinline__ void process_tiles(const ItemDesc &d, int t0, int tco
 #pragma unroll
             for (int u = 0; u < UNR; u++)
                 if (p + u < pe)
-                    load_b<TB, VW>(bv[u], B + (int64_t)s_col[skew(p + u - P0)] * d.ldb + col0);
+                    load_g<TB, VW>(bv[u], B + (int64_t)s_col[skew(p + u - P0)] * d.ldb + col0);
 #pragma unroll
             for (int u = 0; u < UNR; u++) {
                 if (p + u < pe) {
@@ -114,7 +114,7 @@ __device__ __forceinline__ void process_tiles(const ItemDesc &d, int t0, int tco
             }
         }
         const int slot = -1 - tile.y;
-        store_vec<VW>(d.carry + (int64_t)slot * d.ldcarry + col0, acc);
+        store_g<false, VW>(d.carry + (int64_t)slot * d.ldcarry + col0, acc);
         return;
     }
 
@@ -127,13 +127,13 @@ __device__ __forceinline__ void process_tiles(const ItemDesc &d, int t0, int tco
 #pragma unroll
         for (int u = 0; u < UNR; u++)
             if (p + u < pe)
-                load_b<TB, VW>(bv[u], B + (int64_t)s_col[skew(p + u - P0)] * d.ldb + col0);
+                load_g<TB, VW>(bv[u], B + (int64_t)s_col[skew(p + u - P0)] * d.ldb + col0);
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
             const int q = p + u;
             if (q < pe) {
                 while (q >= next_end) {           // row r is complete (or empty)
-                    store_vec_nt<VW>(C + (int64_t)r * d.ldc + col0, acc);
+                    store_g<true, VW>(C + (int64_t)r * d.ldc + col0, acc);
 #pragma unroll
                     for (int k = 0; k < VW; k++) acc[k] = 0.f;
                     ++r;
@@ -146,7 +146,7 @@ __device__ __forceinline__ void process_tiles(const ItemDesc &d, int t0, int tco
         }
     }
     for (; r < re; ++r) {                          // last row, then trailing empty rows
-        store_vec_nt<VW>(C + (int64_t)r * d.ldc + col0, acc);
+        store_g<true, VW>(C + (int64_t)r * d.ldc + col0, acc);
 #pragma unroll
         for (int k = 0; k < VW; k++) acc[k] = 0.f;
     }
@@ -732,7 +732,7 @@ __global__ __launch_bounds__(kBlock) void k_row_blocked(RowBlockLaunch a) {
     const int blk_w = (xcd_remap(blockIdx.x, gridDim.x) * WPB + wv) * G;
     if (blk_w >= a.nblocks) return;              // the whole wavefront leaves
     const int blk = blk_w + g;
-    const int col0 = blockIdx.y * a.slab_w + l * VW;
+    const int col0 = slab_col<VW>(blockIdx.y * a.slab_w + l * VW, a.nv);
     const bool has = blk < a.nblocks;
     const bool active = has && col0 < a.nv;
     int u0 = 0, len = 0;
@@ -775,7 +775,7 @@ __global__ __launch_bounds__(kBlock) void k_row_blocked(RowBlockLaunch a) {
                 if (u + x >= cnt) cm[x].y = 0;
             }
 #pragma unroll
-            for (int x = 0; x < UNR; x++) load_b<TB, VW>(bv[x], B + (int64_t)cm[x].x * a.ldb);
+            for (int x = 0; x < UNR; x++) load_g<TB, VW>(bv[x], B + (int64_t)cm[x].x * a.ldb);
 #pragma unroll
             for (int x = 0; x < UNR; x++) {
                 float v[R];
@@ -798,7 +798,7 @@ __global__ __launch_bounds__(kBlock) void k_row_blocked(RowBlockLaunch a) {
 #pragma unroll
     for (int i = 0; i < R; i++) {
         const int64_t r = r0 + (int64_t)i * a.stride;
-        if (r < a.nr) store_vec_nt<VW>(a.C + r * a.ldc + col0, acc[i]);
+        if (r < a.nr) store_g<true, VW>(a.C + r * a.ldc + col0, acc[i]);
     }
 }
 
@@ -1128,7 +1128,7 @@ __global__ __launch_bounds__(kBlock) void k_row_seq(RowSeqLaunch g, int lg) {
     const int nrow = (int)min((int64_t)G, (int64_t)g.nr - rw);
     const int gi = lane >> lg;
     const int64_t r = rw + gi;
-    const int col0 = blockIdx.y * g.slab_w + (lane & ((1 << lg) - 1)) * VW;
+    const int col0 = slab_col<VW>(blockIdx.y * g.slab_w + (lane & ((1 << lg) - 1)) * VW, g.nv);
     const bool active = gi < nrow && col0 < g.nv;
     const int e0 = g.rowPtr[rw], e1 = g.rowPtr[rw + nrow];
     int start = 0, end = 0;
@@ -1146,7 +1146,7 @@ __global__ __launch_bounds__(kBlock) void k_row_seq(RowSeqLaunch g, int lg) {
             float bv[UNR][VW];
 #pragma unroll
             for (int u = 0; u < UNR; u++)
-                load_b<TB, VW>(bv[u], B + (int64_t)sc[min(p + u, p1 - 1)] * g.ldb);
+                load_g<TB, VW>(bv[u], B + (int64_t)sc[min(p + u, p1 - 1)] * g.ldb);
 #pragma unroll
             for (int u = 0; u < UNR; u++) {
                 if (p + u < p1) {
@@ -1212,7 +1212,7 @@ __global__ __launch_bounds__(kBlock) void k_row_seq(RowSeqLaunch g, int lg) {
             done += cnt;
         }
     }
-    if (active) store_vec_nt<VW>(g.C + r * g.ldc + col0, acc);
+    if (active) store_g<true, VW>(g.C + r * g.ldc + col0, acc);
 }
 
 namespace {

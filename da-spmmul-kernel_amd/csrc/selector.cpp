@@ -75,6 +75,8 @@ bool learned_select(dspmm_matrix_s *A, int nv, dspmm_config *out) {
     dspmm_config c{};
     std::tie(c.variant, c.vec, c.lanes, c.tile_nnz, c.unroll, c.row_stride) = win->first;
     if ((c.variant == DSPMM_VARIANT_SPMV_TILED) != (nv == 1)) return false;
+    // lanes that covered the measured width in one slab cover this one too
+    if (c.lanes > 0 && c.vec > 0 && c.lanes * c.vec >= best_nv) c.lanes = 0;
     *out = c;
     return true;
 }

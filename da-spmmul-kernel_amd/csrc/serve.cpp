@@ -228,8 +228,7 @@ struct dspmm_server_s {
             return true;
         case DSPMM_VARIANT_NNZ_TILED: {
             dspmm_config cc = c;
-            complete_nb(cc, nv, nv, nv, reinterpret_cast<const void *>(256),
-                        reinterpret_cast<const void *>(256), cfg.btype == DSPMM_R_16BF);
+            complete_nb(cc, nv, cfg.btype == DSPMM_R_16BF);
             std::lock_guard<std::mutex> lk(h->mu);
             NbPlan *plan = nullptr;
             return get_plan(h, cc.tile_nnz, &plan) == DSPMM_STATUS_SUCCESS && plan->nsplits == 0;
