@@ -477,16 +477,72 @@ constexpr double kRowBlockMinReuse = 1.2;
 // more than they save.
 constexpr int64_t kTransposedMinWork = 1 << 20;
 
+// Fills the tile size of a single nnz-tiled launch: at most `cap`, and small
+// enough that the launch has kTileWaves wavefronts (a wavefront owns 64 /
+// lanes tiles).  Power law, 262144 rows, BF16 B: nv = 32 and 16 per tile
+// 74 us, 64 142; nv = 128 and 32 per tile 160 us, 256 442 (3100 wavefronts
+// of long serial tiles).  The batch keeps default_tile: its items share the
+// GPU, and small tiles made it slower.
+constexpr int kTileWaves = 2048;
+void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_config &c) {
+    dspmm_config full = c;
+    complete_nb(full, nv, bf16);
+    const int64_t slabs = div_up(nv, full.vec * full.lanes), g = 64 / full.lanes;
+    c.tile_nnz = cap > 0 ? cap : full.lanes <= 4 ? 16 : full.lanes <= 32 ? 32 : 64;
+    while (c.tile_nnz > 8 && A->nnz * slabs / (g * c.tile_nnz) < kTileWaves) c.tile_nnz /= 2;
+}
+
+// Whether one row outlasts the others of a row-per-group kernel.
+bool skewed(const dspmm_matrix_s *A) {
+    return A->max_len > std::max(64.0, 8.0 * A->mean);
+}
+
 dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_t bt) {
+    const bool bf16 = bt == DSPMM_R_16BF;
+    const bool rm = layout == DENSE_ROW_MAJOR;
     dspmm_config c{};
     if (nv == 1) {
         c.variant = DSPMM_VARIANT_SPMV_TILED;
         c.tile_nnz = kSpmvTile;
-    } else if (layout == DENSE_ROW_MAJOR || bt == DSPMM_R_16BF ||
-               (int64_t)A->nnz * nv >= kTransposedMinWork) {
-        c.variant = DSPMM_VARIANT_NNZ_TILED;        // column-major: through transposed copies
-    } else {
+        return c;
+    }
+    if (!rm && !bf16 && (int64_t)A->nnz * nv < kTransposedMinWork) {
         c.variant = DSPMM_VARIANT_CSR_SCALAR;
+        return c;
+    }
+    // Otherwise a row-major kernel; column-major operands go through
+    // transposed copies.  The figures: BF16 B, us, here / the alternative.
+    c.variant = DSPMM_VARIANT_NNZ_TILED;
+    c.unroll = 4;
+    const bool skew = skewed(A);
+    if (nv <= 8) {
+        // four lanes and more per tile: 64^3 stencil, nv = 8, two values a
+        // lane and 32 per tile 43, eight a lane 132 (each gather instruction
+        // then reaches 64 rows of B)
+        c.vec = std::min(2, nv);
+        single_tile(A, nv, bf16, skew ? 16 : 32, c);
+    } else if (skew) {
+        single_tile(A, nv, bf16, 0, c);
+    } else {
+        // rows of like lengths: a group per row, without tiles and split rows
+        // (4096 rows of 16, nv = 20 to 128: 4.7 to 5.5 / 8.7 to 12.3)
+        dspmm_config full{};
+        complete_nb(full, nv, bf16);
+        const bool overflow = A->mean * (64 / full.lanes) > kRowSeqWindow;
+        if (overflow && nv <= 32 && (bf16 || !rm)) {
+            // long rows side by side would wait for one another's windows
+            // (20000 rows of 100, nv = 20: 32 / 66, sliced 38)
+            if (bf16) c.vec = nv <= 16 ? 1 : 2;
+            c.unroll = bf16 ? 4 : 8;
+            c.tile_nnz = 128;
+        } else {
+            c.variant = DSPMM_VARIANT_CSR_SCALAR;
+            c.unroll = bf16 || !rm ? 4 : 0;
+            if (overflow && c.unroll > 0) {
+                c.unroll = 16;
+                c.tile_nnz = 1;                // sliced windows: nv = 64, 32 / 43
+            }
+        }
     }
     return c;
 }
