@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "internal.hpp"
@@ -50,6 +51,154 @@ bool is_col(int which) {
            which == K_SPMM_COO_SCALAR_COL || which == K_SPMM_COO_VECTOR_COL;
 }
 
+// Scratch for one call, in stream order, from a pool of the device that holds
+// at most kScratchPool bytes in all.
+//   * On the legacy default stream, whose work is in order whoever enqueues it,
+//     the calls share one block, kept between them: a call holds the lock until
+//     its last launch is enqueued.
+//   * On any other stream a call takes a block before its launches and gives it
+//     back behind them, so that streams and threads never share one.  That
+//     costs a call 10 us, mostly the marker behind its work.
+// Free blocks beyond kScratchKept go back to the device at the next
+// synchronisation; dspmm_release_scratch, and dspmm_device_alloc where it finds
+// the memory short, give back the rest.
+constexpr size_t kScratchCall = (size_t)256 << 20;   // the most that one call takes
+constexpr size_t kScratchKept = kScratchCall;
+constexpr size_t kScratchPool = 4 * kScratchCall;
+constexpr int kMaxDevices = 64;
+
+struct DevicePool {
+    std::mutex lock;                 // held while the shared block's user enqueues
+    hipMemPool_t pool = nullptr;
+    bool tried = false;
+    void *block = nullptr;           // the legacy default stream's
+    size_t bytes = 0;
+};
+DevicePool g_pools[kMaxDevices];
+
+DevicePool *current_pool() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+    return &g_pools[dev];
+}
+
+// p.lock is held.
+bool make_pool(DevicePool &p, int dev) {
+    if (p.tried) return p.pool != nullptr;
+    p.tried = true;
+    hipMemPoolProps props;
+    std::memset(&props, 0, sizeof(props));
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    props.maxSize = kScratchPool;
+    hipMemPool_t pool = nullptr;
+    if (hipMemPoolCreate(&pool, &props) != hipSuccess) return false;
+    uint64_t kept = kScratchKept;
+    int wait = 0;                    // no stream is made to wait for another one's scratch
+    if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &kept) != hipSuccess ||
+        hipMemPoolSetAttribute(pool, hipMemPoolReuseAllowInternalDependencies, &wait) != hipSuccess) {
+        (void)hipMemPoolDestroy(pool);
+        return false;
+    }
+    p.pool = pool;
+    return true;
+}
+
+// Gives the current device's free scratch back.  Waits for the legacy default
+// stream, whose block it frees.
+dspmm_status_t release_scratch() {
+    DevicePool *p = current_pool();
+    if (!p) return DSPMM_STATUS_SUCCESS;
+    std::lock_guard<std::mutex> held(p->lock);
+    if (!p->pool) return DSPMM_STATUS_SUCCESS;
+    hipError_t e = hipSuccess;
+    if (p->block) e = hipFreeAsync(p->block, nullptr);
+    p->block = nullptr;
+    p->bytes = 0;
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e == hipSuccess) e = hipMemPoolTrimTo(p->pool, 0);
+    return hip_status(e);
+}
+
+class Scratch {
+public:
+    Scratch(size_t need, hipStream_t st) : st_(st) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (st && (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
+            return;
+        DevicePool *p = current_pool();
+        if (!p) return;
+        std::unique_lock<std::mutex> held(p->lock);
+        if (!make_pool(*p, (int)(p - g_pools))) return;
+        size_t bytes = 1 << 20;      // few sizes, so that a freed block fits the next call
+        while (bytes < need) bytes *= 2;
+        if (st) {
+            held.unlock();
+            if (hipMallocFromPoolAsync(&ptr_, bytes, p->pool, st) != hipSuccess) ptr_ = nullptr;
+            return;
+        }
+        if (p->bytes < bytes) {
+            if (p->block) (void)hipFreeAsync(p->block, nullptr);
+            p->block = nullptr;
+            p->bytes = 0;
+            if (hipMallocFromPoolAsync(&p->block, bytes, p->pool, nullptr) != hipSuccess) {
+                p->block = nullptr;
+                return;
+            }
+            p->bytes = bytes;
+        }
+        ptr_ = p->block;
+        held_ = std::move(held);
+    }
+    void *ptr() const { return ptr_; }
+    // Behind the last launch that uses it.
+    dspmm_status_t release() {
+        if (!ptr_) return DSPMM_STATUS_SUCCESS;
+        const dspmm_status_t s = st_ ? hip_status(hipFreeAsync(ptr_, st_)) : DSPMM_STATUS_SUCCESS;
+        if (held_.owns_lock()) held_.unlock();
+        ptr_ = nullptr;
+        return s;
+    }
+
+private:
+    hipStream_t st_;
+    void *ptr_ = nullptr;
+    std::unique_lock<std::mutex> held_;
+};
+
+// Columns at a time with which a column-major product runs on row-major copies
+// (launch_compat_flipped); 0: in place.  In place every product costs a line of
+// B (about 0.22 M gathers a microsecond where B is random, twice that where the
+// L2s hold it), the copies cost three to four launches (10 to 13 us, and on a
+// stream other than the legacy default one 12 us more for the scratch) and a
+// pass over B and C.  So the line lies at a number of products, lower where B
+// is too large for the L2s.  In place / copies, us: 131072 rows of 24, nv = 32
+// (100 M products) 464 / 76; 16384 rows of 32, nv = 8 (4.2 M) csr_vector 15 / 12,
+// coo 21 / 14; 32^3 stencil, nv = 8 (6.6 M) csr_vector 11.5 / 11.7; 5000 rows of 12 over
+// 250000 columns, nv = 16 (0.96 M, B of 16 MB) csr_vector 18 / 14; 131072 rows of 6,
+// nv = 4 (3.1 M) csr_scalar 17 / 16, coo 18 / 21.  Two columns share their lines less:
+// power law, nv = 2 (6.4 M), coo 33 / 37.
+int flip_columns(int which, int nr, int nc, int nnz, int nv, bool null_stream) {
+    if (nv < 2 || nr == 0 || nnz == 0) return 0;
+    const double products = 1e-6 * nnz * nv, b = 1e-6 * nc * nv;
+    bool pays;
+    if (which == K_SPMM_CSR_SCALAR_COL)
+        pays = products >= (null_stream ? 4.1 : 6.0);
+    else if (which == K_SPMM_CSR_VECTOR_COL)
+        pays = null_stream ? products >= 5.0 || (products >= 1.0 && b >= 4.0)
+                           : products >= 14.0 || (products >= 3.4 && b >= 1.5);
+    else if (nv == 2)
+        pays = products >= (null_stream ? 16.0 : 24.0);
+    else
+        pays = null_stream ? products >= 4.1 || (products >= 2.0 && b >= 4.0)
+                           : products >= 10.0 || (products >= 3.8 && b >= 3.0);
+    if (!pays) return 0;
+    int cols = nv;
+    while (cols > 8 && compat_flipped_bytes(nr, nc, cols) > kScratchCall) cols = (cols / 2 + 7) / 8 * 8;
+    return compat_flipped_bytes(nr, nc, cols) <= kScratchCall ? cols : 0;
+}
+
 // One reference-named launcher: packed operands (ld = nv row-major; ld =
 // nc / nr column-major; ld = 1 for the SpMV kernels, whose nv==1 case is
 // the same in both layouts).
@@ -70,6 +219,18 @@ dspmm_status_t run_named(int which, int nr, int nc, int nnz, int nv, const int *
         break;
     default:
         break;
+    }
+    const int cols = is_col(which) ? flip_columns(which, nr, nc, nnz, nv, stream == nullptr) : 0;
+    if (cols) {
+        const hipStream_t hs = as_hip(stream);
+        Scratch mem(compat_flipped_bytes(nr, nc, cols), hs);
+        if (mem.ptr()) {
+            st = launch_compat_flipped(which, nr, nc, nnz, nv, rowPtr, rowIdx, colIdx, values, B, C,
+                                       static_cast<float *>(mem.ptr()), cols, hs);
+            const dspmm_status_t freed = mem.release();
+            return st != DSPMM_STATUS_SUCCESS ? st : freed;
+        }
+        (void)hipGetLastError();     // no scratch (out of memory, a captured stream): without
     }
     int64_t ldb, ldc;
     if (is_col(which)) { ldb = nc; ldc = nr; }
@@ -164,8 +325,15 @@ dspmm_status_t dspmm_device_alloc(void **ptr, size_t bytes) {
     if (!ptr) return DSPMM_STATUS_INVALID_VALUE;
     *ptr = nullptr;
     if (bytes == 0) return DSPMM_STATUS_SUCCESS;
-    return hip_status(hipMalloc(ptr, bytes));
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory && release_scratch() == DSPMM_STATUS_SUCCESS) {
+        (void)hipGetLastError();
+        e = hipMalloc(ptr, bytes);
+    }
+    return hip_status(e);
 }
+
+dspmm_status_t dspmm_release_scratch(void) { return release_scratch(); }
 
 dspmm_status_t dspmm_device_free(void *ptr) {
     if (!ptr) return DSPMM_STATUS_SUCCESS;

@@ -21,6 +21,7 @@
 
 #include "common.hpp"
 #include "internal.hpp"
+#include "native.hpp"
 
 namespace dspmm {
 
@@ -223,8 +224,10 @@ struct LongRow {
 // ===========================================================================
 // Pairs per window at W columns.
 constexpr int stream_pairs(int W) { return W == 1 ? 512 : W == 8 ? 128 : 256; }
-template <int VW, int L>
-__global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_t ldb, int64_t ldc,
+// COL: column-major operands, W = L columns (from W * blockIdx.y on) at a time,
+// one per lane.
+template <int VW, int L, bool COL>
+__global__ __launch_bounds__(kBlock) void k_csr_stream(int nr, int nv, int64_t ldb, int64_t ldc,
                                                            const int *__restrict__ rowPtr,
                                                            const int *__restrict__ colIdx,
                                                            const float *__restrict__ values,
@@ -243,8 +246,14 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_
     const int r = (int)min(rw + ln / W, (int64_t)nr);
     const int start = rowPtr[r], end = mine ? rowPtr[r + 1] : start;
     const int e0 = rowPtr[rw], e1 = rowPtr[min(rw + G, (int64_t)nr)];
+    static_assert(!COL || VW == 1, "a column per lane");
+    if constexpr (COL) {
+        B += (int64_t)blockIdx.y * W * ldb;
+        C += (int64_t)blockIdx.y * W * ldc;
+        nv -= (int)blockIdx.y * W;
+    }
     const int gl = slab_col<VW>((ln % L) * VW, nv);   // first column that this lane gathers
-    const float *__restrict__ Bc = B + (gl < nv ? gl : 0);
+    const float *__restrict__ Bc = B + (gl < nv ? (COL ? gl * ldb : (int64_t)gl) : 0);
     float *sp = s_prod[wv];
     int cc[E];
     float vv[E], b[E][VW];
@@ -256,7 +265,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_
             vv[k] = values[p];
         }
 #pragma unroll
-        for (int k = 0; k < E; k++) load_g<float, VW>(b[k], Bc + (int64_t)cc[k] * ldb);
+        for (int k = 0; k < E; k++) load_g<float, VW>(b[k], Bc + (COL ? (int64_t)cc[k] : (int64_t)cc[k] * ldb));
     };
     float acc = 0.f;
     if (e0 < e1) gather(e0);
@@ -319,7 +328,8 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream_rm(int nr, int nv, int64_
             for (int u = 0; u < 8; u++) acc = acc + (u < n ? x[u] : 0.f);
         }
     }
-    if (mine && c < nv) __builtin_nontemporal_store(acc, C + (int64_t)r * ldc + c);
+    if (mine && c < nv)
+        __builtin_nontemporal_store(acc, C + (COL ? (int64_t)c * ldc + r : (int64_t)r * ldc + c));
 }
 
 // ===========================================================================
@@ -493,42 +503,157 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
 // ===========================================================================
 // Row-balanced, parallel reduction, row-major (spmv_csr_vector,
 // spmm_csr_vector_row).  A team of GT groups x L lanes owns one row; group
-// g takes nonzeros start+g, start+g+GT, ...; the GT partial vectors are
-// combined with a butterfly over stride L..GT*L/2.  Overwrites.
+// g takes nonzeros start+g, start+g+GT, ..., U gathers in flight; the GT
+// partial vectors are combined with a butterfly over stride L..GT*L/2.
+// Overwrites.  Rows that a team would work on long after the others:
+//   * beyond kTeamSteps nonzeros per group the team's whole wavefront sums the row;
+//   * rows of `scout_row` or more nonzeros (a multiple of the mean) are found
+//     and summed by the first `scouts` blocks of the launch, kScoutCols columns
+//     and kScoutRows rows each.
 // ===========================================================================
-template <int VW, int L, int GT>
+constexpr int kTeamSteps = 16;
+constexpr int kVecScoutRow = 256;
+constexpr int64_t kVecScoutWork = 1000000;
+
+// acc += the nonzeros p0, p0 + STRIDE, ... < e, in that order.
+template <int VW, int U>
+__device__ __forceinline__ void strided_accumulate(float (&acc)[VW], int p0, int e, int stride,
+                                                   const int *__restrict__ colIdx,
+                                                   const float *__restrict__ values,
+                                                   const float *__restrict__ Bc, int64_t ldb) {
+    if constexpr (U == 1) {
+        for (int p = p0; p < e; p += stride) {
+            const int c = colIdx[p];
+            const float a = values[p];
+            float b[VW];
+            load_g<float, VW>(b, Bc + (int64_t)c * ldb);
+#pragma unroll
+            for (int k = 0; k < VW; k++) acc[k] = __builtin_fmaf(a, b[k], acc[k]);
+        }
+        return;
+    }
+    const int n = e - p0;
+    for (int i = 0; i < n; i += U * stride) {
+        int c[U];
+        float a[U], b[U][VW];
+#pragma unroll
+        for (int u = 0; u < U; u++) {          // padded with the last nonzero
+            const int q = p0 + min(i + u * stride, n - 1);
+            c[u] = colIdx[q];
+            a[u] = values[q];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) load_g<float, VW>(b[u], Bc + (int64_t)c[u] * ldb);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (i + u * stride < n) {
+#pragma unroll
+                for (int k = 0; k < VW; k++) acc[k] = __builtin_fmaf(a[u], b[u][k], acc[k]);
+            }
+        }
+    }
+}
+
+// A scout block's share: the rows of scout_row or more nonzeros among its
+// kScoutRows, SW columns from `base` on.
+template <int VW, int SW>
+__device__ __forceinline__ void scout_rows(int q0, int q1, int base, int nv, int64_t ldb, int64_t ldc,
+                                        const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
+                                        const float *__restrict__ values, const float *__restrict__ B,
+                                        float *__restrict__ C, int scout_row) {
+    constexpr int SL = SW / VW;                // lanes of a group
+    constexpr int NW = kBlock / kWave;
+    __shared__ uint16_t s_scout[kScoutRows];
+    __shared__ int s_n;
+    __shared__ float s_part[NW][SW];
+    const int t = threadIdx.x, ln = lane_id();
+    if (t == 0) s_n = 0;
+    __syncthreads();
+    for (int q = q0 + t; q < q1; q += kBlock)
+        if (rowPtr[q + 1] - rowPtr[q] >= scout_row) s_scout[atomicAdd(&s_n, 1)] = (uint16_t)(q - q0);
+    __syncthreads();
+    const int col0 = slab_col<VW>(base + (t % SL) * VW, nv);
+    for (int i = 0; i < s_n; i++) {
+        const int q = q0 + s_scout[i];
+        float acc[VW];
+#pragma unroll
+        for (int k = 0; k < VW; k++) acc[k] = 0.f;
+        if (col0 < nv)
+            strided_accumulate<VW, 8>(acc, rowPtr[q] + t / SL, rowPtr[q + 1], kBlock / SL, colIdx, values,
+                                      B + col0, ldb);
+#pragma unroll
+        for (int k = 0; k < VW; k++) acc[k] = butterfly_sum<SL, kWave>(acc[k]);
+        if (ln < SL && col0 < nv) {
+#pragma unroll
+            for (int k = 0; k < VW; k++)       // the last lane may share its neighbour's columns
+                if (col0 + k >= base) s_part[t / kWave][col0 - base + k] = acc[k];
+        }
+        __syncthreads();
+        if (t < SW && base + t < nv) {
+            float sum = s_part[0][t];
+#pragma unroll
+            for (int w = 1; w < NW; w++) sum += s_part[w][t];
+            C[(int64_t)q * ldc + base + t] = sum;
+        }
+        __syncthreads();                       // before the next row's parts
+    }
+}
+
+template <int VW, int L, int GT, int U>
 __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_t ldb, int64_t ldc,
                                                            const int *__restrict__ rowPtr,
                                                            const int *__restrict__ colIdx,
                                                            const float *__restrict__ values,
                                                            const float *__restrict__ B,
-                                                           float *__restrict__ C, int slab_w) {
+                                                           float *__restrict__ C, int slab_w,
+                                                           int scouts, int scout_row) {
     constexpr int T = GT * L;                  // lanes per row
     constexpr int RPB = kBlock / T;
     static_assert(T <= kWave, "team larger than a wavefront");
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int t = threadIdx.x;
+    if (__builtin_expect((int)blockIdx.x < scouts, 0)) {
+        constexpr int SW = L * VW < kScoutCols ? L * VW : kScoutCols;
+        const int parts = (min(slab_w, nv - (int)blockIdx.y * slab_w) + SW - 1) / SW;
+        const int q0 = (int)blockIdx.x / parts * kScoutRows;
+        scout_rows<VW, SW>(q0, min(q0 + kScoutRows, nr), blockIdx.y * slab_w + (int)blockIdx.x % parts * SW,
+                           nv, ldb, ldc, rowPtr, colIdx, values, B, C, scout_row);
+        return;
+    }
+    const int b = xcd_remap(blockIdx.x - scouts, gridDim.x - scouts);
     const int r = b * RPB + t / T;
     const int g = (t % T) / L;
     const int col0 = slab_col<VW>(blockIdx.y * slab_w + (t % L) * VW, nv);
     const bool colok = col0 < nv;
+    const float *__restrict__ Bc = B + (colok ? col0 : 0);
     float acc[VW];
 #pragma unroll
     for (int k = 0; k < VW; k++) acc[k] = 0.f;
-    if (r < nr && colok) {
-        const int s = rowPtr[r], e = rowPtr[r + 1];
-        for (int p = s + g; p < e; p += GT) {
-            const int c = colIdx[p];
-            const float a = values[p];
-            float bv[VW];
-            load_g<float, VW>(bv, B + (int64_t)c * ldb + col0);
-#pragma unroll
-            for (int k = 0; k < VW; k++) acc[k] = __builtin_fmaf(a, bv[k], acc[k]);
-        }
-    }
+    int s = 0, e = 0;
+    if (r < nr) { s = rowPtr[r]; e = rowPtr[r + 1]; }
+    const bool apart = e - s >= scout_row;
+    const bool wide = T < kWave && !apart && e - s > kTeamSteps * GT;
+    const bool mine = r < nr && !apart && !wide;
+    if (mine && colok) strided_accumulate<VW, U>(acc, s + g, e, GT, colIdx, values, Bc, ldb);
 #pragma unroll
     for (int k = 0; k < VW; k++) acc[k] = butterfly_sum<L, T>(acc[k]);
-    if (r < nr && colok && g == 0) store_g<true, VW>(C + (int64_t)r * ldc + col0, acc);
+    if (mine && colok && g == 0) store_g<true, VW>(C + (int64_t)r * ldc + col0, acc);
+    if constexpr (T < kWave) {
+        uint64_t m = __ballot(wide && t % T == 0);
+        if (__builtin_expect(m != 0, 0)) {
+            const int ln = lane_id();
+            for (; m; m &= m - 1) {
+                const int o = __builtin_ctzll(m);
+                const int q = read_lane(r, o), ps = read_lane(s, o), pe = read_lane(e, o);
+#pragma unroll
+                for (int k = 0; k < VW; k++) acc[k] = 0.f;
+                if (colok)
+                    strided_accumulate<VW, 4>(acc, ps + ln / L, pe, kWave / L, colIdx, values, Bc, ldb);
+#pragma unroll
+                for (int k = 0; k < VW; k++) acc[k] = butterfly_sum<L, kWave>(acc[k]);
+                if (ln < L && colok) store_g<true, VW>(C + (int64_t)q * ldc + col0, acc);
+            }
+        }
+    }
 }
 
 // ===========================================================================
@@ -659,11 +784,11 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
             flush(cur, acc);
         }
     } else {
-        // acc becomes the sum of the row's last runs up to this group: rows are
-        // sorted, so equal last rows mean that the groups between hold nothing else
-        segmented_scan<L, VW>(acc, cur);
+        // acc becomes the sum of a row's last runs up to this group, as long as
+        // the groups between hold nothing else
         const int prow = __shfl_up(cur, L);
         const bool joins = ln >= L && prow == first;
+        segmented_scan<L, VW>(acc, segment_id(ln % L == 0 && !(joins && one)));
 #pragma unroll
         for (int k = 0; k < VW; k++) {
             const float p = __shfl_up(acc[k], L);
@@ -716,10 +841,13 @@ __global__ __launch_bounds__(kBlock) void k_coo_spmv(int nnz, const int *__restr
         if (key[u] != INT_MAX) v[u] *= x[(int64_t)c[u] * ldx];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const int kfirst = read_lane(key[u], 0), klast = read_lane(key[u], kWave - 1);
+        const int klast = read_lane(key[u], kWave - 1);
+        const int before = __shfl_up(key[u], 1);
+        const bool begins = ln > 0 && before != key[u];
+        const bool single = __ballot(begins) == 0;   // one row in the whole chunk
         float s[1] = {v[u]};
-        if (kfirst == klast) s[0] = butterfly_sum<1, kWave>(s[0]);
-        else segmented_scan<1, 1>(s, key[u]);
+        if (single) s[0] = butterfly_sum<1, kWave>(s[0]);
+        else segmented_scan<1, 1>(s, segment_id(begins));
         int next = __shfl_down(key[u], 1);
         if (ln == kWave - 1) next = INT_MAX;
         if (u + 1 < U) {                       // a row that goes on: its sum joins the next chunk
@@ -729,7 +857,7 @@ __global__ __launch_bounds__(kBlock) void k_coo_spmv(int nnz, const int *__restr
             if (ln == kWave - 1) next = nk;
         }
         if (key[u] != INT_MAX && next != key[u] &&
-            !(kfirst == klast && ln != kWave - 1))
+            !(single && ln != kWave - 1))
             unsafeAtomicAdd(y + (int64_t)key[u] * ldy, s[0]);
     }
 }
@@ -740,7 +868,8 @@ __global__ __launch_bounds__(kBlock) void k_coo_spmv(int nnz, const int *__restr
 // here a lane carries T columns so A is read ceil(nv/T) times.
 // ===========================================================================
 
-// Row-balanced, sequential (spmm_csr_scalar_col): one lane per row.
+// Row-balanced, sequential (spmm_csr_scalar_col): one lane per row,
+// for products too large for k_csr_stream that find no scratch for row-major copies.
 template <int T>
 __global__ __launch_bounds__(kBlock) void k_csr_scalar_cm(int nr, int nv, int64_t ldb, int64_t ldc,
                                                            const int *__restrict__ rowPtr,
@@ -805,93 +934,50 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_cm(int nr, int nv, int64_
     float acc[T];
 #pragma unroll
     for (int t = 0; t < T; t++) acc[t] = 0.f;
-    if (r < nr) {
-        const int s = rowPtr[r], e = rowPtr[r + 1];
-        for (int p = s + l; p < e; p += L) {
+    int s = 0, e = 0;
+    if (r < nr) { s = rowPtr[r]; e = rowPtr[r + 1]; }
+    auto add = [&](int p0, int pe, int stride) {
+        for (int p = p0; p < pe; p += stride) {
             const int c = colIdx[p];
             const float a = values[p];
 #pragma unroll
             for (int t = 0; t < T; t++)
                 if (t < nt) acc[t] = __builtin_fmaf(a, Bj[(int64_t)t * ldb + c], acc[t]);
         }
-    }
+    };
+    const bool wide = L < kWave && e - s > kTeamSteps * L;
+    if (!wide) add(s + l, e, L);
 #pragma unroll
     for (int t = 0; t < T; t++) acc[t] = group_sum<L>(acc[t]);
-    if (r < nr) {
+    if (r < nr && !wide) {
         // Spread the T stores over the group's lanes.
 #pragma unroll
         for (int t = 0; t < T; t++)
             if (t < nt && (t % L) == l) C[(int64_t)(j0 + t) * ldc + r] = acc[t];
     }
-}
-
-// Nnz-balanced, sequential (spmm_coo_scalar_col): one lane per NE nonzeros.
-template <int T, int NE>
-__global__ __launch_bounds__(kBlock) void k_coo_scalar_cm(int nnz, int nv, int64_t ldb, int64_t ldc,
-                                                           const int *__restrict__ rowIdx,
-                                                           const int *__restrict__ colIdx,
-                                                           const float *__restrict__ values,
-                                                           const float *__restrict__ B,
-                                                           float *__restrict__ C) {
-    constexpr int CH = kBlock * NE;
-    constexpr int PADN = CH + kBlock;
-    __shared__ int s_row[PADN];
-    __shared__ int s_col[PADN];
-    __shared__ float s_val[PADN];
-    const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const int64_t base = (int64_t)b * CH;
-    const int cnt = (int)min<int64_t>(CH, (int64_t)nnz - base);
-    for (int i = threadIdx.x; i < cnt; i += kBlock) {
-        const int j = i + i / NE;
-        s_row[j] = ld_stream(rowIdx + base + i);
-        s_col[j] = ld_stream(colIdx + base + i);
-        s_val[j] = ld_stream(values + base + i);
-    }
-    __syncthreads();
-    const int j0c = blockIdx.y * T;
-    const int nt = min(T, nv - j0c);
-    const float *Bj = B + (int64_t)j0c * ldb;
-    float *Cj = C + (int64_t)j0c * ldc;
-    const int e0 = (int)threadIdx.x * NE, e1 = min(e0 + NE, cnt);
-    if (e0 >= e1) return;
-    const int jb = (int)threadIdx.x * (NE + 1);
-    int cur = s_row[jb];
-    float acc[T];
-    {
-        const int c = s_col[jb];
-        const float a = s_val[jb];
+    if constexpr (L < kWave) {
+        // rows beyond kTeamSteps nonzeros per lane: by the whole wavefront
+        const int ln = lane_id();
+        for (uint64_t m = __ballot(wide && l == 0); __builtin_expect(m != 0, 0); m &= m - 1) {
+            const int o = __builtin_ctzll(m);
+            const int q = read_lane(r, o);
 #pragma unroll
-        for (int t = 0; t < T; t++) acc[t] = (t < nt) ? a * Bj[(int64_t)t * ldb + c] : 0.f;
-    }
-    for (int e = e0 + 1; e < e1; e++) {
-        const int j = jb + (e - e0);
-        const int rr = s_row[j], c = s_col[j];
-        const float a = s_val[j];
-        float bv[T];
+            for (int t = 0; t < T; t++) acc[t] = 0.f;
+            add(read_lane(s, o) + ln, read_lane(e, o), kWave);
 #pragma unroll
-        for (int t = 0; t < T; t++) bv[t] = (t < nt) ? Bj[(int64_t)t * ldb + c] : 0.f;
-        if (rr != cur) {
+            for (int t = 0; t < T; t++) acc[t] = group_sum<kWave>(acc[t]);
 #pragma unroll
             for (int t = 0; t < T; t++)
-                if (t < nt) unsafeAtomicAdd(Cj + (int64_t)t * ldc + cur, acc[t]);
-#pragma unroll
-            for (int t = 0; t < T; t++) acc[t] = a * bv[t];
-            cur = rr;
-        } else {
-#pragma unroll
-            for (int t = 0; t < T; t++) acc[t] = acc[t] + a * bv[t];
+                if (t < nt && t == ln) C[(int64_t)(j0 + t) * ldc + q] = acc[t];
         }
     }
-#pragma unroll
-    for (int t = 0; t < T; t++)
-        if (t < nt) unsafeAtomicAdd(Cj + (int64_t)t * ldc + cur, acc[t]);
 }
 
 // Nnz-balanced, parallel (spmm_coo_vector_col, and spmv_coo_vector for
 // column-major nv=1): a wavefront takes 64 consecutive nonzeros per step,
 // T columns per lane, segmented scan per column.
 template <int T>
-__global__ __launch_bounds__(kBlock) void k_coo_vector_cm(int nnz, int nv, int64_t ldb, int64_t ldc,
+__global__ __launch_bounds__(kBlock) void k_coo_cm(int nnz, int nv, int64_t ldb, int64_t ldc,
                                                            const int *__restrict__ rowIdx,
                                                            const int *__restrict__ colIdx,
                                                            const float *__restrict__ values,
@@ -919,8 +1005,9 @@ __global__ __launch_bounds__(kBlock) void k_coo_vector_cm(int nnz, int nv, int64
             for (int t = 0; t < T; t++)
                 if (t < nt) v[t] = a * Bj[(int64_t)t * ldb + c];
         }
-        const int kfirst = read_lane(key, 0), klast = read_lane(key, kWave - 1);
-        if (kfirst == klast) {
+        const int before = __shfl_up(key, 1);
+        const bool begins = ln > 0 && before != key;
+        if (__ballot(begins) == 0) {           // one row in the whole chunk
 #pragma unroll
             for (int t = 0; t < T; t++) v[t] = group_sum<kWave>(v[t]);
             // Lane t adds column t: one atomic per column, spread over lanes.
@@ -928,12 +1015,64 @@ __global__ __launch_bounds__(kBlock) void k_coo_vector_cm(int nnz, int nv, int64
             for (int t = 0; t < T; t++)
                 if (ln == t && t < nt) unsafeAtomicAdd(Cj + (int64_t)t * ldc + key, v[t]);
         } else {
-            segmented_scan<1, T>(v, key);
-            const bool tail = valid && (ln == kWave - 1 || p + 1 >= nnz || rowIdx[p + 1] != key);
+            segmented_scan<1, T>(v, segment_id(begins));
+            const int next = __shfl_down(key, 1);
+            const bool tail = valid && (ln == kWave - 1 || next != key);
             if (tail) {
 #pragma unroll
                 for (int t = 0; t < T; t++)
                     if (t < nt) unsafeAtomicAdd(Cj + (int64_t)t * ldc + key, v[t]);
+            }
+        }
+    }
+}
+
+// ===========================================================================
+// Row-major copies of column-major operands: src(j, i) = src[j * lds + i], i in
+// [0, n), to dst[i * ldd + j] (TO_ROWS), or back; ADD adds to the destination
+// atomically, as the accumulating algorithms do.  A block takes W columns of
+// kFlipWords / W rows through LDS, so that both sides are read and written in
+// runs: bound by the copy (64 MB at 32 columns: 5 TB/s).
+// ===========================================================================
+constexpr int kFlipWords = 2048;
+
+template <int W, bool TO_ROWS, bool ADD>
+__global__ __launch_bounds__(kBlock) void k_flip(const float *__restrict__ src, int64_t lds, int n,
+                                                 int cols, float *__restrict__ dst, int64_t ldd) {
+    constexpr int R = kFlipWords / W;          // rows of a tile
+    constexpr int S = R + (W < 32 ? 64 / W : 1);   // stride that spreads a row's W words over the banks
+    constexpr int N = kFlipWords / kBlock;     // words per thread
+    __shared__ float tile[W * S];
+    const int64_t i0 = (int64_t)blockIdx.x * R;
+    const int j0 = (int)blockIdx.y * W, t = (int)threadIdx.x;
+    const int ni = (int)min<int64_t>(R, (int64_t)n - i0), nj = min(W, cols - j0);
+    float v[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int q = k * kBlock + t;
+        const int i = TO_ROWS ? q % R : q / W, j = TO_ROWS ? q / R : q % W;
+        v[k] = 0.f;
+        if (i < ni && j < nj)
+            v[k] = TO_ROWS ? src[(int64_t)(j0 + j) * lds + i0 + i] : src[(i0 + i) * lds + j0 + j];
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int q = k * kBlock + t;
+        const int i = TO_ROWS ? q % R : q / W, j = TO_ROWS ? q / R : q % W;
+        tile[j * S + i] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int q = k * kBlock + t;
+        const int i = TO_ROWS ? q / W : q % R, j = TO_ROWS ? q % W : q / R;
+        if (i < ni && j < nj) {
+            const float x = tile[j * S + i];
+            float *d = dst + (TO_ROWS ? (i0 + i) * ldd + j0 + j : (int64_t)(j0 + j) * ldd + i0 + i);
+            if constexpr (ADD) {
+                if (x != 0.f) unsafeAtomicAdd(d, x);   // rows without a nonzero cost nothing
+            } else {
+                *d = x;
             }
         }
     }
@@ -945,7 +1084,6 @@ __global__ __launch_bounds__(kBlock) void k_coo_vector_cm(int nnz, int nv, int64
 namespace {
 
 constexpr int kCmCols = 8;      // columns per lane in the column-major kernels
-constexpr int kCooNE = 8;       // nonzeros per group in the COO scalar kernels
 
 int grid_for_waves(int64_t waves_needed) {
     // Persistent-ish grid for the grid-strided COO vector kernels: enough
@@ -988,7 +1126,7 @@ void with_vw(int vw, F &&f) {
     }
 }
 
-// Rows per wavefront of k_csr_stream_rm: most of a window of pairs, at most one
+// Rows per wavefront of k_csr_stream: most of a window of pairs, at most one
 // row per lane and column.  Fewer pairs leave gathers unused (64^3 stencil,
 // nv = 4: half a window 26.6 us, 3/4 18.6, one 16.1), more make a long row's
 // wavefront later (power law, nv = 1: 60, 61, 83).
@@ -1007,7 +1145,7 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
                 constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
                 if constexpr (VW_ * L_ <= 8) {
                     const int g = stream_rows(VW_ * L_, nnz, nr);
-                    hipLaunchKernelGGL((k_csr_stream_rm<VW_, L_>), dim3(div_up(nr, (int64_t)g * (kBlock / kWave))),
+                    hipLaunchKernelGGL((k_csr_stream<VW_, L_, false>), dim3(div_up(nr, (int64_t)g * (kBlock / kWave))),
                                        dim3(kBlock), 0, st, nr, nv, ldb, ldc, rowPtr, colIdx, values,
                                        B, C, g);
                 }
@@ -1041,17 +1179,34 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
 }
 
 template <int VW, int L, int GT>
-void launch_csr_vector_rm(int nr, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
+void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                           const int *colIdx, const float *values, const float *B, float *C,
                           hipStream_t st, const Slab &s) {
     if constexpr (GT * L <= kWave) {
-        dim3 grid(div_up(nr, kBlock / (GT * L)), s.count);
-        hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
-                           ldc, rowPtr, colIdx, values, B, C, s.width);
+        // Scouts where a long row's wavefront would set the kernel's time; a whole
+        // number per XCD leaves xcd_remap its meaning.
+        int scouts = 0, scout_row = INT_MAX;
+        if ((int64_t)nnz * L >= kVecScoutWork) {
+            const int parts = div_up(std::min(nv, s.width), std::min(s.width, kScoutCols));
+            scouts = div_up((int64_t)div_up(nr, kScoutRows) * parts, kNumXcd) * kNumXcd;
+            scout_row = (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(kVecScoutRow, 8 * (int64_t)nnz / std::max(1, nr)));
+        }
+        dim3 grid(scouts + div_up(nr, kBlock / (GT * L)), s.count);
+        // Four gathers in flight where a group has that many to make: with a B
+        // that the L2s hold, only rows of more than 7 nonzeros per group gain (16384
+        // rows of 32, nv = 64: 15.7 -> 13.4 us; 64^3 stencil, nv = 32: 98.7 -> 83.7;
+        // 32^3 stencil, nv = 64, 6.3 per group: 15.0, with four 16.5).
+        const double per = (double)nnz / ((double)GT * std::max(1, nr));
+        if (per > 7 || (per > 2.5 && (int64_t)nc * nv >= (4 << 20)))
+            hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT, 4>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
+                               ldc, rowPtr, colIdx, values, B, C, s.width, scouts, scout_row);
+        else
+            hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT, 1>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
+                               ldc, rowPtr, colIdx, values, B, C, s.width, scouts, scout_row);
     }
 }
 
-dspmm_status_t csr_vector_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
+dspmm_status_t csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st, int hint) {
     const Slab s = make_slab(nv, choose_vw_any(nv, 4));
@@ -1063,7 +1218,7 @@ dspmm_status_t csr_vector_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
             with_lanes(gt, [&](auto gt_c) {
                 constexpr int GT_ = decltype(gt_c)::value;
-                launch_csr_vector_rm<VW_, L_, GT_>(nr, nv, ldb, ldc, rowPtr, colIdx, values, B, C,
+                launch_csr_vector_rm<VW_, L_, GT_>(nr, nc, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C,
                                                    st, s);
             });
         });
@@ -1135,12 +1290,29 @@ dspmm_status_t coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowI
     return launch_status();
 }
 
-dspmm_status_t csr_scalar_cm(int nr, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
+// Products up to which k_csr_stream, which gathers for long rows with all
+// lanes, is the faster kernel (16384 rows of 32, nv = 2: 52 -> 7 us; power law of
+// 16806 rows, nv = 16: 336 -> 25; 131072 rows of 6, nv = 8, 6.3 M: 33 against 41).
+constexpr int64_t kStreamProducts = 6000000;
+
+dspmm_status_t csr_scalar_cm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st) {
-    dim3 grid(div_up(nr, kBlock), div_up(nv, kCmCols));
-    hipLaunchKernelGGL((k_csr_scalar_cm<kCmCols>), grid, dim3(kBlock), 0, st, nr, nv, ldb, ldc,
-                       rowPtr, colIdx, values, B, C);
+    if ((int64_t)nnz * nv >= kStreamProducts) {
+        dim3 grid(div_up(nr, kBlock), div_up(nv, kCmCols));
+        hipLaunchKernelGGL((k_csr_scalar_cm<kCmCols>), grid, dim3(kBlock), 0, st, nr, nv, ldb, ldc,
+                           rowPtr, colIdx, values, B, C);
+        return launch_status();
+    }
+    with_lanes(std::min(pow2_ceil(nv), kCmCols), [&](auto l_c) {
+        constexpr int L_ = decltype(l_c)::value;
+        if constexpr (L_ <= kCmCols) {
+            const int g = stream_rows(L_, nnz, nr);
+            dim3 grid(div_up(nr, (int64_t)g * (kBlock / kWave)), div_up(nv, L_));
+            hipLaunchKernelGGL((k_csr_stream<1, L_, true>), grid, dim3(kBlock), 0, st, nr, nv, ldb, ldc,
+                               rowPtr, colIdx, values, B, C, g);
+        }
+    });
     return launch_status();
 }
 
@@ -1149,54 +1321,96 @@ dspmm_status_t csr_vector_cm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
                              hipStream_t st, int hint) {
     const double mean = nr ? (double)nnz / nr : 0.0;
     const int L = hint > 0 ? std::min(64, pow2_floor(hint)) : lanes_for_mean(mean, 64);
-    const int T = nv == 1 ? 1 : kCmCols;
+    const int T = std::min(pow2_ceil(nv), kCmCols);
     with_lanes(L, [&](auto l_c) {
         constexpr int L_ = decltype(l_c)::value;
-        if (T == 1) {
-            dim3 grid(div_up(nr, kBlock / L_), nv);
-            hipLaunchKernelGGL((k_csr_vector_cm<1, L_>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
-                               ldc, rowPtr, colIdx, values, B, C);
-        } else {
-            dim3 grid(div_up(nr, kBlock / L_), div_up(nv, kCmCols));
-            hipLaunchKernelGGL((k_csr_vector_cm<kCmCols, L_>), grid, dim3(kBlock), 0, st, nr, nv,
-                               ldb, ldc, rowPtr, colIdx, values, B, C);
+        with_lanes(T, [&](auto t_c) {
+            constexpr int T_ = decltype(t_c)::value;
+            if constexpr (T_ <= kCmCols) {
+                dim3 grid(div_up(nr, kBlock / L_), div_up(nv, T_));
+                hipLaunchKernelGGL((k_csr_vector_cm<T_, L_>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
+                                   ldc, rowPtr, colIdx, values, B, C);
+            }
+        });
+    });
+    return launch_status();
+}
+
+// ALG_COO_SCALAR and ALG_COO_VECTOR, column-major.
+dspmm_status_t coo_cm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
+                             const int *colIdx, const float *values, const float *B, float *C,
+                             hipStream_t st) {
+    with_lanes(std::min(pow2_ceil(nv), kCmCols), [&](auto t_c) {
+        constexpr int T_ = decltype(t_c)::value;
+        if constexpr (T_ <= kCmCols) {
+            dim3 grid(grid_for_waves(((int64_t)nnz + kWave - 1) / kWave), div_up(nv, T_));
+            hipLaunchKernelGGL((k_coo_cm<T_>), grid, dim3(kBlock), 0, st, nnz, nv, ldb, ldc, rowIdx,
+                               colIdx, values, B, C);
         }
     });
     return launch_status();
 }
 
-dspmm_status_t coo_scalar_cm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
-                             const int *colIdx, const float *values, const float *B, float *C,
-                             hipStream_t st) {
-    dim3 grid(div_up(nnz, kBlock * kCooNE), div_up(nv, kCmCols));
-    hipLaunchKernelGGL((k_coo_scalar_cm<kCmCols, kCooNE>), grid, dim3(kBlock), 0, st, nnz, nv, ldb,
-                       ldc, rowIdx, colIdx, values, B, C);
-    return launch_status();
+// C's copy starts on a line of its own.
+size_t align_words(int64_t words) { return ((size_t)words + 63) / 64 * 64; }
+
+template <int W>
+void launch_flip(bool to_rows, bool add, const float *src, int64_t lds, int n, int cols, float *dst,
+                 int64_t ldd, hipStream_t st) {
+    const dim3 grid(div_up(n, kFlipWords / W), div_up(cols, W));
+    if (to_rows)
+        hipLaunchKernelGGL((k_flip<W, true, false>), grid, dim3(kBlock), 0, st, src, lds, n, cols, dst, ldd);
+    else if (add)
+        hipLaunchKernelGGL((k_flip<W, false, true>), grid, dim3(kBlock), 0, st, src, lds, n, cols, dst, ldd);
+    else
+        hipLaunchKernelGGL((k_flip<W, false, false>), grid, dim3(kBlock), 0, st, src, lds, n, cols, dst, ldd);
 }
 
-dspmm_status_t coo_vector_cm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
-                             const int *colIdx, const float *values, const float *B, float *C,
-                             hipStream_t st) {
-    if (nv == 1) {
-        dim3 grid(grid_for_waves(((int64_t)nnz + kWave - 1) / kWave), 1);
-        hipLaunchKernelGGL((k_coo_vector_cm<1>), grid, dim3(kBlock), 0, st, nnz, nv, ldb, ldc,
-                           rowIdx, colIdx, values, B, C);
-    } else {
-        dim3 grid(grid_for_waves(((int64_t)nnz + kWave - 1) / kWave), div_up(nv, kCmCols));
-        hipLaunchKernelGGL((k_coo_vector_cm<kCmCols>), grid, dim3(kBlock), 0, st, nnz, nv, ldb,
-                           ldc, rowIdx, colIdx, values, B, C);
-    }
+dspmm_status_t flip(bool to_rows, bool add, const float *src, int64_t lds, int n, int cols, float *dst,
+                    int64_t ldd, hipStream_t st) {
+    if (cols <= 2) launch_flip<2>(to_rows, add, src, lds, n, cols, dst, ldd, st);
+    else if (cols <= 4) launch_flip<4>(to_rows, add, src, lds, n, cols, dst, ldd, st);
+    else if (cols <= 8) launch_flip<8>(to_rows, add, src, lds, n, cols, dst, ldd, st);
+    else if (cols <= 16) launch_flip<16>(to_rows, add, src, lds, n, cols, dst, ldd, st);
+    else launch_flip<32>(to_rows, add, src, lds, n, cols, dst, ldd, st);
     return launch_status();
 }
 
 }  // namespace
+
+// Column-major operands on row-major copies of B and C in `scratch`, `cols`
+// columns at a time, with the row-major kernel of the same algorithm.
+size_t compat_flipped_bytes(int nr, int nc, int nv) {
+    return (align_words((int64_t)nc * nv) + (size_t)nr * (size_t)nv) * sizeof(float);
+}
+
+dspmm_status_t launch_compat_flipped(int which, int nr, int nc, int nnz, int nv, const int *rowPtr,
+                                     const int *rowIdx, const int *colIdx, const float *values,
+                                     const float *B, float *C, float *scratch, int cols,
+                                     hipStream_t st) {
+    const bool coo = which == K_SPMM_COO_SCALAR_COL || which == K_SPMM_COO_VECTOR_COL;
+    dspmm_status_t s = DSPMM_STATUS_SUCCESS;
+    for (int j = 0; j < nv && s == DSPMM_STATUS_SUCCESS; j += cols) {
+        const int w = std::min(cols, nv - j);
+        float *Bt = scratch, *Ct = scratch + align_words((int64_t)nc * w);
+        s = flip(true, false, B + (int64_t)j * nc, nc, nc, w, Bt, w, st);
+        if (s == DSPMM_STATUS_SUCCESS && coo)
+            s = launch_fill_zero(Ct, (size_t)nr * (size_t)w * sizeof(float), st);
+        if (s != DSPMM_STATUS_SUCCESS) break;
+        if (coo) s = coo_rm(nnz, w, w, w, rowIdx, colIdx, values, Bt, Ct, st);
+        else if (which == K_SPMM_CSR_SCALAR_COL)
+            s = csr_scalar_rm(nr, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st);
+        else s = csr_vector_rm(nr, nc, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st, 0);
+        if (s == DSPMM_STATUS_SUCCESS) s = flip(false, coo, Ct, w, nr, w, C + (int64_t)j * nr, nr, st);
+    }
+    return s;
+}
 
 // Shared entry for the 12 launchers, the dispatcher and the native API.
 dspmm_status_t launch_compat(int which, int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc,
                              const int *rowPtr, const int *rowIdx, const int *colIdx,
                              const float *values, const float *B, float *C, hipStream_t st,
                              int hint) {
-    (void)nc;
     const bool coo = which == K_SPMV_COO_SCALAR || which == K_SPMV_COO_VECTOR ||
                      which == K_SPMM_COO_SCALAR_ROW || which == K_SPMM_COO_VECTOR_ROW ||
                      which == K_SPMM_COO_SCALAR_COL || which == K_SPMM_COO_VECTOR_COL;
@@ -1208,20 +1422,19 @@ dspmm_status_t launch_compat(int which, int nr, int nc, int nnz, int nv, int64_t
         return csr_scalar_rm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
     case K_SPMV_CSR_VECTOR:
     case K_SPMM_CSR_VECTOR_ROW:
-        return csr_vector_rm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st, hint);
+        return csr_vector_rm(nr, nc, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st, hint);
     case K_SPMV_COO_SCALAR:
     case K_SPMM_COO_SCALAR_ROW:
     case K_SPMV_COO_VECTOR:
     case K_SPMM_COO_VECTOR_ROW:
         return coo_rm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
     case K_SPMM_CSR_SCALAR_COL:
-        return csr_scalar_cm(nr, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
+        return csr_scalar_cm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
     case K_SPMM_CSR_VECTOR_COL:
         return csr_vector_cm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st, hint);
     case K_SPMM_COO_SCALAR_COL:
-        return coo_scalar_cm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
     case K_SPMM_COO_VECTOR_COL:
-        return coo_vector_cm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
+        return coo_cm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
     }
     return DSPMM_STATUS_INVALID_VALUE;
 }

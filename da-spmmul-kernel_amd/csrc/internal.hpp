@@ -58,6 +58,14 @@ dspmm_status_t launch_compat(int which, int nr, int nc, int nnz, int nv, int64_t
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t stream, int group_hint);
 
+// The column-major algorithms on row-major copies of B and C, `cols` columns at
+// a time, held in `scratch` (compat_flipped_bytes of that many).
+size_t compat_flipped_bytes(int nr, int nc, int nv);
+dspmm_status_t launch_compat_flipped(int which, int nr, int nc, int nnz, int nv, const int *rowPtr,
+                                     const int *rowIdx, const int *colIdx, const float *values,
+                                     const float *B, float *C, float *scratch, int cols,
+                                     hipStream_t stream);
+
 enum CompatKernel {
     K_SPMV_CSR_SCALAR = 0,
     K_SPMV_COO_SCALAR,

@@ -160,6 +160,13 @@ __device__ __forceinline__ void segmented_scan(float (&v)[NV], int key) {
     }
 }
 
+// The number of lanes up to this one that begin a segment: segmented_scan's
+// keys where equal rows need not be neighbours.
+__device__ __forceinline__ int segment_id(bool begins) {
+    const uint64_t m = __ballot(begins);
+    return __popcll(m & (~0ull >> (63 - lane_id())));
+}
+
 // Read lane `src` of a wave-uniform-independent value (result is uniform).
 __device__ __forceinline__ int read_lane(int v, int src) {
     return __builtin_amdgcn_readlane(v, src);

@@ -167,6 +167,7 @@ def _declare(lib):
         "dspmm_spmm": ([_I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P], _ST),
         "dspmm_device_alloc": ([C.POINTER(C.c_void_p), _SZ], _ST),
         "dspmm_device_free": ([_P], _ST),
+        "dspmm_release_scratch": ([], _ST),
         "dspmm_memcpy_h2d": ([_P, _P, _SZ], _ST),
         "dspmm_memcpy_d2h": ([_P, _P, _SZ], _ST),
         "dspmm_memcpy_d2d": ([_P, _P, _SZ, _P], _ST),

@@ -12,8 +12,11 @@
  *   - rowIdx (COO) is read only by the COO (nnz-balanced) algorithms;
  *   - row-major dense operands are packed with ld = nv, column-major ones
  *     with ld = nc (input) and ld = nr (output);
- *   - all pointers are caller-owned device memory; launchers allocate
- *     nothing and are asynchronous on `stream`.
+ *   - all pointers are caller-owned device memory; launchers are
+ *     asynchronous on `stream`.  They allocate nothing, except that a
+ *     column-major SpMM of some size takes up to 256 MiB of scratch in stream
+ *     order (dspmm_release_scratch); where there is none, and on a stream that
+ *     is being captured, it runs without.
  * Output semantics (spmvspmm_benchmark.cu:141-157):
  *   - CSR (row-balanced) algorithms OVERWRITE every output entry;
  *   - COO (nnz-balanced) algorithms ACCUMULATE into the output with atomic
@@ -138,6 +141,9 @@ DSPMM_API dspmm_status_t dspmm_spmm(SPMV_SPMM_ALG alg, DenseLayout layout,
  * ------------------------------------------------------------------- */
 DSPMM_API dspmm_status_t dspmm_device_alloc(void **ptr, size_t bytes);
 DSPMM_API dspmm_status_t dspmm_device_free(void *ptr);
+/* Gives back the scratch that column-major SpMMs keep on the current device
+ * between calls (at most 256 MiB).  Waits for the default stream. */
+DSPMM_API dspmm_status_t dspmm_release_scratch(void);
 /* Synchronous copies (like CUArray::sync_device / sync_host). */
 DSPMM_API dspmm_status_t dspmm_memcpy_h2d(void *dst, const void *src, size_t bytes);
 DSPMM_API dspmm_status_t dspmm_memcpy_d2h(void *dst, const void *src, size_t bytes);
