@@ -535,6 +535,8 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
             if (bf16) c.vec = nv <= 16 ? 1 : 2;
             c.unroll = bf16 ? 4 : 8;
             c.tile_nnz = 128;
+            complete_nb(full = c, nv, bf16);
+            while (nnz_tiled_lds_bytes(full.lanes, c.tile_nnz) > kMaxTileLds) c.tile_nnz /= 2;
         } else {
             c.variant = DSPMM_VARIANT_CSR_SCALAR;
             c.unroll = bf16 || !rm ? 4 : 0;

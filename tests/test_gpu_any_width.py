@@ -103,3 +103,27 @@ def test_auto_over_widths(name, layout, bf16):
         n = np.repeat(lens, nv) if layout == RM else np.tile(lens, nv)
         assert_fp32(d_C.numpy(), c64.reshape(-1), ab.reshape(-1), n, f"{name} nv={nv}", h32)
     m.close()
+
+
+@pytest.mark.parametrize("mean", [4, 37, 150])
+def test_auto_accepts_every_width(mean):
+    """The static default's tiles fit its kernels whatever lanes the width
+    leaves a row (integers: every order is exact)."""
+    rng = np.random.default_rng(mean)
+    nr, nc = 120_000 // mean, 900
+    rp = np.arange(nr + 1) * mean
+    ci = np.sort(rng.permuted(np.tile(np.arange(nc), (nr, 1)), axis=1)[:, :mean], axis=1).ravel() \
+        if nr * nc < 1 << 24 else rng.integers(0, nc, nr * mean)
+    v = rng.integers(-3, 4, nr * mean).astype(np.float32)
+    m = D.Matrix(nr, nc, rp, ci, v)
+    for nv in (2, 3, 4, 5, 8, 9, 10, 16, 17, 32, 33, 64, 65):
+        for layout, bf16 in ((RM, False), (RM, True), (CM, False), (CM, True)):
+            note(f"mean {mean} nv={nv} layout={layout} bf16={bf16}")
+            B = rng.integers(-3, 4, nc * nv).astype(np.float32)
+            d_B = D.DeviceArray.from_numpy(B)
+            d_b = D.to_bf16_device(d_B) if bf16 else d_B
+            d_C = D.DeviceArray.zeros(nr * nv)
+            m.spmm(d_b, d_C, nv, layout, btype=D.DSPMM_R_16BF if bf16 else D.DSPMM_R_32F)
+            D.synchronize()
+            ref = O.spmm_host32(layout, nr, nc, nv, rp, ci, v, B).reshape(-1)
+            assert_bitwise(d_C.numpy().reshape(-1) + 0.0, ref + 0.0, f"nv={nv}")
