@@ -484,12 +484,19 @@ constexpr int64_t kTransposedMinWork = 1 << 20;
 // of long serial tiles).  The batch keeps default_tile: its items share the
 // GPU, and small tiles made it slower.
 constexpr int kTileWaves = 2048;
+// Halves the tile until the launch's LDS fits.
+void fit_tile(int nv, bool bf16, dspmm_config &c) {
+    dspmm_config full = c;
+    complete_nb(full, nv, bf16);
+    while (nnz_tiled_lds_bytes(full.lanes, c.tile_nnz) > kMaxTileLds) c.tile_nnz /= 2;
+}
 void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
     const int64_t slabs = div_up(nv, full.vec * full.lanes), g = 64 / full.lanes;
     c.tile_nnz = cap > 0 ? cap : full.lanes <= 4 ? 16 : full.lanes <= 32 ? 32 : 64;
     while (c.tile_nnz > 8 && A->nnz * slabs / (g * c.tile_nnz) < kTileWaves) c.tile_nnz /= 2;
+    fit_tile(nv, bf16, c);
 }
 
 // Whether one row outlasts the others of a row-per-group kernel.
@@ -535,8 +542,7 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
             if (bf16) c.vec = nv <= 16 ? 1 : 2;
             c.unroll = bf16 ? 4 : 8;
             c.tile_nnz = 128;
-            complete_nb(full = c, nv, bf16);
-            while (nnz_tiled_lds_bytes(full.lanes, c.tile_nnz) > kMaxTileLds) c.tile_nnz /= 2;
+            fit_tile(nv, bf16, c);
         } else {
             c.variant = DSPMM_VARIANT_CSR_SCALAR;
             c.unroll = bf16 || !rm ? 4 : 0;

@@ -127,3 +127,20 @@ def test_auto_accepts_every_width(mean):
             D.synchronize()
             ref = O.spmm_host32(layout, nr, nc, nv, rp, ci, v, B).reshape(-1)
             assert_bitwise(d_C.numpy().reshape(-1) + 0.0, ref + 0.0, f"nv={nv}")
+
+
+def test_auto_accepts_narrow_bf16_of_many_rows():
+    """Enough nonzeros for the static default's longest tiles, one lane each."""
+    rng = np.random.default_rng(8)
+    nr, nc, mean = 1_200_000, 5000, 4
+    ci = rng.integers(0, nc, nr * mean)
+    v = rng.integers(-3, 4, nr * mean).astype(np.float32)
+    m = D.Matrix(nr, nc, np.arange(nr + 1) * mean, ci, v)
+    for nv in (2, 3, 5):
+        B = rng.integers(-3, 4, (nc, nv)).astype(np.float32)
+        d_b = D.to_bf16_device(D.DeviceArray.from_numpy(B))
+        d_C = D.DeviceArray.zeros(nr * nv)
+        m.spmm(d_b, d_C, nv, btype=D.DSPMM_R_16BF)
+        D.synchronize()
+        ref = (v[:, None] * B[ci]).reshape(nr, mean, nv).sum(1)
+        assert_bitwise(d_C.numpy().reshape(nr, nv) + 0.0, ref + 0.0, f"nv={nv}")
