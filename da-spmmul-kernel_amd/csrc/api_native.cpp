@@ -476,6 +476,12 @@ constexpr double kRowBlockMinReuse = 1.2;
 // reference-class column-major kernel: below it, the two transposes cost
 // more than they save.
 constexpr int64_t kTransposedMinWork = 1 << 20;
+// The parallel reference class in place instead (rows of like lengths or up to
+// 7 columns; us, in place / transposed copies): 40000 rows of 19, nv = 5 (3.8 M)
+// 19 / 31; 24000 rows of 60, nv = 6 (8.6 M) 35 / 29; 4893 rows of 77, nv = 9 (3.4 M)
+// 11 / 34; 12678 rows of 41, nv = 19 (9.8 M) 35 / 20.  Up to 3 columns the copies
+// never pay: 157000 rows of 35, nv = 3 69 / 134; 90^3 stencil, nv = 2 65 / 474.
+constexpr int64_t kInPlaceWork = 5500000;
 
 // Fills the tile size of a single nnz-tiled launch: at most `cap`, and small
 // enough that the launch has kTileWaves wavefronts (a wavefront owns 64 /
@@ -495,7 +501,12 @@ void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_conf
     complete_nb(full, nv, bf16);
     const int64_t slabs = div_up(nv, full.vec * full.lanes), g = 64 / full.lanes;
     c.tile_nnz = cap > 0 ? cap : full.lanes <= 4 ? 16 : full.lanes <= 32 ? 32 : 64;
-    while (c.tile_nnz > 8 && A->nnz * slabs / (g * c.tile_nnz) < kTileWaves) c.tile_nnz /= 2;
+    // a tile that just holds the longest row stays: smaller ones would split
+    // rows and need the combine launch (32^3 stencil, BF16, nv = 11: 32 per tile
+    // 10.5 us, 16 per tile 22)
+    while (c.tile_nnz > 8 && !(A->max_len <= c.tile_nnz && A->max_len > c.tile_nnz / 2) &&
+           A->nnz * slabs / (g * c.tile_nnz) < kTileWaves)
+        c.tile_nnz /= 2;
     fit_tile(nv, bf16, c);
 }
 
@@ -513,7 +524,12 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
         c.tile_nnz = kSpmvTile;
         return c;
     }
-    if (!rm && !bf16 && (int64_t)A->nnz * nv < kTransposedMinWork) {
+    const int64_t work = (int64_t)A->nnz * nv;
+    if (!rm && !bf16 && nv < 8 && (nv <= 3 || work < kInPlaceWork)) {
+        c.variant = DSPMM_VARIANT_CSR_VECTOR;
+        return c;
+    }
+    if (!rm && !bf16 && work < kTransposedMinWork) {
         c.variant = DSPMM_VARIANT_CSR_SCALAR;
         return c;
     }
@@ -522,13 +538,29 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
     c.variant = DSPMM_VARIANT_NNZ_TILED;
     c.unroll = 4;
     const bool skew = skewed(A);
-    if (nv <= 8) {
+    if ((bf16 || !rm) && nv < 8 && !skew && A->mean <= 48 && A->nr >= 512 * A->mean) {
+        // a lane per row, where enough wavefronts of them hide its gathers: 98^3
+        // stencil, nv = 2: 95, tiles 569; 38111 rows of 18, nv = 6: 13.6, 23; but
+        // 2131 rows of 25, nv = 6: 10.1, 8.3 and 24000 rows of 103, nv = 2: 231, 32;
+        // FP32 copies, 97096 rows of 34, nv = 6: 47, 77
+        c.variant = DSPMM_VARIANT_CSR_SCALAR;
+    } else if (nv <= 8) {
         // four lanes and more per tile: 64^3 stencil, nv = 8, two values a
         // lane and 32 per tile 43, eight a lane 132 (each gather instruction
         // then reaches 64 rows of B)
         c.vec = std::min(2, nv);
         single_tile(A, nv, bf16, skew ? 16 : 32, c);
     } else if (skew) {
+        if (bf16 && nv > 32)
+            // few nonzeros: more lanes per tile before shorter tiles (11257 rows,
+            // the longest 1100, nv = 81: two values a lane 15.9, eight 19.7; 8729
+            // rows, the longest 2600, nv = 122: 18.6, 31.5)
+            for (c.vec = 8; c.vec > 2; c.vec /= 2) {
+                dspmm_config full = c;
+                complete_nb(full, nv, bf16);
+                if ((int64_t)A->nnz * div_up(nv, full.vec * full.lanes) / (64 / full.lanes * 32) >= kTileWaves)
+                    break;
+            }
         single_tile(A, nv, bf16, 0, c);
     } else {
         // rows of like lengths: a group per row, without tiles and split rows
@@ -539,10 +571,22 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
         if (overflow && nv <= 32 && (bf16 || !rm)) {
             // long rows side by side would wait for one another's windows
             // (20000 rows of 100, nv = 20: 32 / 66, sliced 38)
-            if (bf16) c.vec = nv <= 16 ? 1 : 2;
-            c.unroll = bf16 ? 4 : 8;
-            c.tile_nnz = 128;
-            fit_tile(nv, bf16, c);
+            if (!bf16 && work < kInPlaceWork) {
+                c.variant = DSPMM_VARIANT_CSR_VECTOR;
+            } else if (bf16 && A->mean <= 64 && A->nnz >= 2000000) {
+                // sliced: 84200 rows of 48, nv = 28: 36, tiles 76 and more
+                c.variant = DSPMM_VARIANT_CSR_SCALAR;
+                c.tile_nnz = 1;
+            } else if (bf16) {
+                // 4120 rows of 91, nv = 12: 10.3, 128 per tile 31.4; 3368 rows of 70,
+                // nv = 30: 10.1, 31.1
+                c.vec = 4;
+                single_tile(A, nv, bf16, A->max_len <= 32 ? 32 : 16, c);
+            } else {
+                c.unroll = 8;
+                c.tile_nnz = 128;
+                fit_tile(nv, bf16, c);
+            }
         } else {
             c.variant = DSPMM_VARIANT_CSR_SCALAR;
             c.unroll = bf16 || !rm ? 4 : 0;
@@ -553,6 +597,39 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
         }
     }
     return c;
+}
+
+// The selector's picks were measured before the reference classes gave long rows
+// to whole wavefronts and blocks and gathered for short ones with all lanes; where these are
+// now clearly ahead they replace the pick (row-major, FP32; us, here / pick).
+void adjust_pick(dspmm_matrix_s *A, int nv, dspmm_config &c) {
+    if (c.variant == DSPMM_VARIANT_RING) return;
+    const bool skew = skewed(A);
+    int v = c.variant;
+    int unroll = 0;
+    if (nv == 1) {
+        // rows that the tiles queue one per wavefront, off the diagonal slices:
+        // 20490 rows of 22 4.3 / 7.0, 143583 rows of 23 12.8 / 19.8, 107445 rows of 66 38.7 / 36.6
+        if (skew || A->mean <= 16 || A->mean > 64 || column_reuse(A) >= kRowBlockMinReuse) return;
+        v = DSPMM_VARIANT_CSR_VECTOR;
+    } else if (nv <= 8) {
+        v = DSPMM_VARIANT_CSR_VECTOR;          // skewed rows: 0.58 of the pick's time, at most 0.66
+        if (!skew && A->mean <= 32 && (int64_t)A->nnz * nv >= 16000000 && column_reuse(A) >= kRowBlockMinReuse) {
+            // neighbouring rows share B rows: 74^3 stencil, nv = 3: 32 / 55; 64^3, nv = 5: 26 / 36
+            // (78714 rows of 72 on 2463 columns, nv = 5: 98 / 52)
+            if (nv <= 3) v = DSPMM_VARIANT_CSR_SCALAR;
+            if (nv >= 5) { v = DSPMM_VARIANT_CSR_SCALAR; unroll = 4; }
+        }
+    } else if (nv <= 32 && v == DSPMM_VARIANT_CSR_VECTOR && !skew && A->mean <= 32 && A->nnz >= 400000) {
+        // 65^3 stencil, nv = 15: 27 / 75; 58782 rows of 20, nv = 15: 20 / 24; below that many
+        // nonzeros, or with longer rows, no faster
+        v = DSPMM_VARIANT_CSR_SCALAR;
+    } else {
+        return;
+    }
+    c = dspmm_config{};
+    c.variant = v;
+    c.unroll = unroll;
 }
 
 // Row-major-only native kernels: on column-major operands they run on
@@ -1014,7 +1091,10 @@ dspmm_config resolve(dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_
         // the selector was measured with FP32 B; with BF16 B only its B-row
         // ring picks carry over (the ring takes either, with the vector width
         // left to the operands)
-        if (bt == DSPMM_R_32F) return c;
+        if (bt == DSPMM_R_32F) {
+            adjust_pick(A, nv, c);
+            return c;
+        }
         if (c.variant == DSPMM_VARIANT_RING) {
             c.vec = 0;
             c.lanes = 0;
