@@ -175,7 +175,7 @@ private:
 // pass over B and C.  So the line lies at a number of products, lower where B
 // is too large for the L2s.  In place / copies, us: 131072 rows of 24, nv = 32
 // (100 M products) 464 / 76; 16384 rows of 32, nv = 8 (4.2 M) csr_vector 15 / 12,
-// coo 21 / 14; 32^3 stencil, nv = 8 (6.6 M) csr_vector 11.5 / 11.7; 5000 rows of 12 over
+// coo 21 / 14; 39^3 stencil, nv = 4 (6.1 M) csr_vector 10 / 13; 5000 rows of 12 over
 // 250000 columns, nv = 16 (0.96 M, B of 16 MB) csr_vector 18 / 14; 131072 rows of 6,
 // nv = 4 (3.1 M) csr_scalar 17 / 16, coo 18 / 21.  Two columns share their lines less:
 // power law, nv = 2 (6.4 M), coo 33 / 37.
@@ -186,7 +186,7 @@ int flip_columns(int which, int nr, int nc, int nnz, int nv, bool null_stream) {
     if (which == K_SPMM_CSR_SCALAR_COL)
         pays = products >= (null_stream ? 4.1 : 6.0);
     else if (which == K_SPMM_CSR_VECTOR_COL)
-        pays = null_stream ? products >= 5.0 || (products >= 1.0 && b >= 4.0)
+        pays = null_stream ? products >= 8.0 || (products >= 5.0 && b >= 1.0) || (products >= 1.0 && b >= 4.0)
                            : products >= 14.0 || (products >= 3.4 && b >= 1.5);
     else if (nv == 2)
         pays = products >= (null_stream ? 16.0 : 24.0);

@@ -210,7 +210,8 @@ struct LongRow {
 
 // ===========================================================================
 // Row-balanced, sequential reduction, row-major, for few columns
-// (spmv_csr_scalar; spmm_csr_scalar_row with L * VW <= 8).  A wavefront owns
+// (spmv_csr_scalar; spmm_csr_scalar_row with L * VW <= 8 and few
+// rows, or with 4).  A wavefront owns
 // G consecutive rows, at most 64 / (L * VW).  In windows of PW of their pairs,
 // every lane gathers B for its share of the window at once, the next window's
 // while this one is added, and the products go to the wavefront's LDS region,
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream(int nr, int nv, int64_t l
 
 // ===========================================================================
 // Row-balanced, sequential reduction, row-major (spmm_csr_scalar_row with more
-// than 8 columns).  A group of L lanes owns one row; each lane
+// than 8 columns, or more than 4 and many rows).  A group of L lanes owns one row; each lane
 // owns VW consecutive columns of the slab.  The block's rows' nonzeros are
 // staged through LDS in windows; every lane reads its row's (col, val) as an
 // LDS broadcast within its group.  Overwrites every row (empty rows -> 0).
@@ -1135,11 +1136,17 @@ int stream_rows(int W, int nnz, int nr) {
     return std::max(1, std::min(kWave / W, (int)(0.75 * stream_pairs(W) / mean)));
 }
 
+// Rows from which 5 to 8 columns run with a lane group per row (k_csr_scalar_rm):
+// below, too few wavefronts of 32 rows hide their gathers.  nv = 8, stream / groups:
+// 64^3 stencil 37.6 / 19.9 us, power law of 262144 rows 197 / 116, 131072 rows of 6
+// 9.9 / 8.7, 100000 of 20 12.4 / 12.5; power law of 60916 27 / 42, 16384 rows of 32 6.2 / 14.8.
+constexpr int kGroupRows8 = 98304;
+
 dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st) {
     const Slab s = make_slab(nv, choose_vw_any(nv, 4));
-    if (s.width <= 8) {
+    if (s.width <= (nr >= kGroupRows8 ? 4 : 8)) {
         with_vw(s.vw, [&](auto vw_c) {
             with_lanes(s.lanes, [&](auto l_c) {
                 constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
@@ -1160,7 +1167,7 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
     with_vw(s.vw, [&](auto vw_c) {
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-            if constexpr (VW_ * L_ > 8) {
+            if constexpr (VW_ * L_ >= 8) {
                 // scouts: one per kScoutRows rows and kScoutCols columns; a whole
                 // number per XCD, which leaves xcd_remap its meaning
                 const int parts = div_up(std::min(nv, s.width), std::min(s.width, kScoutCols));

@@ -105,3 +105,18 @@ def test_csr_scalar_long_rows_bit_exact(kind):
         assert st == 0, D.status_string(st)
         D.synchronize()
         assert_bitwise(c.output(nv), c.ref(D.DENSE_ROW_MAJOR, nv)[0], f"{kind} nv={nv}")
+
+
+def test_csr_scalar_many_rows_few_columns():
+    """Enough rows for a lane group each at 5 to 8 columns, some of them long."""
+    rng = np.random.default_rng(14)
+    lens = rng.integers(0, 5, 98304)
+    lens[[0, 511, 40000, 98303]] = [97, 1025, 300, 1300]
+    c = float_case("many_rows", lens, 3000, 8)
+    for nv in (4, 5, 6, 7, 8):
+        c.fill_output(np.nan)
+        st = D.launch("spmm_csr_scalar_row", c.nr, c.nc, c.nnz, nv, c.d_rp, c.d_ri, c.d_ci, c.d_v,
+                      c.d_B, c.d_C)
+        assert st == 0, D.status_string(st)
+        D.synchronize()
+        assert_bitwise(c.output(nv), c.ref(D.DENSE_ROW_MAJOR, nv)[0], f"many rows nv={nv}")
