@@ -15,22 +15,38 @@
 
 namespace dspmm {
 
+// Tiles of a batch's items.  One launch keeps as many wavefronts on a CU as its
+// LDS, sized for the item that stages most, and its registers allow; so every
+// item stages at most kBatchPairs nonzeros per wavefront, which with four
+// gathers in flight (two of eight values each for BF16) fits 24 wavefronts (16
+// for BF16), and tiles end at kBatchTile.  An item whose B is beyond an XCD's L2
+// (kBatchL2 bytes) runs in slabs of kBatchSlab columns, one after the other or
+// on XCDs of their own.  Measured, 16 nonzeros per lane and eight gathers before:
+// FP32, 128 / 35 / 66 items 1352 / 574 / 452 us -> 1100 / 393 / 377 (without the slabs
+// 1287 / 573); slabs of 32 columns with eight gathers 1618, of 96 with four 1287; 384
+// nonzeros 1216, 640 1246.  BF16, 91 / 50 / 17 items 855 / 498 / 137.  Plain tiles
+// of 768 with four gathers 715 / 407 / 137, with two 640 / 365 / 122, tiles of at most
+// 128 with four 738 / 381 / 85; slabs of 128 columns 763.
+constexpr int kBatchPairs = 512, kBatchPairsBf16 = 768;
+constexpr int kBatchTile = 128;
+constexpr double kBatchL2 = 4e6;
+constexpr int kBatchSlab = 64;
+
 dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc, const void *B,
                              const void *C, dspmm_dtype_t btype, ItemFragment &f) {
     const bool bf16 = btype == DSPMM_R_16BF;
     f = ItemFragment{};
     if (!A || nv < 1 || ldb < nv || ldc < nv) return DSPMM_STATUS_INVALID_VALUE;
     std::lock_guard<std::mutex> lk(A->mu);
-    // The static nnz-tiled default: configurations tuned on single
-    // launches (where one matrix has the whole GPU and its caches) make
-    // the batch slower, not faster.
+    // Not the configurations tuned on single launches, where one matrix has the
+    // whole GPU and its caches: they make the batch slower.
     dspmm_config c{};
     c.variant = DSPMM_VARIANT_NNZ_TILED;
     complete_nb(c, nv, bf16);
-    if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) {
-        c.tile_nnz = 16;
-        if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) return DSPMM_STATUS_NOT_SUPPORTED;
-    }
+    if (!bf16 && (double)A->nc * nv * sizeof(float) > kBatchL2 && c.vec * c.lanes > kBatchSlab)
+        c.lanes = kBatchSlab / c.vec;
+    c.tile_nnz = std::max(8, std::min(kBatchTile, (bf16 ? kBatchPairsBf16 : kBatchPairs) * c.lanes / kWave));
+    if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) return DSPMM_STATUS_NOT_SUPPORTED;
     NbPlan *plan = nullptr;
     dspmm_status_t st = get_plan(A, c.tile_nnz, &plan);
     if (st != DSPMM_STATUS_SUCCESS) return st;

@@ -209,7 +209,9 @@ __device__ __forceinline__ void with_class(int cls, F &&f) {
 // matrices, whose B rows then stay in that XCD's L2).  A wavefront finds its
 // first unit's segment by binary search and then walks forward; it stages
 // into and reads from its own LDS region only, so wavefronts never wait for
-// one another.
+// one another.  The gathers in flight per lane set the registers and so the
+// wavefronts per SIMD (FP32: eight 97 registers and 4, four 73 and 6, two 64 and 8;
+// BF16: 168 and 3, 128 and 4, 116 and 4).
 template <typename TB>
 __global__ __launch_bounds__(kBlock) void k_nnz_tiled_batched(const ItemDesc *__restrict__ items,
                                                               const int4 *__restrict__ segs,
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void k_nnz_tiled_batched(const ItemDesc *__
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
             if constexpr (sizeof(TB) == 4 && VW_ == 8) {
             } else {
-                process_tiles<TB, VW_, L_, 8>(d, t0, tcount, slab, w);
+                process_tiles<TB, VW_, L_, sizeof(TB) == 4 ? 4 : 2>(d, t0, tcount, slab, w);
             }
         });
         wave_lds_sync();                            // LDS is restaged for the next unit
