@@ -608,9 +608,11 @@ void adjust_pick(dspmm_matrix_s *A, int nv, dspmm_config &c) {
     int v = c.variant;
     int unroll = 0;
     if (nv == 1) {
-        // rows that the tiles queue one per wavefront, off the diagonal slices:
-        // 20490 rows of 22 4.3 / 7.0, 143583 rows of 23 12.8 / 19.8, 107445 rows of 66 38.7 / 36.6
-        if (skew || A->mean <= 16 || A->mean > 64 || column_reuse(A) >= kRowBlockMinReuse) return;
+        // no products through LDS where many rows are summed by several lanes, off
+        // the diagonal slices: 110136 rows of 30 15.9 / 18.2, 143583 of 23 13.2 /
+        // 15.1; 107445 of 66 36.8 / 33.6, 12691 of 50 the same
+        if (skew || A->mean <= 20 || A->mean > 64 || A->nnz < 2000000 ||
+            column_reuse(A) >= kRowBlockMinReuse) return;
         v = DSPMM_VARIANT_CSR_VECTOR;
     } else if (nv <= 8) {
         v = DSPMM_VARIANT_CSR_VECTOR;          // skewed rows: 0.58 of the pick's time, at most 0.66
@@ -1101,7 +1103,9 @@ dspmm_config resolve(dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_
             return c;
         }
     }
-    return heuristic(A, layout, nv, bt);
+    c = heuristic(A, layout, nv, bt);
+    if (nv == 1 && layout == DENSE_ROW_MAJOR && bt == DSPMM_R_32F) adjust_pick(A, nv, c);
+    return c;
 }
 
 // Workspace of a resolved configuration (caller holds A->mu).
@@ -1296,8 +1300,11 @@ dspmm_status_t dspmm_matrix_prepare(dspmm_matrix_t A, DenseLayout layout, int nv
     const RunMode mode = (flags & DSPMM_PREPARE_HANDLE_BUFFERS) ? kRunPrepare : kRunPlans;
     float *Cw = const_cast<float *>(C);
     st = run_ex(A, layout, nv, B, ldb, btype, Cw, ldc, c, nullptr, 0, nullptr, nullptr, mode);
-    if (auto_cfg) {
-        // the static default AUTO falls back to when the pick cannot run
+    if (auto_cfg && (st != DSPMM_STATUS_SUCCESS || c.variant == DSPMM_VARIANT_NNZ_CACHED ||
+                     c.variant == DSPMM_VARIANT_RING)) {
+        // the static default AUTO falls back to when the pick cannot run: the
+        // kernels that stage B in LDS refuse operands by their alignment, the
+        // others take any once they take these sizes
         const dspmm_status_t sh = run_ex(A, layout, nv, B, ldb, btype, Cw, ldc,
                                          heuristic(A, layout, nv, btype), nullptr, 0, nullptr,
                                          nullptr, mode);

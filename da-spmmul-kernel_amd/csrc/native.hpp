@@ -157,6 +157,7 @@ dspmm_status_t launch_diag_fill(const int *off, const int *diags, int ndiags, co
                                 float4 *vals, uint32_t *didx, hipStream_t st);
 constexpr int kSpmvRowMax = 256;   // longest row of a multi-row SpMV tile
 constexpr int kSpmvThreadRow = 16; // longest row summed by one thread
+constexpr int kSpmvRowLanes = 16;  // lanes on a longer row of a tile
 constexpr int kSpmvLongTiles = 16; // rows up to 16 T nonzeros get one workgroup
 bool spmv_tile_ok(int T);          // SpMV tile sizes with a kernel: 512 .. 4096
 size_t nnz_tiled_lds_bytes(int lanes, int S);

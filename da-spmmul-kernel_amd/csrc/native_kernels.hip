@@ -351,8 +351,11 @@ __global__ __launch_bounds__(kBlock) void k_split_combine_batched(const ItemDesc
 // and writes the products to LDS.  After one barrier, thread i sums row
 // r0+i from LDS in nonzero order if the row has at most kSpmvThreadRow
 // nonzeros -- bit-exact with the host loop; longer rows of the tile are
-// queued in LDS and taken one per wavefront: lane l sums products l, l+64,
-// ... in order, then a fixed butterfly.  A tile of one longer row (up to
+// queued in LDS and taken by kSpmvRowLanes lanes each: lane l sums products l,
+// l + kSpmvRowLanes, ... in order, then a fixed butterfly.  (A wavefront per row
+// made rows of 17 to 100 the kernel's time: 143583 rows of 23 19.8 us, 16 lanes
+// 15.4, 8 14.8; 39950 of 22 8.8, 6.9, 6.7; power law with rows of up to 500 5.1, 5.1,
+// 5.8.)  A tile of one longer row (up to
 // kSpmvLongTiles * T nonzeros) or of one T-chunk of a still longer row is
 // reduced by the workgroup: thread t sums products t, t+256, t+512, ... in
 // that order, then a pairwise tree; the result goes to y (whole row) or to
@@ -410,13 +413,13 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
             }
         }
         __syncthreads();
-        const int wv = t / kWave, ln = t % kWave;
-        for (int k = wv; k < nlong; k += kBlock / kWave) {      // wave-uniform
+        constexpr int LR = kSpmvRowLanes;
+        for (int k = t / LR; k < nlong; k += kBlock / LR) {
             const int4 q = lrange[k];
             float s = 0.f;
-            for (int p = q.x + ln; p < q.y; p += kWave) s = s + prod[p];
-            s = butterfly_sum<1, kWave>(s);
-            if (ln == 0) d.C[(int64_t)q.z * d.ldc] = s;
+            for (int p = q.x + t % LR; p < q.y; p += LR) s = s + prod[p];
+            s = group_sum<LR>(s);
+            if (t % LR == 0) d.C[(int64_t)q.z * d.ldc] = s;
         }
         return;
     }
