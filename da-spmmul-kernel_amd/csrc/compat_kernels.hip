@@ -670,9 +670,9 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
 //
 // What bounds it: the atomics, then the gathers.  L2 takes about 19 G
 // atomic accesses a second, one per 64-byte line that an instruction touches,
-// so a run is added with its columns contiguous over the lanes (through LDS
-// where a lane holds several columns), and runs are as long as the nonzeros
-// of a wavefront allow.  Both reference algorithms run this kernel: without
+// so finished runs are added by the whole wavefront with their columns contiguous
+// over the lanes (through LDS where a lane holds several columns), and runs are as
+// long as the nonzeros of a wavefront allow.  Both reference algorithms run this kernel: without
 // the join a row costs an atomic per group (64^3 27-point stencil, nv = 64:
 // 395 us against 279 with it, before the contiguous additions; 133 with both;
 // an atomic per eight nonzeros and four strided ones per float4 took 947 and
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
     __shared__ int s_row[WPB][PADN];
     __shared__ int s_col[WPB][PADN];
     __shared__ float s_val[WPB][PADN];
-    __shared__ __align__(16) float s_flush[WPB][VW > 1 ? kWave * VW : 1];
+    __shared__ __align__(16) float s_flush[WPB][VW > 1 ? kWave * VW : 1];   // a group's columns in order
     const int wv = (int)threadIdx.x / kWave, ln = lane_id();
     const int64_t base = ((int64_t)xcd_remap(blockIdx.x, gridDim.x) * WPB + wv) * CH;
     if (base >= nnz) return;                   // the whole wavefront leaves; no barrier follows
@@ -710,31 +710,46 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
         s_val[wv][j] = NT ? ld_stream(values + p) : values[p];
     }
     wave_lds_sync();
+    constexpr int W = L * VW;                  // columns of a group
     const int g = ln / L;
     const int col0 = blockIdx.y * slab_w + (ln % L) * VW;
     const bool colok = col0 < nv;
     const int n = max(0, min(NE, cnt - g * NE));   // nonzeros of this group
-    const int *sr = s_row[wv] + g * (NE + 1), *sc = s_col[wv] + g * (NE + 1);
-    const float *sv = s_val[wv] + g * (NE + 1);
+    const int at = n > 0 ? g * (NE + 1) : 0;       // (without any: the first group's, not added)
+    const int *sr = s_row[wv] + at, *sc = s_col[wv] + at;
+    const float *sv = s_val[wv] + at;
     const float *__restrict__ Bc = B + (colok ? col0 : 0);
-    // Adds v to row r of C.  An atomic instruction costs one L2 access per
-    // 64-byte line it touches, so the group's lanes trade their VW consecutive
-    // columns for columns L apart (through LDS) and each instruction covers L
-    // consecutive floats.
-    auto flush = [&](int r, const float (&v)[VW]) {
-        float *c = C + (int64_t)r * ldc + blockIdx.y * slab_w;
-        const int l = ln % L;
+    float *__restrict__ Cs = C + blockIdx.y * slab_w;
+    const int ncol = nv - (int)blockIdx.y * slab_w;
+    // Adds v to row r of C for the groups with `mine`.  An atomic instruction
+    // costs one L2 access per 64-byte line it touches, so the wavefront's lanes
+    // take the groups' columns in order, from LDS: 64 / W groups to an instruction.
+    auto flush = [&](bool mine, int r, const float (&v)[VW]) {
         if constexpr (VW == 1) {
-            if (colok) unsafeAtomicAdd(c + l, v[0]);
+            if (mine && colok) unsafeAtomicAdd(Cs + (int64_t)r * ldc + ln % L, v[0]);
         } else {
-            float *f = s_flush[wv] + (ln - l) * VW;
-            wave_lds_sync();                   // the group's previous flush has been read
-            store_vec<VW>(f + l * VW, v);
+            uint64_t m = __ballot(mine && ln % L == 0);
+            if (m == 0) return;
+            wave_lds_sync();                   // the previous flush has been read
+            if (mine) store_vec<VW>(s_flush[wv] + ln * VW, v);
             wave_lds_sync();
-            const int ncol = nv - (int)blockIdx.y * slab_w;
+            constexpr int P = W < kWave ? kWave / W : 1;
+            while (m) {
+                int o = -1;                    // first lane of the group whose columns this lane adds
 #pragma unroll
-            for (int k = 0; k < VW; k++)
-                if (k * L + l < ncol) unsafeAtomicAdd(c + k * L + l, f[k * L + l]);
+                for (int k = 0; k < P; k++) {
+                    if (m && ln / W % P == k) o = __builtin_ctzll(m);
+                    m &= m - 1;                // (no bit left: stays 0)
+                }
+                const int row = __shfl(r, max(o, 0));
+                if (o >= 0) {
+#pragma unroll
+                    for (int k = 0; k < W; k += kWave) {
+                        const int c = k + ln % (W < kWave ? W : kWave);
+                        if (c < ncol) unsafeAtomicAdd(Cs + (int64_t)row * ldc + c, s_flush[wv][o * VW + c]);
+                    }
+                }
+            }
         }
     };
     int cur = INT_MAX, first = INT_MAX;        // rows of the running and of the first run
@@ -743,11 +758,11 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
 #pragma unroll
     for (int k = 0; k < VW; k++) acc[k] = head[k] = 0.f;
     if (n > 0) cur = first = sr[0];
-    for (int e = 0; e < n; e += UNR) {
+    for (int e = 0; e < min(NE, cnt); e += UNR) {  // the same in every group
         float bv[UNR][VW];
 #pragma unroll
         for (int u = 0; u < UNR; u++)          // padded with the last entry: no branch around loads
-            load_vec<VW>(bv[u], Bc + (int64_t)sc[min(e + u, n - 1)] * ldb);
+            load_vec<VW>(bv[u], Bc + (int64_t)sc[max(0, min(e + u, n - 1))] * ldb);
         // summed per block of UNR, the blocks' sums then in order: a run of 32
         // rounds no worse than the scan over eight lanes that it replaces
         float part[VW];
@@ -755,23 +770,28 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
         for (int k = 0; k < VW; k++) part[k] = 0.f;
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
-            if (e + u < n) {
-                const int r = sr[e + u];
-                const float a = sv[e + u];
-                if (r != cur) {
+            const bool in = e + u < n;
+            const int r = in ? sr[e + u] : cur;
+            const float a = in ? sv[e + u] : 0.f;
+            const bool ends = r != cur;
+            if (__ballot(ends)) {
+                if (ends) {
 #pragma unroll
                     for (int k = 0; k < VW; k++) acc[k] += part[k];
                     if (one) {                 // the first run may continue the previous group's
 #pragma unroll
                         for (int k = 0; k < VW; k++) head[k] = acc[k];
-                        one = false;
-                    } else {
-                        flush(cur, acc);
                     }
+                }
+                flush(ends && !one, cur, acc);
+                if (ends) {
+                    one = false;
                     cur = r;
 #pragma unroll
                     for (int k = 0; k < VW; k++) acc[k] = part[k] = 0.f;
                 }
+            }
+            if (in) {
 #pragma unroll
                 for (int k = 0; k < VW; k++) part[k] = __builtin_fmaf(a, bv[u][k], part[k]);
             }
@@ -779,12 +799,8 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
 #pragma unroll
         for (int k = 0; k < VW; k++) acc[k] += part[k];
     }
-    if constexpr (L == kWave) {
-        if (n > 0) {
-            if (!one) flush(first, head);
-            flush(cur, acc);
-        }
-    } else {
+    bool ends = n > 0;
+    if constexpr (L < kWave) {
         // acc becomes the sum of a row's last runs up to this group, as long as
         // the groups between hold nothing else
         const int prow = __shfl_up(cur, L);
@@ -795,12 +811,12 @@ __global__ __launch_bounds__(kBlock) void k_coo_rm(int nnz, int nv, int64_t ldb,
             const float p = __shfl_up(acc[k], L);
             if (joins && !one) head[k] += p;
         }
-        if (n > 0 && !one) flush(first, head);
         // the last group of a row's runs adds it (the next group's head takes it otherwise)
         const int nfirst = __shfl_down(first, L);
-        const bool ends = ln >= kWave - L || nfirst != cur;
-        if (n > 0 && ends) flush(cur, acc);
+        ends = ends && (ln >= kWave - L || nfirst != cur);
     }
+    flush(n > 0 && !one, first, head);
+    flush(ends, cur, acc);
 }
 
 // ===========================================================================
@@ -1238,6 +1254,7 @@ dspmm_status_t csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64
 // runs are then cut; at most kCooPairs per wavefront, which its LDS holds.
 constexpr int64_t kCooWaves = 8192;
 constexpr int kCooPairs = 512;
+constexpr int kCooRun = 16;      // nonzeros per row from which runs are long
 
 template <int VW, int L, int NE>
 void launch_coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx, const int *colIdx,
@@ -1268,15 +1285,17 @@ dspmm_status_t coo_spmv(int nnz, int64_t ldx, int64_t ldy, const int *rowIdx, co
 }
 
 // ALG_COO_SCALAR and ALG_COO_VECTOR, row-major.
-dspmm_status_t coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
+dspmm_status_t coo_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowIdx,
                       const int *colIdx, const float *values, const float *B, float *C,
                       hipStream_t st) {
     if (nv == 1) return coo_spmv(nnz, ldb, ldc, rowIdx, colIdx, values, B, C, st);
-    // The widest vectors that leave a group 16 lanes, a 64-byte line of C per
-    // atomic instruction: at nv = 32 two floats (stencil 64^3 90 us, power law
-    // 75 us; four floats 93 and 88, one 128 and 78), at nv = 64 four
-    // (stencil 133 us; two 157, one 243).
-    const int widest = nv >= 64 ? 4 : nv >= 32 ? 2 : 1;
+    // Wide vectors gather more rows of B per instruction, narrow ones leave
+    // fewer groups to share a flush: four floats where runs are long, else the
+    // widest that leaves a group 16 lanes.  nv = 32, four / two floats: 64^3 stencil 57.8 /
+    // 82.2 us, 16384 rows of 32 7.7 / 10.5, 100000 of 20 20.1 / 26.6, power law of mean 12 73.1 /
+    // 70.1; nv = 16, four / one: 45.0 / 65.3, 6.5 / 8.7, 15.7 / 21.3, 59.1 / 56.2.
+    const bool runs = nnz >= (int64_t)kCooRun * nr && (nv >= 16 || (nv >= 8 && nnz >= 800000));
+    const int widest = nv >= 64 || runs ? 4 : nv >= 32 ? 2 : 1;
     const Slab s = make_slab(nv, choose_vw(nv, ldb, ldc, B, C, 4, widest));
     int ne = 32;
     while (ne > 8 && (ne * (kWave / s.lanes) > kCooPairs ||
@@ -1285,7 +1304,7 @@ dspmm_status_t coo_rm(int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowI
     with_vw(s.vw, [&](auto vw_c) {
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-            if constexpr (L_ >= (VW_ > 1 ? 16 : 2)) {
+            if constexpr (VW_ * L_ >= 2) {
                 switch (ne) {
                 case 32: launch_coo_rm<VW_, L_, 32>(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st, s); break;
                 case 16: launch_coo_rm<VW_, L_, 16>(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st, s); break;
@@ -1404,7 +1423,7 @@ dspmm_status_t launch_compat_flipped(int which, int nr, int nc, int nnz, int nv,
         if (s == DSPMM_STATUS_SUCCESS && coo)
             s = launch_fill_zero(Ct, (size_t)nr * (size_t)w * sizeof(float), st);
         if (s != DSPMM_STATUS_SUCCESS) break;
-        if (coo) s = coo_rm(nnz, w, w, w, rowIdx, colIdx, values, Bt, Ct, st);
+        if (coo) s = coo_rm(nr, nnz, w, w, w, rowIdx, colIdx, values, Bt, Ct, st);
         else if (which == K_SPMM_CSR_SCALAR_COL)
             s = csr_scalar_rm(nr, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st);
         else s = csr_vector_rm(nr, nc, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st, 0);
@@ -1434,7 +1453,7 @@ dspmm_status_t launch_compat(int which, int nr, int nc, int nnz, int nv, int64_t
     case K_SPMM_COO_SCALAR_ROW:
     case K_SPMV_COO_VECTOR:
     case K_SPMM_COO_VECTOR_ROW:
-        return coo_rm(nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
+        return coo_rm(nr, nnz, nv, ldb, ldc, rowIdx, colIdx, values, B, C, st);
     case K_SPMM_CSR_SCALAR_COL:
         return csr_scalar_cm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
     case K_SPMM_CSR_VECTOR_COL:

@@ -146,3 +146,18 @@ def test_coo_in_any_order():
             launch(c, name, nv)
             D.synchronize()
             assert_bitwise(c.output(nv) + 0.0, c.ref(layout, nv)[0] + 0.0, f"{name} nv={nv}")
+
+
+@pytest.mark.parametrize("kind", ["even_16", "ends_together", "sparse_runs"])
+def test_coo_long_runs(kind):
+    """Runs that several groups finish at once and at different steps, four
+    columns to a lane."""
+    rng = np.random.default_rng(3)
+    lens = {"even_16": np.full(777, 16), "ends_together": np.tile([8, 24, 32, 8], 1500),
+            "sparse_runs": rng.integers(0, 3, 5000) * 27}[kind]
+    c = int_case(kind, lens, 400, 132)
+    for nv in (4, 8, 12, 16, 20, 32, 48, 64, 68, 128, 132):
+        c.fill_output(1.0)
+        launch(c, "spmm_coo_vector_row", nv)
+        D.synchronize()
+        assert_bitwise(c.output(nv) + 0.0, c.ref(D.DENSE_ROW_MAJOR, nv)[0] + 1.0, f"{kind} nv={nv}")
