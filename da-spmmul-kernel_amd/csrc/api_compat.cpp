@@ -58,7 +58,7 @@ bool is_col(int which) {
 //     its last launch is enqueued.
 //   * On any other stream a call takes a block before its launches and gives it
 //     back behind them, so that streams and threads never share one.  That
-//     costs a call 10 us, mostly the marker behind its work.
+//     costs a call 18 us, mostly the marker behind its work.
 // Free blocks beyond kScratchKept go back to the device at the next
 // synchronisation; dspmm_release_scratch, and dspmm_device_alloc where it finds
 // the memory short, give back the rest.
@@ -171,7 +171,7 @@ private:
 // (launch_compat_flipped); 0: in place.  In place every product costs a line of
 // B (about 0.22 M gathers a microsecond where B is random, twice that where the
 // L2s hold it), the copies cost three to four launches (10 to 13 us, and on a
-// stream other than the legacy default one 12 us more for the scratch) and a
+// stream other than the legacy default one 18 us more for the scratch) and a
 // pass over B and C.  So the line lies at a number of products, lower where B
 // is too large for the L2s.  In place / copies, us: 131072 rows of 24, nv = 32
 // (100 M products) 464 / 76; 16384 rows of 32, nv = 8 (4.2 M) csr_vector 15 / 12,
