@@ -14,6 +14,19 @@
 
 namespace dspmm {
 
+// Stable by falling number of chunks: counted, since power-law matrices have
+// tens of thousands of split rows with few different numbers.
+static void most_chunks_first(std::vector<int4> &splits) {
+    int most = 0;
+    for (const int4 &s : splits) most = std::max(most, s.w);
+    std::vector<int> at((size_t)most + 2, 0);        // at[w + 1]: splits of more than w chunks
+    for (const int4 &s : splits) at[(size_t)s.w]++;
+    for (int w = most; w >= 0; w--) at[(size_t)w] += at[(size_t)w + 1];
+    std::vector<int4> out(splits.size());
+    for (const int4 &s : splits) out[(size_t)at[(size_t)s.w + 1]++] = s;
+    splits.swap(out);
+}
+
 // Cuts rows [0, nr) into tiles of <= S nonzeros and <= S rows that start and
 // end on row boundaries; a row longer than S becomes ceil(len/S) chunks of
 // S nonzeros, each with its own carry slot, and one split record.
@@ -22,6 +35,7 @@ void build_tiles(const std::vector<int> &rp, int nr, int S, std::vector<int4> &t
     tiles.clear();
     splits.clear();
     nslots = 0;
+    tiles.reserve((size_t)rp[(size_t)nr] / (size_t)S * 3 / 2 + (size_t)nr / (size_t)S + 16);
     int r = 0;
     while (r < nr) {
         const int len = rp[(size_t)r + 1] - rp[(size_t)r];
@@ -46,8 +60,7 @@ void build_tiles(const std::vector<int> &rp, int nr, int S, std::vector<int4> &t
     // Split rows with the most chunks first: their combine is the longest,
     // so it starts first.  A row's own combine order does not depend on
     // its place in this list.
-    std::stable_sort(splits.begin(), splits.end(),
-                     [](const int4 &a, const int4 &b) { return a.w > b.w; });
+    most_chunks_first(splits);
 }
 
 void build_spmv_tiles(const std::vector<int> &rp, int nr, int T, int row_max,
