@@ -77,16 +77,51 @@ __device__ __forceinline__ void stage_window(int *s_col, float *s_val, const int
 // gathering: at least kLongRow nonzeros and twice the block's mean row, so
 // that the row's own group would otherwise work on alone.
 constexpr int kLongRow = 96;
-// The longest rows (kScoutRow nonzeros or more) are found and summed by the
-// first blocks of the launch, each of which looks at kScoutRows rows and sums
+// The longest rows (kScoutRow nonzeros or more, and kScoutMean times the mean,
+// so that most blocks have none) are found and summed by the first blocks of
+// the launch, the scouts, each of which looks at up to kScoutRows rows and sums
 // kScoutCols of their columns: begun last, or with the gathers of one block
 // only, one of them would set the kernel's time.  On a power-law matrix
 // (262144 rows, the longest 4900, nv = 64): 32 columns 160 us, 16
 // (64-byte gathers) 192, without these blocks 203, with a lane group alone on
-// each row 660.
+// each row 660.  A scout's rows lie far apart, since long rows may be neighbours:
+// 65536 such rows sorted by length, nv = 32, csr_vector 73 us, with consecutive
+// rows to a scout 2300.  128 rows each instead of 512 are faster there (65536 rows,
+// nv = 32, csr_vector 39 and 54 us) and slower on rows of like lengths, for whose
+// blocks so many scouts leave less room (65536 rows of 12 to 24, nv = 16: 5 to 10%).
 constexpr int kScoutRow = 1024;
+constexpr int kScoutMean = 8;
 constexpr int kScoutRows = 512;
 constexpr int kScoutCols = 32;
+
+// The scouts of a launch: their number and the length from which rows are theirs.
+struct Scouts {
+    int blocks = 0, row = INT_MAX;
+};
+
+// One of the rows that scout `i` of `n` looks at: its k-th.  Many rows go in
+// fours, since one by one their lines of rowPtr are read 32 times (power law of
+// 262144 rows, nv = 1, csr_vector: 27.3 us, in fours 24.5).
+__device__ __forceinline__ int64_t scout_at(int i, int n, int nr, int k) {
+    const int w = nr / n >= 128 ? 4 : 1;
+    return ((int64_t)(k / w) * n + i) * w + k % w;
+}
+constexpr int kScoutList = kScoutRows + 4;     // rows that one scout may look at
+
+// Collects the scout's long rows (their k's) in s_scout; *s_n is their number.
+// Every thread calls it (barriers inside).
+__device__ __forceinline__ void scout_look(int i, int n, int nr, const int *__restrict__ rowPtr,
+                                           int scout_row, uint16_t *s_scout, int *s_n) {
+    if (threadIdx.x == 0) *s_n = 0;
+    __syncthreads();
+    for (int k = threadIdx.x; scout_at(i, n, nr, k) < nr; k += kBlock) {   // k < kScoutList
+        const int64_t q = scout_at(i, n, nr, k);
+        const auto p = *reinterpret_cast<const VecAt<int, 2, 4>::type *>(rowPtr + q);
+        if (p[1] - p[0] >= scout_row) s_scout[atomicAdd(s_n, 1)] = (uint16_t)k;
+    }
+    __syncthreads();
+}
+
 __device__ __forceinline__ bool is_long_row(int len, int block_nnz, int block_rows) {
     return len >= kLongRow && (int64_t)len * block_rows >= 2 * (int64_t)block_nnz;
 }
@@ -356,7 +391,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
                                                            const float *__restrict__ values,
                                                            const float *__restrict__ B,
                                                            float *__restrict__ C, int slab_w,
-                                                           int scouts) {
+                                                           int scouts, int scout_row) {
     constexpr int RPB = kBlock / L;
     constexpr int NW = kBlock / kWave;
     using Long = LongRow<VW, L, (L >= 32 ? 4 : L >= 16 ? 2 : 1)>;
@@ -369,20 +404,17 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
     int *s_col = reinterpret_cast<int *>(s_mem);
     float *s_val = s_mem + kWin;
     __shared__ int s_long[RPB];                // rows that the block sums together
-    __shared__ uint16_t s_scout[kScoutRows];
+    __shared__ uint16_t s_scout[kScoutList];
     __shared__ int s_nlong;
     __shared__ int s_tab[SLICED ? 2 * RPB + NW : 1];   // slice start, count per rank; per-wave counts
     if ((int)blockIdx.x < scouts) {            // the longest rows first
         const int parts = (min(slab_w, nv - (int)blockIdx.y * slab_w) + SW - 1) / SW;
-        const int q0 = (int)blockIdx.x / parts * kScoutRows, q1 = min(q0 + kScoutRows, nr);
-        if (threadIdx.x == 0) s_nlong = 0;
-        __syncthreads();
-        for (int q = q0 + (int)threadIdx.x; q < q1; q += kBlock)
-            if (rowPtr[q + 1] - rowPtr[q] >= kScoutRow) s_scout[atomicAdd(&s_nlong, 1)] = (uint16_t)(q - q0);
-        __syncthreads();
+        const int me = (int)blockIdx.x / parts, all = scouts / parts;
+        if (me >= all) return;
+        scout_look(me, all, nr, rowPtr, scout_row, s_scout, &s_nlong);
         const int cb = blockIdx.y * slab_w + (int)blockIdx.x % parts * SW;
         for (int i = 0; i < s_nlong; i++) {
-            const int q = q0 + s_scout[i];
+            const int q = (int)scout_at(me, all, nr, s_scout[i]);
             const float sum = Scout::sum(rowPtr[q], rowPtr[q + 1], colIdx, values, B, ldb, cb,
                                          nv, s_mem);
             if ((int)threadIdx.x < SW && cb + (int)threadIdx.x < nv)
@@ -404,7 +436,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
     for (int k = 0; k < VW; k++) acc[k] = 0.f;
     // Rows that this block's groups sum together, or the scouts do.
     auto apart = [&](int len) {
-        return is_long_row(len, be - bs, rlast - r0) || len >= kScoutRow;
+        return is_long_row(len, be - bs, rlast - r0) || len >= scout_row;
     };
     int nlong = 0;
     if (be - bs >= kLongRow) {                 // the same in every thread
@@ -415,7 +447,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
         nlong = s_nlong;
         for (int i = 0; i < nlong; i++) {
             const int q = s_long[i], p0 = rowPtr[q], p1 = rowPtr[q + 1];
-            if (p1 - p0 >= kScoutRow) continue;
+            if (p1 - p0 >= scout_row) continue;
             const float sum = Long::sum(p0, p1, colIdx, values, B, ldb, blockIdx.y * slab_w, nv, s_mem);
             const int c = blockIdx.y * slab_w + (int)threadIdx.x;
             if ((int)threadIdx.x < L * VW && c < nv)
@@ -509,9 +541,9 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
 // Overwrites.  Rows that a team would work on long after the others (a gather's
 // latency per nonzero and group is what bounds them):
 //   * beyond kTeamSteps nonzeros per group the team's whole wavefront sums the row;
-//   * rows of `scout_row` or more nonzeros (kVecScoutRow, and 8 times the mean)
-//     are found and summed by the first `scouts` blocks of the launch, kScoutCols
-//     columns and kScoutRows rows each.
+//   * rows of `scout_row` or more nonzeros (kVecScoutRow, and kScoutMean times the
+//     mean) are found and summed by the first `scouts` blocks of the launch,
+//     kScoutCols columns and up to kScoutRows rows each.
 // Power law (262144 rows, the longest 4900): nv = 1 165 -> 28 us, nv = 8 288 -> 61,
 // nv = 64 600 -> 153; 2567 rows, the longest 346, nv = 8: 16 -> 5.6.  The common path's
 // code is contiguous, the rare ones out of its way: the other order, or a real call
@@ -562,27 +594,23 @@ __device__ __forceinline__ void strided_accumulate(float (&acc)[VW], int p0, int
     }
 }
 
-// A scout block's share: the rows of scout_row or more nonzeros among its
-// kScoutRows, SW columns from `base` on.
+// A scout block's share: the rows of scout_row or more nonzeros among its own
+// (scout `me` of `all`), SW columns from `base` on.
 template <int VW, int SW>
-__device__ __forceinline__ void scout_rows(int q0, int q1, int base, int nv, int64_t ldb, int64_t ldc,
+__device__ __forceinline__ void scout_rows(int me, int all, int nr, int base, int nv, int64_t ldb, int64_t ldc,
                                         const int *__restrict__ rowPtr, const int *__restrict__ colIdx,
                                         const float *__restrict__ values, const float *__restrict__ B,
                                         float *__restrict__ C, int scout_row) {
     constexpr int SL = SW / VW;                // lanes of a group
     constexpr int NW = kBlock / kWave;
-    __shared__ uint16_t s_scout[kScoutRows];
+    __shared__ uint16_t s_scout[kScoutList];
     __shared__ int s_n;
     __shared__ float s_part[NW][SW];
     const int t = threadIdx.x, ln = lane_id();
-    if (t == 0) s_n = 0;
-    __syncthreads();
-    for (int q = q0 + t; q < q1; q += kBlock)
-        if (rowPtr[q + 1] - rowPtr[q] >= scout_row) s_scout[atomicAdd(&s_n, 1)] = (uint16_t)(q - q0);
-    __syncthreads();
+    scout_look(me, all, nr, rowPtr, scout_row, s_scout, &s_n);
     const int col0 = slab_col<VW>(base + (t % SL) * VW, nv);
     for (int i = 0; i < s_n; i++) {
-        const int q = q0 + s_scout[i];
+        const int q = (int)scout_at(me, all, nr, s_scout[i]);
         float acc[VW];
 #pragma unroll
         for (int k = 0; k < VW; k++) acc[k] = 0.f;
@@ -622,9 +650,10 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
     if (__builtin_expect((int)blockIdx.x < scouts, 0)) {
         constexpr int SW = L * VW < kScoutCols ? L * VW : kScoutCols;
         const int parts = (min(slab_w, nv - (int)blockIdx.y * slab_w) + SW - 1) / SW;
-        const int q0 = (int)blockIdx.x / parts * kScoutRows;
-        scout_rows<VW, SW>(q0, min(q0 + kScoutRows, nr), blockIdx.y * slab_w + (int)blockIdx.x % parts * SW,
-                           nv, ldb, ldc, rowPtr, colIdx, values, B, C, scout_row);
+        const int me = (int)blockIdx.x / parts, all = scouts / parts;
+        if (me < all)
+            scout_rows<VW, SW>(me, all, nr, blockIdx.y * slab_w + (int)blockIdx.x % parts * SW, nv, ldb,
+                               ldc, rowPtr, colIdx, values, B, C, scout_row);
         return;
     }
     const int b = xcd_remap(blockIdx.x - scouts, gridDim.x - scouts);
@@ -1150,6 +1179,28 @@ void with_vw(int vw, F &&f) {
     }
 }
 
+// Scouts beside `blocks` other blocks, for rows of at least `least` nonzeros:
+// enough that each looks at no more than kScoutRows rows, and where the others
+// leave the GPU room, more of them, up to kScoutBlocks, since all nonzeros may lie
+// in a few hundred rows; a whole number per XCD, which leaves xcd_remap its
+// meaning.  4096 rows, 512 neighbours of 2000 nonzeros, the others of 4, nv = 32,
+// csr_scalar: 8 scouts 11400 us, 31 369, 62 176, 249 67.  Beside many blocks they cost: 30000
+// rows of 128, nv = 1, csr_vector: 59 scouts 7.5 us, 234 8.6.
+// `all`: scouts take every row of `least` nonzeros, however long the others are.
+constexpr int kScoutBlocks = 256;
+constexpr int kScoutWork = 4096;
+
+Scouts scouts_for(int nr, int nnz, int nv, int slab_w, int least, int64_t blocks, bool all) {
+    Scouts s;
+    const int parts = div_up(std::min(nv, slab_w), std::min(slab_w, kScoutCols));
+    const int room = blocks < kScoutBlocks ? kScoutBlocks : blocks <= 4 * kScoutBlocks ? kScoutBlocks / 2 : 0;
+    const int rows = std::max(div_up(nr, kScoutRows), std::min({nr, nnz / kScoutWork, room}));
+    s.blocks = div_up((int64_t)rows * parts, kNumXcd) * kNumXcd;
+    s.row = all ? least
+                : (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(least, kScoutMean * (int64_t)nnz / std::max(1, nr)));
+    return s;
+}
+
 // Rows per wavefront of k_csr_stream: most of a window of pairs, at most one
 // row per lane and column.  Fewer pairs leave gathers unused (64^3 stencil,
 // nv = 4: half a window 26.6 us, 3/4 18.6, one 16.1), more make a long row's
@@ -1191,17 +1242,18 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
             if constexpr (VW_ * L_ >= 8) {
-                // scouts: one per kScoutRows rows and kScoutCols columns; a whole
-                // number per XCD, which leaves xcd_remap its meaning
-                const int parts = div_up(std::min(nv, s.width), std::min(s.width, kScoutCols));
-                const int scouts = div_up((int64_t)div_up(nr, kScoutRows) * parts, kNumXcd) * kNumXcd;
-                dim3 grid(scouts + div_up(nr, kBlock / L_), s.count);
+                const int blocks = div_up(nr, kBlock / L_);
+                const int64_t others = (int64_t)blocks * s.count;
+                const Scouts sc = scouts_for(nr, nnz, nv, s.width, kScoutRow, others, others < kScoutBlocks);
+                dim3 grid(sc.blocks + blocks, s.count);
                 if (sliced)
                     hipLaunchKernelGGL((k_csr_scalar_rm<VW_, L_, true>), grid, dim3(kBlock), 0, st, nr,
-                                       nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width, scouts);
+                                       nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width, sc.blocks,
+                                       sc.row);
                 else
                     hipLaunchKernelGGL((k_csr_scalar_rm<VW_, L_, false>), grid, dim3(kBlock), 0, st, nr,
-                                       nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width, scouts);
+                                       nv, ldb, ldc, rowPtr, colIdx, values, B, C, s.width, sc.blocks,
+                                       sc.row);
             }
         });
     });
@@ -1213,15 +1265,12 @@ void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t 
                           const int *colIdx, const float *values, const float *B, float *C,
                           hipStream_t st, const Slab &s) {
     if constexpr (GT * L <= kWave) {
-        // Scouts where a long row's wavefront would set the kernel's time; a whole
-        // number per XCD leaves xcd_remap its meaning.
-        int scouts = 0, scout_row = INT_MAX;
-        if ((int64_t)nnz * L >= kVecScoutWork) {
-            const int parts = div_up(std::min(nv, s.width), std::min(s.width, kScoutCols));
-            scouts = div_up((int64_t)div_up(nr, kScoutRows) * parts, kNumXcd) * kNumXcd;
-            scout_row = (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(kVecScoutRow, 8 * (int64_t)nnz / std::max(1, nr)));
-        }
-        dim3 grid(scouts + div_up(nr, kBlock / (GT * L)), s.count);
+        // Scouts where a long row's wavefront would set the kernel's time.
+        Scouts sc;
+        const int blocks = div_up(nr, kBlock / (GT * L));
+        if ((int64_t)nnz * L >= kVecScoutWork)
+            sc = scouts_for(nr, nnz, nv, s.width, kVecScoutRow, (int64_t)blocks * s.count, false);
+        dim3 grid(sc.blocks + blocks, s.count);
         // Four gathers in flight where a group has that many to make: with a B
         // that the L2s hold, only rows of more than 7 nonzeros per group gain (16384
         // rows of 32, nv = 64: 15.7 -> 13.4 us; 64^3 stencil, nv = 32: 98.7 -> 83.7;
@@ -1229,10 +1278,10 @@ void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t 
         const double per = (double)nnz / ((double)GT * std::max(1, nr));
         if (per > 7 || (per > 2.5 && (int64_t)nc * nv >= (4 << 20)))
             hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT, 4>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
-                               ldc, rowPtr, colIdx, values, B, C, s.width, scouts, scout_row);
+                               ldc, rowPtr, colIdx, values, B, C, s.width, sc.blocks, sc.row);
         else
             hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT, 1>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
-                               ldc, rowPtr, colIdx, values, B, C, s.width, scouts, scout_row);
+                               ldc, rowPtr, colIdx, values, B, C, s.width, sc.blocks, sc.row);
     }
 }
 
