@@ -555,8 +555,10 @@ constexpr int kVecScoutRow = 256;
 // wavefront takes the longest row that there can be in a few steps.
 constexpr int64_t kVecScoutWork = 1000000;
 
-// acc += the nonzeros p0, p0 + STRIDE, ... < e, in that order.
-template <int VW, int U>
+// acc += the nonzeros p0, p0 + stride, ... < e.  PARTS sums each U of them first,
+// which shortens the chains (256 nonzeros to four groups: error 9.5e-8 of the
+// result's norm, else 1.5e-7) and costs time (15000 rows of 100, nv = 64: 36.8 and 31.6 us).
+template <int VW, int U, bool PARTS = false>
 __device__ __forceinline__ void strided_accumulate(float (&acc)[VW], int p0, int e, int stride,
                                                    const int *__restrict__ colIdx,
                                                    const float *__restrict__ values,
@@ -584,11 +586,26 @@ __device__ __forceinline__ void strided_accumulate(float (&acc)[VW], int p0, int
         }
 #pragma unroll
         for (int u = 0; u < U; u++) load_g<float, VW>(b[u], Bc + (int64_t)c[u] * ldb);
+        if constexpr (PARTS) {
+            float part[VW];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (i + u * stride < n) {
+            for (int k = 0; k < VW; k++) part[k] = a[0] * b[0][k];
 #pragma unroll
-                for (int k = 0; k < VW; k++) acc[k] = __builtin_fmaf(a[u], b[u][k], acc[k]);
+            for (int u = 1; u < U; u++) {
+                if (i + u * stride < n) {
+#pragma unroll
+                    for (int k = 0; k < VW; k++) part[k] = __builtin_fmaf(a[u], b[u][k], part[k]);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < VW; k++) acc[k] += part[k];
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (i + u * stride < n) {
+#pragma unroll
+                    for (int k = 0; k < VW; k++) acc[k] = __builtin_fmaf(a[u], b[u][k], acc[k]);
+                }
             }
         }
     }
@@ -635,7 +652,7 @@ __device__ __forceinline__ void scout_rows(int me, int all, int nr, int base, in
     }
 }
 
-template <int VW, int L, int GT, int U>
+template <int VW, int L, int GT, int U, bool PARTS>
 __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_t ldb, int64_t ldc,
                                                            const int *__restrict__ rowPtr,
                                                            const int *__restrict__ colIdx,
@@ -670,7 +687,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
     const bool apart = e - s >= scout_row;
     const bool wide = T < kWave && !apart && e - s > kTeamSteps * GT;
     const bool mine = r < nr && !apart && !wide;
-    if (mine && colok) strided_accumulate<VW, U>(acc, s + g, e, GT, colIdx, values, Bc, ldb);
+    if (mine && colok) strided_accumulate<VW, U, PARTS>(acc, s + g, e, GT, colIdx, values, Bc, ldb);
 #pragma unroll
     for (int k = 0; k < VW; k++) acc[k] = butterfly_sum<L, T>(acc[k]);
     if (mine && colok && g == 0) store_g<true, VW>(C + (int64_t)r * ldc + col0, acc);
@@ -684,7 +701,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_rm(int nr, int nv, int64_
 #pragma unroll
                 for (int k = 0; k < VW; k++) acc[k] = 0.f;
                 if (colok)
-                    strided_accumulate<VW, 4>(acc, ps + ln / L, pe, kWave / L, colIdx, values, Bc, ldb);
+                    strided_accumulate<VW, 4, PARTS>(acc, ps + ln / L, pe, kWave / L, colIdx, values, Bc, ldb);
 #pragma unroll
                 for (int k = 0; k < VW; k++) acc[k] = butterfly_sum<L, kWave>(acc[k]);
                 if (ln < L && colok) store_g<true, VW>(C + (int64_t)q * ldc + col0, acc);
@@ -1263,7 +1280,7 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
 template <int VW, int L, int GT>
 void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                           const int *colIdx, const float *values, const float *B, float *C,
-                          hipStream_t st, const Slab &s) {
+                          hipStream_t st, const Slab &s, bool parts) {
     if constexpr (GT * L <= kWave) {
         // Scouts where a long row's wavefront would set the kernel's time.
         Scouts sc;
@@ -1276,29 +1293,39 @@ void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t 
         // rows of 32, nv = 64: 15.7 -> 13.4 us; 64^3 stencil, nv = 32: 98.7 -> 83.7;
         // 32^3 stencil, nv = 64, 6.3 per group: 15.0, with four 16.5).
         const double per = (double)nnz / ((double)GT * std::max(1, nr));
-        if (per > 7 || (per > 2.5 && (int64_t)nc * nv >= (4 << 20)))
-            hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT, 4>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
-                               ldc, rowPtr, colIdx, values, B, C, s.width, sc.blocks, sc.row);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, nr, nv, ldb, ldc, rowPtr, colIdx,
+                               values, B, C, s.width, sc.blocks, sc.row);
+        };
+        if (parts)
+            launch(k_csr_vector_rm<VW, L, GT, 4, true>);
+        else if (per > 7 || (per > 2.5 && (int64_t)nc * nv >= (4 << 20)))
+            launch(k_csr_vector_rm<VW, L, GT, 4, false>);
         else
-            hipLaunchKernelGGL((k_csr_vector_rm<VW, L, GT, 1>), grid, dim3(kBlock), 0, st, nr, nv, ldb,
-                               ldc, rowPtr, colIdx, values, B, C, s.width, sc.blocks, sc.row);
+            launch(k_csr_vector_rm<VW, L, GT, 1, false>);
     }
 }
 
 dspmm_status_t csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
-                             hipStream_t st, int hint) {
-    const Slab s = make_slab(nv, choose_vw_any(nv, 4));
+                             hipStream_t st, int hint, int min_groups = 0) {
+    Slab s = make_slab(nv, choose_vw_any(nv, 4));
+    if (min_groups > 0 && s.lanes > 64 / min_groups) {
+        s.lanes = 64 / min_groups;
+        s.width = s.lanes * s.vw;
+        s.count = div_up(nv, s.width);
+    }
     const double mean = nr ? (double)nnz / nr : 0.0;
     int gt = hint > 0 ? pow2_floor(hint) : lanes_for_mean(mean, 64);
     gt = std::max(1, std::min(gt, 64 / s.lanes));
+    const bool parts = min_groups > 0 && mean > 4.0 * gt;   // chains of more than four
     with_vw(s.vw, [&](auto vw_c) {
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
             with_lanes(gt, [&](auto gt_c) {
                 constexpr int GT_ = decltype(gt_c)::value;
                 launch_csr_vector_rm<VW_, L_, GT_>(nr, nc, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C,
-                                                   st, s);
+                                                   st, s, parts);
             });
         });
     });
@@ -1460,6 +1487,8 @@ dspmm_status_t flip(bool to_rows, bool add, const float *src, int64_t lds, int n
 
 }  // namespace
 
+constexpr int kFlipChain = 16;
+
 // Column-major operands on row-major copies of B and C in `scratch`, `cols`
 // columns at a time, with the row-major kernel of the same algorithm.
 size_t compat_flipped_bytes(int nr, int nc, int nv) {
@@ -1472,6 +1501,14 @@ dspmm_status_t launch_compat_flipped(int which, int nr, int nc, int nnz, int nv,
                                      hipStream_t st) {
     const bool coo = which == K_SPMM_COO_SCALAR_COL || which == K_SPMM_COO_VECTOR_COL;
     dspmm_status_t s = DSPMM_STATUS_SUCCESS;
+    // k_csr_vector_cm gives a row up to 64 lanes; the few groups that many columns
+    // leave would add longer chains, which round worse: at least one for each
+    // kFlipChain nonzeros of the mean row.  Error of the result's norm, in place / here
+    // / with as few groups as columns allow: 2048 rows of 256, nv = 128 7.8e-8 / 7.9e-8
+    // / 2.0e-7 (40 / 25 / 32 us); 7500 of 200, nv = 64 7.6e-8 / 7.8e-8 / 1.3e-7 (335 / 59
+    // / 37); 15000 of 100, nv = 64 7.3e-8 / 7.3e-8 / 9.9e-8 (354 / 44 / 42).
+    int groups = 1;
+    while (groups < 64 && (int64_t)groups * kFlipChain * nr < nnz) groups *= 2;
     for (int j = 0; j < nv && s == DSPMM_STATUS_SUCCESS; j += cols) {
         const int w = std::min(cols, nv - j);
         float *Bt = scratch, *Ct = scratch + align_words((int64_t)nc * w);
@@ -1482,7 +1519,7 @@ dspmm_status_t launch_compat_flipped(int which, int nr, int nc, int nnz, int nv,
         if (coo) s = coo_rm(nr, nnz, w, w, w, rowIdx, colIdx, values, Bt, Ct, st);
         else if (which == K_SPMM_CSR_SCALAR_COL)
             s = csr_scalar_rm(nr, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st);
-        else s = csr_vector_rm(nr, nc, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st, 0);
+        else s = csr_vector_rm(nr, nc, nnz, w, w, w, rowPtr, colIdx, values, Bt, Ct, st, 0, groups);
         if (s == DSPMM_STATUS_SUCCESS) s = flip(false, coo, Ct, w, nr, w, C + (int64_t)j * nr, nr, st);
     }
     return s;

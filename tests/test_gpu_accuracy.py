@@ -1,0 +1,85 @@
+"""Rounding error of whole results against 64 bits, no larger than that of the
+summation order that a path replaced: the order is computed here in FP32 on
+the CPU, and a path may be 5% above it (the spread of such a measure over the
+few hundred thousand outputs used).  Rows are of one length, so that one order
+describes them all.
+"""
+import numpy as np
+import pytest
+
+import dspmm as D
+from gpu_common import note
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+MARGIN = 1.05
+
+
+def fma(a, b, c):
+    return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(F)
+
+
+def chain(a, b):
+    """One FMA after the other along the last axis."""
+    s = np.zeros(np.broadcast_shapes(a.shape, b.shape)[:-1], F)
+    for i in range(a.shape[-1]):
+        s = fma(a[..., i], b[..., i], s)
+    return s
+
+
+def pairwise(parts):
+    while len(parts) > 1:
+        h = len(parts) // 2
+        parts = [parts[i] + parts[i + h] for i in range(h)]
+    return parts[0]
+
+
+def over_lanes(a, b, lanes):
+    """Lane l sums nonzeros l, l + lanes, ...; then a tree over the lanes."""
+    n = a.shape[-1]
+    return pairwise([chain(a[..., l:n:lanes], b[..., l:n:lanes]) if l < n else
+                     np.zeros(b.shape[:-1], F) for l in range(lanes)])
+
+
+def error(got, exact):
+    return float(np.sqrt(((got - exact) ** 2).mean() / (exact ** 2).mean()))
+
+
+class Rows:
+    """nr rows of n nonzeros over nc columns; B of maxnv columns, row-major."""
+
+    def __init__(self, nr, n, nc, maxnv, seed=3):
+        rng = np.random.default_rng(seed)
+        self.nr, self.n, self.nc = nr, n, nc
+        self.col = np.sort(np.argsort(rng.random((nr, nc), F), axis=1)[:, :n], axis=1).astype(np.int32)
+        self.val = rng.standard_normal((nr, n)).astype(F)
+        self.B = rng.uniform(-1, 1, (nc, maxnv)).astype(F)
+        self.ptr = (np.arange(nr + 1) * n).astype(np.int32)
+
+    def operands(self, nv, cols):
+        """Values and gathered B of the first `cols` columns, nonzeros last."""
+        b = self.B[:, :cols][self.col]                     # nr, n, cols
+        return self.val[:, None, :], np.ascontiguousarray(b.transpose(0, 2, 1))
+
+    def exact(self, a, b):
+        return (a.astype(np.float64) * b).sum(-1)
+
+
+@pytest.mark.parametrize("n,nv", [(40, 64), (100, 64), (256, 128)])
+def test_column_major_vector(n, nv):
+    """spmm_csr_vector_col adds each row over up to 64 lanes, also where it
+    runs on row-major copies."""
+    cols = 16
+    m = Rows(4000 if n < 200 else 2000, n, 3000, nv)
+    a, b = m.operands(nv, cols)
+    exact = m.exact(a, b)
+    d = [D.DeviceArray.from_numpy(x) for x in (m.ptr, np.repeat(np.arange(m.nr, dtype=np.int32), n),
+                                               m.col, m.val, np.ascontiguousarray(m.B[:, :nv].T))]
+    out = D.DeviceArray.from_numpy(np.full((nv, m.nr), np.nan, F))
+    st = D.launch("spmm_csr_vector_col", m.nr, m.nc, m.nr * n, nv, *d, out)
+    assert st == 0, D.status_string(st)
+    D.synchronize()
+    got = error(out.numpy().T[:, :cols], exact)
+    ref = error(over_lanes(a, b, 64 if n > 64 else 32), exact)
+    note(f"rows of {n}, nv={nv}: {got:.3g}, over the lanes {ref:.3g}")
+    assert got <= MARGIN * ref
