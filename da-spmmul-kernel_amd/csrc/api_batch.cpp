@@ -32,20 +32,73 @@ constexpr int kBatchTile = 128;
 constexpr double kBatchL2 = 4e6;
 constexpr int kBatchSlab = 64;
 
+// A row longer than a tile costs its carries and a wavefront of the combine, 0.7 ns
+// with a busy GPU.  So an item whose short tiles would split a row per
+// kBatchSplit bytes of its traffic or less takes tiles of 16 nonzeros per lane,
+// as single launches do, just long enough to leave those rows whole: narrow
+// items, whose tiles are the shortest.  Batches of widths 1 to 8, 64 items of 256
+// to 16384 rows, us, such rows split / whole: FP32 282 / 273, 173 / 159, BF16 245 /
+// 237; 65536 rows of 16, nv = 1, alone 59 / 13.  With a limit of 4096 bytes items of 16 columns
+// take them too, and the LDS they ask for costs a batch of mixed widths more than
+// their splits did (128 items 1059 -> 1492).
+// A whole batch takes them where it has little else to do: a row split per
+// kBatchSplitAll bytes of all its traffic.  us, split / whole: one per 3 KB (37500 rows
+// of 40, nv = 16, alone) 29 / 16.5; per 12.4 KB (16666 of 90, nv = 32, alone) 39 / 30, but
+// 96 mixed items of 16 columns 142 / 165; per 60 KB (128 items of mixed widths) 1059 / 1462.
+constexpr double kBatchSplit = 2048;
+constexpr double kBatchSplitAll = 10000;
+
+// Bytes that an item moves, roughly.
+static double item_cost(const dspmm_matrix_s *A, int nv, bool bf16) {
+    return (double)A->nnz * (8.0 + (double)nv * (bf16 ? 2 : 4)) + (double)A->nr * nv * 4.0;
+}
+
+// An item's configuration with vectors of `vec` values (0: the widest).
+static dspmm_config item_config(const dspmm_matrix_s *A, int nv, bool bf16, int vec) {
+    dspmm_config c{};
+    c.variant = DSPMM_VARIANT_NNZ_TILED;
+    c.vec = vec;
+    complete_nb(c, nv, bf16);
+    if (!bf16 && (double)A->nc * nv * sizeof(float) > kBatchL2 && c.vec * c.lanes > kBatchSlab)
+        c.lanes = kBatchSlab / c.vec;
+    return c;
+}
+
+// An item with short tiles and with such that leave more rows whole (the short
+// ones again if there are none), and how many rows those are.  Longer tiles may
+// need more lanes, so vectors as narrow as those that divide nv.
+struct ItemTiles {
+    dspmm_config brief, whole;
+    int kept = 0;
+};
+static ItemTiles item_tiles(const dspmm_matrix_s *A, int nv, bool bf16) {
+    ItemTiles t;
+    t.brief = t.whole = item_config(A, nv, bf16, 0);
+    t.brief.tile_nnz = std::max(8, std::min(kBatchTile, (bf16 ? kBatchPairsBf16 : kBatchPairs) * t.brief.lanes / kWave));
+    const int least = choose_vw(nv, nv, nv, nullptr, nullptr, bf16 ? 2 : 4, bf16 ? 8 : 4);
+    while (default_tile(t.whole.lanes) < A->max_len && t.whole.vec > least)
+        t.whole = item_config(A, nv, bf16, t.whole.vec / 2);
+    t.whole.tile_nnz = std::min(default_tile(t.whole.lanes), (A->max_len + 7) / 8 * 8);
+    if (t.whole.tile_nnz > t.brief.tile_nnz)
+        for (int r = 0; r < A->nr; r++) {
+            const int len = A->h_rowPtr[(size_t)r + 1] - A->h_rowPtr[(size_t)r];
+            t.kept += len > t.brief.tile_nnz && len <= t.whole.tile_nnz;
+        }
+    if (t.kept == 0) t.whole = t.brief;
+    return t;
+}
+
 dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc, const void *B,
-                             const void *C, dspmm_dtype_t btype, ItemFragment &f) {
+                             const void *C, dspmm_dtype_t btype, ItemFragment &f, bool whole) {
     const bool bf16 = btype == DSPMM_R_16BF;
     f = ItemFragment{};
     if (!A || nv < 1 || ldb < nv || ldc < nv) return DSPMM_STATUS_INVALID_VALUE;
     std::lock_guard<std::mutex> lk(A->mu);
     // Not the configurations tuned on single launches, where one matrix has the
     // whole GPU and its caches: they make the batch slower.
-    dspmm_config c{};
-    c.variant = DSPMM_VARIANT_NNZ_TILED;
-    complete_nb(c, nv, bf16);
-    if (!bf16 && (double)A->nc * nv * sizeof(float) > kBatchL2 && c.vec * c.lanes > kBatchSlab)
-        c.lanes = kBatchSlab / c.vec;
-    c.tile_nnz = std::max(8, std::min(kBatchTile, (bf16 ? kBatchPairsBf16 : kBatchPairs) * c.lanes / kWave));
+    const ItemTiles t = item_tiles(A, nv, bf16);
+    const double cost = item_cost(A, nv, bf16);
+    const dspmm_config c = whole || t.kept * kBatchSplit > cost ? t.whole : t.brief;
     if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) return DSPMM_STATUS_NOT_SUPPORTED;
     NbPlan *plan = nullptr;
     dspmm_status_t st = get_plan(A, c.tile_nnz, &plan);
@@ -67,7 +120,7 @@ dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc
     d.nsplits = plan->nsplits;
     const int G = kWave / c.lanes;
     f.units = d.nslabs * div_up(plan->ntiles, G);
-    f.cost = (double)A->nnz * (8.0 + (double)nv * (bf16 ? 2 : 4)) + (double)A->nr * nv * 4.0;
+    f.cost = cost;
     f.lds_ints = (int)(nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) / (kBlock / kWave) / 4);
     f.nslots = plan->nslots;
     f.nsplits = plan->nsplits;
@@ -75,13 +128,23 @@ dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc
 }
 
 dspmm_status_t build_schedule(const dspmm_batch_item *items, int count, dspmm_dtype_t btype,
-                              BatchSchedule &s) {
+                              BatchSchedule &s, bool together) {
     std::vector<ItemFragment> frags((size_t)count);
     std::vector<const ItemFragment *> fp((size_t)count);
+    const bool bf16 = btype == DSPMM_R_16BF;
+    double cost = 0, kept = 0;
     for (int i = 0; i < count; i++) {
         const dspmm_batch_item &it = items[i];
-        if (!it.A || (it.A->nr > 0 && !it.C) || (it.A->nnz > 0 && !it.B)) return DSPMM_STATUS_INVALID_VALUE;
-        dspmm_status_t st = schedule_item(it.A, it.nv, it.ldb, it.ldc, it.B, it.C, btype, frags[(size_t)i]);
+        if (!it.A || it.nv < 1 || (it.A->nr > 0 && !it.C) || (it.A->nnz > 0 && !it.B))
+            return DSPMM_STATUS_INVALID_VALUE;
+        cost += item_cost(it.A, it.nv, bf16);
+        kept += item_tiles(it.A, it.nv, bf16).kept;
+    }
+    const bool whole = together && kept * kBatchSplitAll > cost;
+    for (int i = 0; i < count; i++) {
+        const dspmm_batch_item &it = items[i];
+        dspmm_status_t st = schedule_item(it.A, it.nv, it.ldb, it.ldc, it.B, it.C, btype,
+                                          frags[(size_t)i], whole);
         if (st != DSPMM_STATUS_SUCCESS) return st;
         fp[(size_t)i] = &frags[(size_t)i];
     }
@@ -201,7 +264,7 @@ dspmm_status_t dspmm_batch_create(dspmm_batch_t *out, const dspmm_batch_item *it
     b->count = count;
     b->btype = btype;
     b->items.assign(items, items + count);
-    dspmm_status_t st = build_schedule(items, count, btype, b->sch);
+    dspmm_status_t st = build_schedule(items, count, btype, b->sch, true);
     if (st != DSPMM_STATUS_SUCCESS) {
         free_batch(b);
         return st;

@@ -37,17 +37,21 @@ struct ItemFragment {
     int nslots = 0, nsplits = 0;
 };
 
-// The fragment of matrix A with nv columns (locks A while reading it).
+// The fragment of matrix A with nv columns (locks A while reading it).  `whole`:
+// with tiles that leave more rows whole, where there are such.
 dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc, const void *B,
-                             const void *C, dspmm_dtype_t btype, ItemFragment &f);
+                             const void *C, dspmm_dtype_t btype, ItemFragment &f,
+                             bool whole = false);
 // A schedule from one fragment per item (frags[i] for items[i], whose
 // operands and strides are bound here): carry offsets, split prefix sums and
 // the per-XCD segments.
 dspmm_status_t assemble_schedule(const ItemFragment *const *frags, const dspmm_batch_item *items,
                                  int count, BatchSchedule &s);
-// schedule_item for every item, then assemble_schedule.
+// schedule_item for every item, then assemble_schedule.  `together`: the items'
+// tiles are chosen for the batch as a whole; without, an item's tiles, and so the
+// bits of its result, do not depend on its company.
 dspmm_status_t build_schedule(const dspmm_batch_item *items, int count, dspmm_dtype_t btype,
-                              BatchSchedule &s);
+                              BatchSchedule &s, bool together);
 // Workgroups of the launch: blocks_per_cu > 0 -> persistent grid.
 int schedule_blocks(const BatchSchedule &s, int blocks_per_cu);
 

@@ -174,6 +174,7 @@ void ring_bind_plan(dspmm_matrix_s *A, const RingPlan &plan, RingLaunch &a);
 int ring_auto_z(dspmm_matrix_s *A, int w, int h);
 int cached_smax(int umax);
 int64_t carry_ld(int nv);
+int default_tile(int lanes);
 void complete_nb(dspmm_config &c, int nv, bool bf16);
 // The configuration a call runs: cfg unless AUTO, else the tuned one cached
 // for (layout, nv, bt), else (with `learned`, row-major only) the

@@ -337,7 +337,7 @@ struct dspmm_server_s {
             if (st == DSPMM_STATUS_SUCCESS && own.empty())
                 st = assemble_schedule(fp.data(), items.data(), (int)items.size(), sch);
         } else {
-            st = build_schedule(items.data(), (int)items.size(), cfg.btype, sch);
+            st = build_schedule(items.data(), (int)items.size(), cfg.btype, sch, false);
         }
         if (st == DSPMM_STATUS_SUCCESS) {
             for (size_t i = 0; i < jobs.size() && i < sch.items.size(); i++) sch.items[i].carry = jobs[i].carry;
