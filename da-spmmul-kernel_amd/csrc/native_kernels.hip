@@ -365,11 +365,12 @@ __global__ __launch_bounds__(kBlock) void k_split_combine_batched(const ItemDesc
 // and writes the products to LDS.  After one barrier, thread i sums row
 // r0+i from LDS in nonzero order if the row has at most kSpmvThreadRow
 // nonzeros -- bit-exact with the host loop; longer rows of the tile are
-// queued in LDS and taken by kSpmvRowLanes lanes each: lane l sums products l,
-// l + kSpmvRowLanes, ... in order, then a fixed butterfly.  (A wavefront per row
+// queued in LDS and taken by kSpmvRowLanes lanes each, with four sums to a lane, so that
+// chains are no longer than a wavefront's: 64 sums of products l, l + 64, ... in order,
+// then a fixed tree.  (A wavefront per row
 // made rows of 17 to 100 the kernel's time: 143583 rows of 23 19.8 us, 16 lanes
 // 15.4, 8 14.8; 39950 of 22 8.8, 6.9, 6.7; power law with rows of up to 500 5.1, 5.1,
-// 5.8.)  A tile of one longer row (up to
+// 5.8.  One sum to a lane: 200 nonzeros 9.1e-8 of the result's norm, four 7.9e-8.)  A tile of one longer row (up to
 // kSpmvLongTiles * T nonzeros) or of one T-chunk of a still longer row is
 // reduced by the workgroup: thread t sums products t, t+256, t+512, ... in
 // that order, then a pairwise tree; the result goes to y (whole row) or to
@@ -428,12 +429,19 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
         }
         __syncthreads();
         constexpr int LR = kSpmvRowLanes;
+        static_assert(kWave / LR == 4, "four sums to a lane");
         for (int k = t / LR; k < nlong; k += kBlock / LR) {
             const int4 q = lrange[k];
-            float s = 0.f;
-            for (int p = q.x + t % LR; p < q.y; p += LR) s = s + prod[p];
-            s = group_sum<LR>(s);
-            if (t % LR == 0) d.C[(int64_t)q.z * d.ldc] = s;
+            float s[kWave / LR];
+#pragma unroll
+            for (int j = 0; j < kWave / LR; j++) s[j] = 0.f;
+            for (int p = q.x + t % LR; p < q.y; p += kWave) {
+#pragma unroll
+                for (int j = 0; j < kWave / LR; j++)
+                    if (p + j * LR < q.y) s[j] = s[j] + prod[p + j * LR];
+            }
+            const float sum = group_sum<LR>((s[0] + s[1]) + (s[2] + s[3]));
+            if (t % LR == 0) d.C[(int64_t)q.z * d.ldc] = sum;
         }
         return;
     }

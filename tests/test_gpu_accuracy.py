@@ -83,3 +83,27 @@ def test_column_major_vector(n, nv):
     ref = error(over_lanes(a, b, 64 if n > 64 else 32), exact)
     note(f"rows of {n}, nv={nv}: {got:.3g}, over the lanes {ref:.3g}")
     assert got <= MARGIN * ref
+
+
+@pytest.mark.parametrize("n", [20, 64, 100, 200, 256])
+def test_spmv_tiles(n):
+    """Rows of 17 to 256 nonzeros of an SpMV tile: products over 64 lanes, then
+    a tree."""
+    m = Rows(3000, n, 2500, 1)
+    a, b = m.operands(1, 1)
+    exact = m.exact(a, b)[:, 0]
+    h = D.Matrix(m.nr, m.nc, m.ptr, m.col.reshape(-1), m.val.reshape(-1))
+    d_x, d_y = D.DeviceArray.from_numpy(m.B[:, 0].copy()), D.DeviceArray.zeros(m.nr)
+    h.spmm(d_x, d_y, 1, config=D.make_config(D.VARIANT_SPMV_TILED, tile_nnz=1024))
+    D.synchronize()
+    prod = (a * b)[:, 0, :]
+    lanes = []
+    for lane in range(64):
+        s = np.zeros(m.nr, F)
+        for i in range(lane, n, 64):
+            s = s + prod[:, i]
+        lanes.append(s)
+    got, ref = error(d_y.numpy(), exact), error(pairwise(lanes), exact)
+    note(f"rows of {n}: {got:.3g}, 64 lanes {ref:.3g}")
+    assert got <= MARGIN * ref
+    h.close()
