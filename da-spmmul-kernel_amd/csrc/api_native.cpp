@@ -940,9 +940,10 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         if (nv != 1) return DSPMM_STATUS_NOT_SUPPORTED;
         const int T = cfg.tile_nnz > 0 ? cfg.tile_nnz : kSpmvTile;
         if (!spmv_tile_ok(T)) return DSPMM_STATUS_NOT_SUPPORTED;
-        // On few diagonals the slices replace the tiles at every size: 100^3
-        // 27-point stencil 32 us against 92 (5 bytes a nonzero instead of 8,
-        // 4.5 TB/s), 64^3 8.9 against 30, 32^3 4.8 against 8.4.
+        // On few diagonals the slices replace the tiles, at every number of rows:
+        // 100^3 27-point stencil 32 us against 92 (5 bytes a nonzero instead of 8,
+        // 4.5 TB/s), 64^3 8.9 against 30, 32^3 4.8 against 8.4; 2048 rows of 27 4.7
+        // against 5.2.
         DiagPlan *dp = nullptr;
         dspmm_status_t s = get_diag_plan(A, &dp, build);
         if (s != DSPMM_STATUS_SUCCESS) return s;

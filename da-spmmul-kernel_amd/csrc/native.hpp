@@ -149,6 +149,12 @@ struct SpmvDiagLaunch {
 };
 constexpr int kDiagRows = 64;      // a wavefront's lanes
 constexpr int kDiagMax = 256;
+// The longest row of a matrix in slices: a wavefront adds its 64 rows side by
+// side, each in four chains, so that long rows take long and round worse than the
+// tiles' 64 sums.  us, tiles / slices, and the error of the result's norm: 30000 rows
+// of 40 4.4 / 5.7, 6.8e-8 / 7.1e-8; of 64 4.3 / 7.6, 7.1e-8 / 8.5e-8; of 256 17.0 / 35.4,
+// 8.2e-8 / 1.5e-7; 512 rows of 256 4.3 / 23.4.  100000 rows of 64 lose 16.5 / 11.8.
+constexpr int kDiagRowMax = 32;
 constexpr double kDiagPad = 1.25;
 dspmm_status_t launch_spmv_diag(const SpmvDiagLaunch &a, hipStream_t st);
 // Fills vals and didx of the slices from the device CSR arrays.

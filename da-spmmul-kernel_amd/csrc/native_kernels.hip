@@ -483,8 +483,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_tiled(ItemDesc d, int ntiles) {
 // nonzero takes 5 bytes, read 16 + 4 per lane and group, and the lanes'
 // x are neighbours, since neighbouring rows share their diagonals.  Rows of at
 // most kSpmvThreadRow nonzeros are summed in order with a rounded multiply and
-// add -- the host loop's bits -- and longer ones in four interleaved FMA sums,
-// whose rounding is no worse than the 64-lane tree's.
+// add -- the host loop's bits -- and longer ones, of at most kDiagRowMax, in four
+// interleaved FMA sums.
 // What bounds it: reading the slices.
 template <typename TB, bool UNIT>
 __global__ __launch_bounds__(kBlock) void k_spmv_diag(SpmvDiagLaunch a) {

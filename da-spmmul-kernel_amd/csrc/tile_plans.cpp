@@ -202,8 +202,9 @@ bool build_row_blocks(const std::vector<int> &rp, const std::vector<int> &ci,
 }
 
 // The distinct column-minus-row distances, ascending, and the slices' offsets
-// (see SpmvDiagLaunch); false if there are more than kDiagMax, or if padding
-// the slices would store more than kDiagPad times the nonzeros.
+// (see SpmvDiagLaunch); false if there are more than kDiagMax, if a row is longer
+// than kDiagRowMax, or if padding the slices would store more than kDiagPad times
+// the nonzeros.
 bool build_diag_slices(const std::vector<int> &rp, const std::vector<int> &ci, int nr,
                        std::vector<int> &diags, std::vector<int> &off) {
     diags.clear();
@@ -215,6 +216,7 @@ bool build_diag_slices(const std::vector<int> &rp, const std::vector<int> &ci, i
         const int r1 = (int)std::min<int64_t>(nr, ((int64_t)s + 1) * kDiagRows);
         for (int r = s * kDiagRows; r < r1; r++)
             longest = std::max(longest, rp[(size_t)r + 1] - rp[(size_t)r]);
+        if (longest > kDiagRowMax) return false;
         groups += (longest + 3) / 4;
         if (groups * (4 * kDiagRows) > INT_MAX) return false;
         off[(size_t)s + 1] = (int)groups;

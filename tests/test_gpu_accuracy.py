@@ -107,3 +107,34 @@ def test_spmv_tiles(n):
     note(f"rows of {n}: {got:.3g}, 64 lanes {ref:.3g}")
     assert got <= MARGIN * ref
     h.close()
+
+
+@pytest.mark.parametrize("n", [27, 32, 33, 64, 256])
+def test_spmv_band(n):
+    """A banded matrix, which may run in slices of diagonals, rounds no worse
+    than the tiles' 64 sums, and takes no longer than a multiple of the tiles."""
+    rng = np.random.default_rng(n)
+    nr = 4000
+    nc = nr + 3 * n
+    col = (np.arange(nr)[:, None] + 3 * np.arange(n)).astype(np.int32)
+    val = rng.standard_normal((nr, n)).astype(F)
+    x = rng.uniform(-1, 1, nc).astype(F)
+    prod = val * x[col]
+    exact = (val.astype(np.float64) * x[col]).sum(1)
+    lanes = [chain(val[:, i::64], x[col][:, i::64]) if i < n else np.zeros(nr, F) for i in range(64)]
+    ptr = (np.arange(nr + 1) * n).astype(np.int32)
+    h = D.Matrix(nr, nc, ptr, col.reshape(-1), val.reshape(-1))
+    # the same rows on scattered columns: no diagonals
+    t = D.Matrix(nr, nc, ptr, np.sort(rng.permutation(nc)[:nc][col % nc], 1).reshape(-1), val.reshape(-1))
+    d_x, d_y = D.DeviceArray.from_numpy(x), D.DeviceArray.zeros(nr)
+    ms = {}
+    for name, mat in (("band", h), ("scattered", t)):
+        ms[name] = min(mat.benchmark(d_x, d_y, 1, warmup=5, reps=40, per_call=False)[0] for _ in range(3))
+    h.spmm(d_x, d_y, 1)
+    D.synchronize()
+    got, ref = error(d_y.numpy(), exact), error(pairwise(lanes), exact)
+    note(f"rows of {n}: {got:.3g}, 64 lanes {ref:.3g}; {ms}")
+    assert got <= 1.15 * ref                   # 4000 outputs spread by a few percent
+    assert ms["band"] <= 1.5 * ms["scattered"] + 0.002
+    h.close()
+    t.close()
