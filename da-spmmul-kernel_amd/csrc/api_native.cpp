@@ -319,11 +319,12 @@ dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build) {
                 s = launch_diag_fill(p.d_off, p.d_diags, nd, A->rowPtr, A->colIdx, A->values, A->nr,
                                      p.nslices, p.d_vals, p.d_didx, nullptr);
             if (s == DSPMM_STATUS_SUCCESS) s = hip_status(hipStreamSynchronize(nullptr));
-            if (s != DSPMM_STATUS_SUCCESS) {
+            p.usable = s == DSPMM_STATUS_SUCCESS;
+            if (!p.usable) {                       // the tiles need almost no memory: they run
+                (void)hipGetLastError();
                 free_diag_plan(p);
-                return s;
+                p.known = true;
             }
-            p.usable = true;
         }
         A->diag = p;
     }

@@ -161,7 +161,7 @@ dspmm_status_t get_ring_plan(dspmm_matrix_s *A, int w, int h, int zchunk, RingPl
                              bool build = true);
 // The matrix's diagonal-slice plan, looked for and built on first use
 // (build == false: DSPMM_STATUS_NOT_PREPARED if it was not); *out is NULL for
-// a matrix that has none.
+// a matrix that has none, or none that the device had memory for.
 dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build = true);
 // The plan's shape for tile w x h (one row distance: w * h consecutive rows
 // per tile, walked along that distance).  Reads the sampled row distances.

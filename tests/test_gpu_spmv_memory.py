@@ -1,0 +1,52 @@
+"""SpMV where the device has no memory left for a second copy of the matrix:
+the slices of diagonals are given up, the tiles run."""
+import numpy as np
+import pytest
+
+import dspmm as D
+import oracle as O
+import workloads as W
+from gpu_common import assert_fp32, note
+
+pytestmark = pytest.mark.gpu
+RM = D.DENSE_ROW_MAJOR
+LEFT = 48 << 20                      # bytes left free; the slices of the stencil need 120 MB
+
+
+def test_slices_without_memory():
+    a = W.c3_matrix(90)
+    m = D.Matrix(a.nr, a.nc, a.rowPtr, a.colIdx, a.values)
+    x = np.random.default_rng(1).uniform(-1, 1, a.nc).astype(np.float32)
+    d_x, d_y = D.DeviceArray.from_numpy(x), D.DeviceArray.from_numpy(np.full(a.nr, np.nan, np.float32))
+    small = W.c3_matrix(8)           # the kernels are loaded before the memory goes
+    s = D.Matrix(small.nr, small.nc, small.rowPtr, small.colIdx, small.values)
+    s.spmm(d_x, d_y, 1)
+    D.synchronize()
+    s.close()
+    d_y = D.DeviceArray.from_numpy(np.full(a.nr, np.nan, np.float32))
+    before = m.describe()["hbm_bytes"]
+    taken = []
+    try:
+        step = 64 << 30
+        while step >= 16 << 20:
+            free = D.device_info()["free_mem"]
+            if free < LEFT + step:
+                step //= 2
+                continue
+            try:
+                taken.append(D.DeviceArray(step, np.uint8, (step,)))
+            except RuntimeError:
+                step //= 2
+        note(f"free {D.device_info()['free_mem'] >> 20} MiB of {D.device_info()['total_mem'] >> 30} GiB")
+        for _ in range(2):
+            m.spmm(d_x, d_y, 1)
+            D.synchronize()
+    finally:
+        for t in taken:
+            t.free()
+    assert m.describe()["hbm_bytes"] - before < 32 << 20
+    h32 = O.spmm_host32(RM, a.nr, a.nc, 1, a.rowPtr, a.colIdx, a.values, x).reshape(-1)
+    c64, ab = O.spmm_fp64(RM, a.nr, a.nc, 1, a.rowPtr, a.colIdx, a.values, x)
+    assert_fp32(d_y.numpy(), c64.reshape(-1), ab.reshape(-1), np.diff(a.rowPtr).astype(np.float64),
+                "tiles", h32)
+    m.close()
