@@ -290,21 +290,33 @@ dspmm_status_t get_ring_plan(dspmm_matrix_s *A, int w, int h, int zchunk, RingPl
     return DSPMM_STATUS_SUCCESS;
 }
 
+bool diag_fits(dspmm_matrix_s *A) {
+    DiagPlan &p = A->diag;
+    if (!p.looked) {
+        p.looked = true;
+        p.fits = build_diag_slices(A->h_rowPtr, A->h_colIdx, A->nr, p.h_diags, p.h_off);
+        if (!p.fits) {
+            p.h_diags = std::vector<int>();
+            p.h_off = std::vector<int>();
+        }
+    }
+    return p.fits;
+}
+
 dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build) {
     *out = nullptr;
-    if (!A->diag.known) {
+    DiagPlan &p = A->diag;
+    if (!p.known) {
         if (!build) return DSPMM_STATUS_NOT_PREPARED;
-        std::vector<int> diags, off;
-        DiagPlan p;
         p.known = true;
-        if (build_diag_slices(A->h_rowPtr, A->h_colIdx, A->nr, diags, off)) {
-            p.nslices = (int)off.size() - 1;
-            const int nd = (int)diags.size();
-            diags.resize((size_t)kDiagMax, INT_MAX);
-            const size_t cells = (size_t)off.back() * kDiagRows;
+        if (diag_fits(A)) {
+            p.nslices = (int)p.h_off.size() - 1;
+            const int nd = (int)p.h_diags.size();
+            const size_t cells = (size_t)p.h_off.back() * kDiagRows;
             // values, diagonal bytes, diagonals and slice offsets, in this order
-            std::vector<int> head(diags);
-            head.insert(head.end(), off.begin(), off.end());
+            std::vector<int> head(p.h_diags);
+            head.resize((size_t)kDiagMax, INT_MAX);
+            head.insert(head.end(), p.h_off.begin(), p.h_off.end());
             p.bytes = (sizeof(float4) + sizeof(uint32_t)) * cells + sizeof(int) * head.size();
             dspmm_status_t s = hip_status(hipMalloc(&p.d_mem, p.bytes));
             if (s == DSPMM_STATUS_SUCCESS) {
@@ -322,13 +334,15 @@ dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build) {
             p.usable = s == DSPMM_STATUS_SUCCESS;
             if (!p.usable) {                       // the tiles need almost no memory: they run
                 (void)hipGetLastError();
-                free_diag_plan(p);
-                p.known = true;
+                (void)hipFree(p.d_mem);
+                p.d_mem = nullptr;
+                p.bytes = 0;
             }
+            p.h_diags = std::vector<int>();
+            p.h_off = std::vector<int>();
         }
-        A->diag = p;
     }
-    if (A->diag.usable) *out = &A->diag;
+    if (p.usable) *out = &p;
     return DSPMM_STATUS_SUCCESS;
 }
 
@@ -521,8 +535,7 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
     const bool rm = layout == DENSE_ROW_MAJOR;
     dspmm_config c{};
     if (nv == 1) {
-        c.variant = DSPMM_VARIANT_SPMV_TILED;
-        c.tile_nnz = kSpmvTile;
+        c.variant = DSPMM_VARIANT_SPMV_TILED;      // slices of diagonals, or tiles of kSpmvTile
         return c;
     }
     const int64_t work = (int64_t)A->nnz * nv;
@@ -941,12 +954,13 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         if (nv != 1) return DSPMM_STATUS_NOT_SUPPORTED;
         const int T = cfg.tile_nnz > 0 ? cfg.tile_nnz : kSpmvTile;
         if (!spmv_tile_ok(T)) return DSPMM_STATUS_NOT_SUPPORTED;
-        // On few diagonals the slices replace the tiles, at every number of rows:
-        // 100^3 27-point stencil 32 us against 92 (5 bytes a nonzero instead of 8,
+        // Without a tile size, on few diagonals, the slices replace the tiles, at
+        // every number of rows: 100^3 27-point stencil 32 us against 92 (5 bytes a nonzero instead of 8,
         // 4.5 TB/s), 64^3 8.9 against 30, 32^3 4.8 against 8.4; 2048 rows of 27 4.7
         // against 5.2.
         DiagPlan *dp = nullptr;
-        dspmm_status_t s = get_diag_plan(A, &dp, build);
+        dspmm_status_t s = DSPMM_STATUS_SUCCESS;
+        if (cfg.tile_nnz <= 0) s = get_diag_plan(A, &dp, build);
         if (s != DSPMM_STATUS_SUCCESS) return s;
         if (dp) {
             if (!launch) return s;
@@ -1092,6 +1106,8 @@ dspmm_config resolve(dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_
     if (it != A->prepared.end()) return it->second;
     dspmm_config c;
     if (learned && layout == DENSE_ROW_MAJOR && learned_select(A, nv, &c)) {
+        // a tile size picked for the tiles gives way to the slices of diagonals
+        if (c.variant == DSPMM_VARIANT_SPMV_TILED && diag_fits(A)) c.tile_nnz = 0;
         // the selector was measured with FP32 B; with BF16 B only its B-row
         // ring picks carry over (the ring takes either, with the vector width
         // left to the operands)
@@ -1124,7 +1140,8 @@ dspmm_status_t ex_workspace_bytes(dspmm_matrix_s *A, DenseLayout layout, int nv,
     }
     if (c.variant == DSPMM_VARIANT_SPMV_TILED && nv == 1) {
         DiagPlan *dp = nullptr;
-        dspmm_status_t st = get_diag_plan(A, &dp);
+        dspmm_status_t st = DSPMM_STATUS_SUCCESS;
+        if (c.tile_nnz <= 0) st = get_diag_plan(A, &dp);
         if (st != DSPMM_STATUS_SUCCESS || dp) return st;          // no split rows
         NbPlan *plan = nullptr;
         st = get_plan(A, c.tile_nnz > 0 ? c.tile_nnz : kSpmvTile, &plan, kPlanSpmv);
@@ -1639,7 +1656,13 @@ std::vector<dspmm_config> autotune_candidates(dspmm_matrix_s *A, DenseLayout lay
             }
     }
     if (nv == 1) {
-        for (int T : {512, 1024, 2048, 4096}) {
+        bool slices;
+        {
+            std::lock_guard<std::mutex> lk(A->mu);
+            slices = diag_fits(A);
+        }
+        for (int T : {0, 512, 1024, 2048, 4096}) {
+            if (T == 0 && !slices) continue;           // 0: the slices of diagonals
             dspmm_config c{};
             c.variant = DSPMM_VARIANT_SPMV_TILED;
             c.tile_nnz = T;

@@ -58,7 +58,11 @@ struct DiagPlan {
     uint32_t *d_didx = nullptr;
     int nslices = 0;
     size_t bytes = 0;
-    bool known = false;              // the matrix has been looked at
+    // The host's look at the matrix: whether it goes in slices, and until they are
+    // on the device their diagonals and offsets.
+    bool looked = false, fits = false;
+    std::vector<int> h_diags, h_off;
+    bool known = false;              // the slices are on the device, or there are none
     bool usable = false;
 };
 
@@ -159,6 +163,8 @@ int shared_row_stride2(dspmm_matrix_s *A);
 // on first use (build == false: DSPMM_STATUS_NOT_PREPARED if missing).
 dspmm_status_t get_ring_plan(dspmm_matrix_s *A, int w, int h, int zchunk, RingPlan **out,
                              bool build = true);
+// Whether the matrix goes in diagonal slices (computed once per matrix).
+bool diag_fits(dspmm_matrix_s *A);
 // The matrix's diagonal-slice plan, looked for and built on first use
 // (build == false: DSPMM_STATUS_NOT_PREPARED if it was not); *out is NULL for
 // a matrix that has none, or none that the device had memory for.

@@ -269,11 +269,13 @@ typedef enum dspmm_variant {
     DSPMM_VARIANT_COO_VECTOR = 5,
     DSPMM_VARIANT_SPMV_TILED = 6,/* nv == 1 only: workgroup per nnz tile, products
                                     in LDS, per-row sums (row-exact), tree for
-                                    long rows; tile_nnz = tile size.  A matrix
-                                    whose nonzeros lie on at most 256 diagonals
-                                    is stored as slices of 64 rows instead
-                                    (5 bytes a nonzero); rows of at most 16
-                                    nonzeros are summed like the host loop in
+                                    long rows; tile_nnz = tile size.  With
+                                    tile_nnz 0 a matrix whose nonzeros lie on at
+                                    most 256 diagonals, at most 32 in a row, is
+                                    stored as slices of 64 rows instead (a second
+                                    copy, 5 to 7 bytes a nonzero, where the
+                                    device has memory for it); rows of at most
+                                    16 nonzeros are summed like the host loop in
                                     both */
     DSPMM_VARIANT_NNZ_CACHED = 7,/* row-major, lanes * vec >= nv: tiles of whole
                                     rows whose distinct columns' B rows are

@@ -50,3 +50,37 @@ def test_slices_without_memory():
     assert_fp32(d_y.numpy(), c64.reshape(-1), ab.reshape(-1), np.diff(a.rowPtr).astype(np.float64),
                 "tiles", h32)
     m.close()
+
+
+def test_a_tile_size_asks_for_the_tiles():
+    """SPMV_TILED with a tile size runs the tiles also on few diagonals; without
+    one, and under AUTO, the slices; the autotuner times the slices once."""
+    a = W.c3_matrix(24)
+    x = np.random.default_rng(2).uniform(-1, 1, a.nc).astype(np.float32)
+    d_x, d_y = D.DeviceArray.from_numpy(x), D.DeviceArray.zeros(a.nr)
+    grown = {}
+    for name, cfg in (("tiles", D.make_config(D.VARIANT_SPMV_TILED, tile_nnz=1024)),
+                      ("default", D.make_config(D.VARIANT_SPMV_TILED)), ("auto", None)):
+        m = D.Matrix(a.nr, a.nc, a.rowPtr, a.colIdx, a.values)
+        before = m.describe()["hbm_bytes"]
+        m.spmm(d_x, d_y, 1, config=cfg)
+        D.synchronize()
+        grown[name] = (m.describe()["hbm_bytes"] - before) / a.nnz
+        if cfg is None:
+            table = m.autotune_table(d_x, d_y, 1, reps=1)
+            sizes = [c.tile_nnz for c, _ in table if c.variant == D.VARIANT_SPMV_TILED]
+            assert sorted(sizes) == [0, 512, 1024, 2048, 4096]
+        m.close()
+    note(str(grown))
+    assert grown["tiles"] < 1 and grown["default"] > 5 and grown["auto"] > 5
+
+
+def test_autotuner_without_diagonals():
+    rng = np.random.default_rng(3)
+    ci = np.sort(rng.integers(0, 3000, (2000, 8)), 1).astype(np.int32)
+    m = D.Matrix(2000, 3000, (np.arange(2001) * 8).astype(np.int32), ci.reshape(-1),
+                 rng.standard_normal(16000).astype(np.float32))
+    d_x, d_y = D.DeviceArray.from_numpy(rng.uniform(-1, 1, 3000).astype(np.float32)), D.DeviceArray.zeros(2000)
+    table = m.autotune_table(d_x, d_y, 1, reps=1)
+    assert sorted(c.tile_nnz for c, _ in table if c.variant == D.VARIANT_SPMV_TILED) == [512, 1024, 2048, 4096]
+    m.close()
