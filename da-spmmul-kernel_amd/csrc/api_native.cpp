@@ -303,6 +303,12 @@ bool diag_fits(dspmm_matrix_s *A) {
     return p.fits;
 }
 
+size_t diag_bytes(const dspmm_matrix_s *A) {
+    const std::vector<int> &off = A->diag.h_off;
+    return (sizeof(float4) + sizeof(uint32_t)) * (size_t)off.back() * kDiagRows +
+           sizeof(int) * ((size_t)kDiagMax + off.size());
+}
+
 dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build) {
     *out = nullptr;
     DiagPlan &p = A->diag;
@@ -317,7 +323,7 @@ dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build) {
             std::vector<int> head(p.h_diags);
             head.resize((size_t)kDiagMax, INT_MAX);
             head.insert(head.end(), p.h_off.begin(), p.h_off.end());
-            p.bytes = (sizeof(float4) + sizeof(uint32_t)) * cells + sizeof(int) * head.size();
+            p.bytes = diag_bytes(A);
             dspmm_status_t s = hip_status(hipMalloc(&p.d_mem, p.bytes));
             if (s == DSPMM_STATUS_SUCCESS) {
                 p.d_vals = reinterpret_cast<float4 *>(p.d_mem);

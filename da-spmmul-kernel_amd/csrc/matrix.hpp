@@ -165,6 +165,8 @@ dspmm_status_t get_ring_plan(dspmm_matrix_s *A, int w, int h, int zchunk, RingPl
                              bool build = true);
 // Whether the matrix goes in diagonal slices (computed once per matrix).
 bool diag_fits(dspmm_matrix_s *A);
+// Device bytes of the slices of a matrix that goes in them and has none yet.
+size_t diag_bytes(const dspmm_matrix_s *A);
 // The matrix's diagonal-slice plan, looked for and built on first use
 // (build == false: DSPMM_STATUS_NOT_PREPARED if it was not); *out is NULL for
 // a matrix that has none, or none that the device had memory for.

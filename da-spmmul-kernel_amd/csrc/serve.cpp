@@ -108,6 +108,7 @@ struct Job {
     const void *B = nullptr;
     float *C = nullptr;
     float *carry = nullptr;
+    const dspmm_config *own = nullptr; // of a request that runs alone (NULL: AUTO)
 };
 
 struct Slot {
@@ -191,6 +192,28 @@ struct dspmm_server_s {
         return cfg.plain == 0 && (int64_t)m.nnz >= (cfg.alone_nnz > 0 ? cfg.alone_nnz : kServeAloneNnz);
     }
 
+    // The configuration of a request that runs its matrix's own AUTO kernel: NULL
+    // (AUTO), except that an SpMV may want the matrix a second time, as slices of
+    // diagonals.  They count as the cache's memory; where it has none left for
+    // them, the tiles run.
+    const dspmm_config *own_config(SMat &m, int nv) {
+        static const dspmm_config tiles = {DSPMM_VARIANT_SPMV_TILED, 0, 0, 1024, 0, 0};
+        if (nv != 1) return nullptr;
+        std::lock_guard<std::mutex> lk(m.h->mu);
+        const dspmm_config c = resolve(m.h, DENSE_ROW_MAJOR, 1, cfg.btype, nullptr);
+        if (c.variant != DSPMM_VARIANT_SPMV_TILED || c.tile_nnz > 0 || !diag_fits(m.h)) return nullptr;
+        if (!m.h->diag.known) {
+            if (cache_used + diag_bytes(m.h) > cfg.cache_bytes) return &tiles;
+            DiagPlan *plan = nullptr;
+            if (get_diag_plan(m.h, &plan) == DSPMM_STATUS_SUCCESS && plan) {
+                m.bytes += plan->bytes;
+                cache_used += plan->bytes;
+                cache_peak = std::max(cache_peak, cache_used);
+            }
+        }
+        return nullptr;
+    }
+
     // The (matrix, nv) fragment, computed on the first request and kept
     // while the matrix stays resident: admission copies it.  The arena's
     // operands are 256-byte aligned with ld = nv, so one alignment class.
@@ -201,11 +224,13 @@ struct dspmm_server_s {
         if (schedule_item(m.h, nv, nv, nv, reinterpret_cast<const void *>(256),
                           reinterpret_cast<const void *>(256), cfg.btype, fr.f) != DSPMM_STATUS_SUCCESS)
             return nullptr;
-        if (dspmm_spmm_ex_resolve(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, nullptr, &fr.own) ==
-                DSPMM_STATUS_SUCCESS &&
-            dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, &fr.own, &fr.own_ws) ==
-                DSPMM_STATUS_SUCCESS)
-            fr.own_ok = fr.f.nsplits == 0 && row_exact(m.h, nv, fr.own);
+        // (the workspace query builds the kernel's plan: only where it may run)
+        fr.own_ok = fr.f.nsplits == 0 &&
+                    dspmm_spmm_ex_resolve(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, nullptr, &fr.own) ==
+                        DSPMM_STATUS_SUCCESS &&
+                    row_exact(m.h, nv, fr.own) &&
+                    dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, &fr.own,
+                                                 &fr.own_ws) == DSPMM_STATUS_SUCCESS;
         // the own kernel's plan (a ring plan, say) built now, at admission,
         // not inside a launch (placeholder operands: only their alignment
         // class and strides matter)
@@ -246,8 +271,10 @@ struct dspmm_server_s {
         if (runs_alone(m)) {
             // its own AUTO configuration's workspace (slots run concurrently,
             // so the handle's internal buffer cannot be shared)
-            (void)dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, r.nv, cfg.btype, nullptr,
-                                               &carry);
+            j.own = own_config(m, r.nv);
+            (void)dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, r.nv, cfg.btype, j.own, &carry);
+        } else if (cfg.plain == 2) {
+            // the handle's own buffers
         } else if (const Frag *fr = fragment(m, r.nv)) {
             carry = sizeof(float) * (size_t)fr->f.nslots * (size_t)fr->f.d.ldcarry;
             if (fr->own_ok) carry = std::max(carry, fr->own_ws);
@@ -336,7 +363,7 @@ struct dspmm_server_s {
             if (own.size() != jobs.size() || jobs.size() > kServeOwnMax) own.clear();
             if (st == DSPMM_STATUS_SUCCESS && own.empty())
                 st = assemble_schedule(fp.data(), items.data(), (int)items.size(), sch);
-        } else {
+        } else if (!alone && cfg.plain != 2) {
             st = build_schedule(items.data(), (int)items.size(), cfg.btype, sch, false);
         }
         if (st == DSPMM_STATUS_SUCCESS) {
@@ -354,7 +381,7 @@ struct dspmm_server_s {
             } else if (alone) {
                 const Job &j = jobs[0];
                 st = dspmm_spmm_ex(items[0].A, DENSE_ROW_MAJOR, j.r.nv, j.B, j.r.nv, cfg.btype, j.C,
-                                   j.r.nv, nullptr, j.carry, j.szK,
+                                   j.r.nv, j.own, j.carry, j.szK,
                                    reinterpret_cast<dspmm_stream_t>(sl.st));
             } else if (cfg.plain == 2) {
                 // the matrix's own AUTO configuration and workspace (requests
@@ -362,7 +389,7 @@ struct dspmm_server_s {
                 // by two launches at once)
                 const Job &j = jobs[0];
                 st = dspmm_spmm_ex(items[0].A, DENSE_ROW_MAJOR, j.r.nv, j.B, j.r.nv, cfg.btype, j.C,
-                                   j.r.nv, nullptr, nullptr, 0,
+                                   j.r.nv, own_config(mats[(size_t)j.r.matrix], j.r.nv), nullptr, 0,
                                    reinterpret_cast<dspmm_stream_t>(sl.st));
             } else if (cfg.plain) {
                 const Job &j = jobs[0];
