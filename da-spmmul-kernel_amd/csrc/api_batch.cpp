@@ -89,7 +89,8 @@ static ItemTiles item_tiles(const dspmm_matrix_s *A, int nv, bool bf16) {
 }
 
 dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc, const void *B,
-                             const void *C, dspmm_dtype_t btype, ItemFragment &f, bool whole) {
+                             const void *C, dspmm_dtype_t btype, ItemFragment &f, bool whole,
+                             size_t most_carry) {
     const bool bf16 = btype == DSPMM_R_16BF;
     f = ItemFragment{};
     if (!A || nv < 1 || ldb < nv || ldc < nv) return DSPMM_STATUS_INVALID_VALUE;
@@ -98,7 +99,8 @@ dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc
     // whole GPU and its caches: they make the batch slower.
     const ItemTiles t = item_tiles(A, nv, bf16);
     const double cost = item_cost(A, nv, bf16);
-    const dspmm_config c = whole || t.kept * kBatchSplit > cost ? t.whole : t.brief;
+    dspmm_config c = whole || t.kept * kBatchSplit > cost ? t.whole : t.brief;
+    while (carry_bytes(A, c.tile_nnz, nv) > most_carry && longer_tiles(nv, bf16, c)) complete_nb(c, nv, bf16);
     if (nnz_tiled_lds_bytes(c.lanes, c.tile_nnz) > kMaxTileLds) return DSPMM_STATUS_NOT_SUPPORTED;
     NbPlan *plan = nullptr;
     dspmm_status_t st = get_plan(A, c.tile_nnz, &plan);
@@ -128,7 +130,7 @@ dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc
 }
 
 dspmm_status_t build_schedule(const dspmm_batch_item *items, int count, dspmm_dtype_t btype,
-                              BatchSchedule &s, bool together) {
+                              BatchSchedule &s, bool together, size_t most_carry) {
     std::vector<ItemFragment> frags((size_t)count);
     std::vector<const ItemFragment *> fp((size_t)count);
     const bool bf16 = btype == DSPMM_R_16BF;
@@ -144,7 +146,7 @@ dspmm_status_t build_schedule(const dspmm_batch_item *items, int count, dspmm_dt
     for (int i = 0; i < count; i++) {
         const dspmm_batch_item &it = items[i];
         dspmm_status_t st = schedule_item(it.A, it.nv, it.ldb, it.ldc, it.B, it.C, btype,
-                                          frags[(size_t)i], whole);
+                                          frags[(size_t)i], whole, most_carry);
         if (st != DSPMM_STATUS_SUCCESS) return st;
         fp[(size_t)i] = &frags[(size_t)i];
     }
@@ -273,11 +275,19 @@ dspmm_status_t dspmm_batch_create(dspmm_batch_t *out, const dspmm_batch_item *it
         b->align_vw.push_back(choose_vw(it.nv, it.ldb, it.ldc, it.B, it.C,
                                         btype == DSPMM_R_16BF ? 2 : 4,
                                         btype == DSPMM_R_16BF ? 8 : 4));
-    b->nblocks = schedule_blocks(b->sch, blocks_per_cu);
-    if (b->sch.carry_floats > 0) {
+    auto alloc_carry = [&]() -> dspmm_status_t {
         b->carry_bytes = sizeof(float) * (size_t)b->sch.carry_floats;
-        st = hip_status(hipMalloc((void **)&b->carry, b->carry_bytes));
+        if (b->carry_bytes == 0) return DSPMM_STATUS_SUCCESS;
+        return hip_status(hipMalloc((void **)&b->carry, b->carry_bytes));
+    };
+    st = alloc_carry();
+    if (st == DSPMM_STATUS_ALLOC_FAILED) {         // the longest tiles have the fewest carries
+        (void)hipGetLastError();
+        b->carry = nullptr;
+        st = build_schedule(items, count, btype, b->sch, true, 0);
+        if (st == DSPMM_STATUS_SUCCESS) st = alloc_carry();
     }
+    b->nblocks = schedule_blocks(b->sch, blocks_per_cu);
     for (int i = 0; i < count && st == DSPMM_STATUS_SUCCESS; i++)
         b->sch.items[(size_t)i].carry = b->carry ? b->carry + b->sch.carry_off[(size_t)i] : nullptr;
     if (st == DSPMM_STATUS_SUCCESS) st = to_device(&b->d_items, b->sch.items);

@@ -69,6 +69,7 @@ void compute_stats(dspmm_matrix_s *A) {
         A->max_len = std::max(A->max_len, len);
         s += len;
         s2 += (double)len * len;
+        for (int k = 0; k < 6 && len > 8 << k; k++) A->slots[k] += (len + (8 << k) - 1) / (8 << k);
     }
     A->mean = A->nr ? s / A->nr : 0.0;
     const double var = A->nr ? std::max(0.0, s2 / A->nr - A->mean * A->mean) : 0.0;
@@ -466,6 +467,21 @@ dspmm_status_t get_plan(dspmm_matrix_s *A, int S, NbPlan **out, int kind, int st
 int64_t carry_ld(int nv) { return ((int64_t)nv + 7) / 8 * 8; }
 
 
+int64_t carry_slots(const dspmm_matrix_s *A, int S) {
+    for (int k = 0; k < 6; k++)
+        if (S == 8 << k) return A->slots[k];
+    int64_t n = 0;
+    for (int r = 0; r < A->nr; r++) {
+        const int len = A->h_rowPtr[(size_t)r + 1] - A->h_rowPtr[(size_t)r];
+        if (len > S) n += (len + S - 1) / S;
+    }
+    return n;
+}
+
+size_t carry_bytes(const dspmm_matrix_s *A, int S, int nv) {
+    return sizeof(float) * (size_t)carry_slots(A, S) * (size_t)carry_ld(nv);
+}
+
 int default_tile(int lanes) { return std::max(16, std::min(256, 16 * lanes)); }
 
 // Unset fields of a configuration whose vectors may be auto_vw wide.
@@ -488,6 +504,7 @@ void complete_aligned(dspmm_config &c, int nv, int64_t ldb, int64_t ldc, const v
     complete_vw(c, nv, choose_vw(nv, ldb, ldc, B, C, bf16 ? 2 : 4, bf16 ? 8 : 4));
 }
 
+size_t transposed_bytes(const dspmm_matrix_s *A, int nv, bool bf16);
 constexpr int kSpmvTile = 1024;
 constexpr int kCachedUmaxDefault = 128;
 constexpr double kCachedMinReuse = 1.5;   // sampled nonzeros per distinct column
@@ -508,16 +525,40 @@ constexpr int64_t kInPlaceWork = 5500000;
 // enough that the launch has kTileWaves wavefronts (a wavefront owns 64 /
 // lanes tiles).  Power law, 262144 rows, BF16 B: nv = 32 and 16 per tile
 // 74 us, 64 142; nv = 128 and 32 per tile 160 us, 256 442 (3100 wavefronts
-// of long serial tiles).  The batch keeps default_tile: its items share the
-// GPU, and small tiles made it slower.
+// of long serial tiles).  A batch sizes its items' tiles by other rules: they
+// share the GPU.
 constexpr int kTileWaves = 2048;
+bool longer_tiles(int nv, bool bf16, dspmm_config &c) {
+    dspmm_config full = c;
+    complete_nb(full, nv, bf16);
+    if (full.tile_nnz >= kTileMost) return false;
+    if (nnz_tiled_lds_bytes(full.lanes, 2 * full.tile_nnz) <= kMaxTileLds) {
+        c.tile_nnz = 2 * full.tile_nnz;
+    } else if (full.vec > 1) {                     // more lanes per tile: fewer tiles staged
+        c.tile_nnz = full.tile_nnz;
+        c.vec = full.vec / 2;
+        c.lanes = 0;
+    } else {
+        return false;
+    }
+    return true;
+}
+// Longer tiles while the carries of split rows exceed what dspmm_spmm_ex_noalloc
+// has for them (and the handle would keep).  Power law, BF16 B, 262144 rows, nv = 256:
+// 64 per tile 79 MB of carries, 128 39 MB; 1000000 rows, nv = 128: 64 per tile 150 MB, 256 38.
+void fit_carries(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, dspmm_config &c) {
+    const size_t copies = rm ? 0 : transposed_bytes(A, nv, bf16);
+    const size_t most = DSPMM_NOALLOC_SCRATCH_BYTES;
+    const size_t left = copies < most ? most - copies : most;
+    while (carry_bytes(A, c.tile_nnz, nv) > left && longer_tiles(nv, bf16, c)) {}
+}
 // Halves the tile until the launch's LDS fits.
 void fit_tile(int nv, bool bf16, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
     while (nnz_tiled_lds_bytes(full.lanes, c.tile_nnz) > kMaxTileLds) c.tile_nnz /= 2;
 }
-void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_config &c) {
+void single_tile(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, int cap, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
     const int64_t slabs = div_up(nv, full.vec * full.lanes), g = 64 / full.lanes;
@@ -529,6 +570,7 @@ void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_conf
            A->nnz * slabs / (g * c.tile_nnz) < kTileWaves)
         c.tile_nnz /= 2;
     fit_tile(nv, bf16, c);
+    fit_carries(A, rm, nv, bf16, c);
 }
 
 // Whether one row outlasts the others of a row-per-group kernel.
@@ -569,7 +611,7 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
         // lane and 32 per tile 43, eight a lane 132 (each gather instruction
         // then reaches 64 rows of B)
         c.vec = std::min(2, nv);
-        single_tile(A, nv, bf16, skew ? 16 : 32, c);
+        single_tile(A, rm, nv, bf16, skew ? 16 : 32, c);
     } else if (skew) {
         if (bf16 && nv > 32)
             // few nonzeros: more lanes per tile before shorter tiles (11257 rows,
@@ -581,7 +623,7 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
                 if ((int64_t)A->nnz * div_up(nv, full.vec * full.lanes) / (64 / full.lanes * 32) >= kTileWaves)
                     break;
             }
-        single_tile(A, nv, bf16, 0, c);
+        single_tile(A, rm, nv, bf16, 0, c);
     } else {
         // rows of like lengths: a group per row, without tiles and split rows
         // (4096 rows of 16, nv = 20 to 128: 4.7 to 5.5 / 8.7 to 12.3)
@@ -601,11 +643,12 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
                 // 4120 rows of 91, nv = 12: 10.3, 128 per tile 31.4; 3368 rows of 70,
                 // nv = 30: 10.1, 31.1
                 c.vec = 4;
-                single_tile(A, nv, bf16, A->max_len <= 32 ? 32 : 16, c);
+                single_tile(A, rm, nv, bf16, A->max_len <= 32 ? 32 : 16, c);
             } else {
                 c.unroll = 8;
                 c.tile_nnz = 128;
                 fit_tile(nv, bf16, c);
+                fit_carries(A, rm, nv, bf16, c);
             }
         } else {
             c.variant = DSPMM_VARIANT_CSR_SCALAR;
@@ -1388,14 +1431,28 @@ dspmm_status_t dspmm_spmm_ex(dspmm_matrix_t A, DenseLayout layout, int nv, const
     if (A->nr == 0) return DSPMM_STATUS_SUCCESS;
     std::lock_guard<std::mutex> lk(A->mu);
     const dspmm_config c = resolve(A, layout, nv, btype, cfg);
-    st = run_ex(A, layout, nv, B, ldb, btype, C, ldc, c, workspace, workspace_bytes, as_hip(stream));
-    if (st == DSPMM_STATUS_NOT_SUPPORTED && (!cfg || cfg->variant == DSPMM_VARIANT_AUTO)) {
-        // a selected configuration these operands cannot run (alignment,
-        // LDS): the static default instead
-        const dspmm_config h = heuristic(A, layout, nv, btype);
-        st = run_ex(A, layout, nv, B, ldb, btype, C, ldc, h, workspace, workspace_bytes,
-                    as_hip(stream));
-    }
+    const bool auto_cfg = !cfg || cfg->variant == DSPMM_VARIANT_AUTO;
+    const bool tuned = A->tuned.count(std::make_tuple((int)layout, nv, (int)btype)) != 0;
+    auto run = [&](const dspmm_config &rc) -> dspmm_status_t {
+        dspmm_status_t s = run_ex(A, layout, nv, B, ldb, btype, C, ldc, rc, workspace, workspace_bytes,
+                                  as_hip(stream));
+        if (s != DSPMM_STATUS_WORKSPACE_TOO_SMALL || !workspace || !auto_cfg || tuned ||
+            rc.variant != DSPMM_VARIANT_NNZ_TILED)
+            return s;
+        // AUTO's own tiles: longer ones need fewer carries
+        const bool bf16 = btype == DSPMM_R_16BF;
+        const size_t copies = layout == DENSE_COL_MAJOR && nv > 1 ? transposed_bytes(A, nv, bf16) : 0;
+        dspmm_config l = rc;
+        while (longer_tiles(nv, bf16, l))
+            if (copies + carry_bytes(A, l.tile_nnz, nv) <= workspace_bytes)
+                return run_ex(A, layout, nv, B, ldb, btype, C, ldc, l, workspace, workspace_bytes,
+                              as_hip(stream));
+        return s;
+    };
+    st = run(c);
+    // a selected configuration these operands cannot run (alignment, LDS): the
+    // static default instead
+    if (st == DSPMM_STATUS_NOT_SUPPORTED && auto_cfg) st = run(heuristic(A, layout, nv, btype));
     return st;
 }
 

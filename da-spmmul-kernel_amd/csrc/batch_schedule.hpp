@@ -2,6 +2,7 @@
 // (shared by dspmm_batch_* and the serving loop).
 #pragma once
 
+#include <cstdint>
 #include <vector>
 
 #include "dspmm.h"
@@ -38,10 +39,11 @@ struct ItemFragment {
 };
 
 // The fragment of matrix A with nv columns (locks A while reading it).  `whole`:
-// with tiles that leave more rows whole, where there are such.
+// with tiles that leave more rows whole, where there are such.  Tiles grow until
+// the carries take at most `most_carry` bytes, as far as tiles go.
 dspmm_status_t schedule_item(dspmm_matrix_s *A, int nv, int64_t ldb, int64_t ldc, const void *B,
                              const void *C, dspmm_dtype_t btype, ItemFragment &f,
-                             bool whole = false);
+                             bool whole = false, size_t most_carry = SIZE_MAX);
 // A schedule from one fragment per item (frags[i] for items[i], whose
 // operands and strides are bound here): carry offsets, split prefix sums and
 // the per-XCD segments.
@@ -51,7 +53,7 @@ dspmm_status_t assemble_schedule(const ItemFragment *const *frags, const dspmm_b
 // tiles are chosen for the batch as a whole; without, an item's tiles, and so the
 // bits of its result, do not depend on its company.
 dspmm_status_t build_schedule(const dspmm_batch_item *items, int count, dspmm_dtype_t btype,
-                              BatchSchedule &s, bool together);
+                              BatchSchedule &s, bool together, size_t most_carry = SIZE_MAX);
 // Workgroups of the launch: blocks_per_cu > 0 -> persistent grid.
 int schedule_blocks(const BatchSchedule &s, int blocks_per_cu);
 

@@ -113,6 +113,7 @@ struct dspmm_matrix_s {
     std::vector<float> h_values;
     int max_len = 0;
     double mean = 0, cv = 0;
+    int64_t slots[6] = {0};     // carry slots of nnz tiles of 8, 16, ... 256 nonzeros
     size_t base_bytes = 0;
     std::mutex mu;
     std::map<int64_t, dspmm::NbPlan> plans;                        // by 4 * (tile size + 16 * (stride - 1)) + kind
@@ -182,6 +183,13 @@ void ring_bind_plan(dspmm_matrix_s *A, const RingPlan &plan, RingLaunch &a);
 int ring_auto_z(dspmm_matrix_s *A, int w, int h);
 int cached_smax(int umax);
 int64_t carry_ld(int nv);
+// Carry slots that tiles of S nonzeros need, and their bytes at nv columns.
+int64_t carry_slots(const dspmm_matrix_s *A, int S);
+size_t carry_bytes(const dspmm_matrix_s *A, int S, int nv);
+// The next configuration with longer tiles, up to kTileMost nonzeros; false if
+// there is none.
+bool longer_tiles(int nv, bool bf16, dspmm_config &c);
+constexpr int kTileMost = 256;
 int default_tile(int lanes);
 void complete_nb(dspmm_config &c, int nv, bool bf16);
 // The configuration a call runs: cfg unless AUTO, else the tuned one cached

@@ -108,7 +108,7 @@ struct Job {
     const void *B = nullptr;
     float *C = nullptr;
     float *carry = nullptr;
-    const dspmm_config *own = nullptr; // of a request that runs alone (NULL: AUTO)
+    dspmm_config own{};                // of a request that runs alone
 };
 
 struct Slot {
@@ -192,18 +192,38 @@ struct dspmm_server_s {
         return cfg.plain == 0 && (int64_t)m.nnz >= (cfg.alone_nnz > 0 ? cfg.alone_nnz : kServeAloneNnz);
     }
 
-    // The configuration of a request that runs its matrix's own AUTO kernel: NULL
-    // (AUTO), except that an SpMV may want the matrix a second time, as slices of
-    // diagonals.  They count as the cache's memory; where it has none left for
-    // them, the tiles run.
-    const dspmm_config *own_config(SMat &m, int nv) {
-        static const dspmm_config tiles = {DSPMM_VARIANT_SPMV_TILED, 0, 0, 1024, 0, 0};
-        if (nv != 1) return nullptr;
+    // Bytes of the arena that a request with operands of its own leaves for
+    // carries.  What fits depends on the matrix and nv alone, not on the requests
+    // in flight, so that a result has the same bits each time.
+    size_t carry_room(const SMat &m, int nv) const {
+        const size_t dense = round_up((size_t)m.nc * (size_t)nv * elem_b(), 256) +
+                             round_up((size_t)m.nr * (size_t)nv * sizeof(float), 256);
+        return dense < arena.size() ? arena.size() - dense : SIZE_MAX;
+    }
+
+    // The configuration of a request that runs its matrix's own AUTO kernel; AUTO,
+    // except that
+    //   * an SpMV may want the matrix a second time, as slices of diagonals.  They
+    //     count as the cache's memory; where it has none left, the tiles run;
+    //   * tiles grow until their carries fit the arena.
+    dspmm_config own_config(SMat &m, int nv) {
         std::lock_guard<std::mutex> lk(m.h->mu);
-        const dspmm_config c = resolve(m.h, DENSE_ROW_MAJOR, 1, cfg.btype, nullptr);
-        if (c.variant != DSPMM_VARIANT_SPMV_TILED || c.tile_nnz > 0 || !diag_fits(m.h)) return nullptr;
+        dspmm_config c = resolve(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, nullptr);
+        const dspmm_config as_is{};
+        const bool bf16 = cfg.btype == DSPMM_R_16BF;
+        if (c.variant == DSPMM_VARIANT_NNZ_TILED && cfg.plain == 0) {
+            complete_nb(c, nv, bf16);
+            if (carry_bytes(m.h, c.tile_nnz, nv) <= carry_room(m, nv)) return as_is;
+            while (carry_bytes(m.h, c.tile_nnz, nv) > carry_room(m, nv) && longer_tiles(nv, bf16, c)) {}
+            return c;
+        }
+        if (nv != 1 || c.variant != DSPMM_VARIANT_SPMV_TILED || c.tile_nnz > 0 || !diag_fits(m.h))
+            return as_is;
         if (!m.h->diag.known) {
-            if (cache_used + diag_bytes(m.h) > cfg.cache_bytes) return &tiles;
+            if (cache_used + diag_bytes(m.h) > cfg.cache_bytes) {
+                c.tile_nnz = 1024;
+                return c;
+            }
             DiagPlan *plan = nullptr;
             if (get_diag_plan(m.h, &plan) == DSPMM_STATUS_SUCCESS && plan) {
                 m.bytes += plan->bytes;
@@ -211,7 +231,7 @@ struct dspmm_server_s {
                 cache_peak = std::max(cache_peak, cache_used);
             }
         }
-        return nullptr;
+        return as_is;
     }
 
     // The (matrix, nv) fragment, computed on the first request and kept
@@ -222,7 +242,8 @@ struct dspmm_server_s {
         if (it != m.frags.end()) return &it->second;
         Frag fr;
         if (schedule_item(m.h, nv, nv, nv, reinterpret_cast<const void *>(256),
-                          reinterpret_cast<const void *>(256), cfg.btype, fr.f) != DSPMM_STATUS_SUCCESS)
+                          reinterpret_cast<const void *>(256), cfg.btype, fr.f, false,
+                          carry_room(m, nv)) != DSPMM_STATUS_SUCCESS)
             return nullptr;
         // (the workspace query builds the kernel's plan: only where it may run)
         fr.own_ok = fr.f.nsplits == 0 &&
@@ -272,7 +293,15 @@ struct dspmm_server_s {
             // its own AUTO configuration's workspace (slots run concurrently,
             // so the handle's internal buffer cannot be shared)
             j.own = own_config(m, r.nv);
-            (void)dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, r.nv, cfg.btype, j.own, &carry);
+            (void)dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, r.nv, cfg.btype, &j.own, &carry);
+            if (carry > carry_room(m, r.nv)) {
+                // what AUTO falls back to may want more: its tiles grow to fit
+                dspmm_config c;
+                size_t need = 0;
+                (void)dspmm_spmm_ex_resolve(m.h, DENSE_ROW_MAJOR, r.nv, cfg.btype, &j.own, &c);
+                (void)dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, r.nv, cfg.btype, &c, &need);
+                carry = std::max(need, carry_room(m, r.nv));
+            }
         } else if (cfg.plain == 2) {
             // the handle's own buffers
         } else if (const Frag *fr = fragment(m, r.nv)) {
@@ -364,7 +393,9 @@ struct dspmm_server_s {
             if (st == DSPMM_STATUS_SUCCESS && own.empty())
                 st = assemble_schedule(fp.data(), items.data(), (int)items.size(), sch);
         } else if (!alone && cfg.plain != 2) {
-            st = build_schedule(items.data(), (int)items.size(), cfg.btype, sch, false);
+            const Job &j = jobs[0];                       // plain: one request at a time
+            st = build_schedule(items.data(), (int)items.size(), cfg.btype, sch, false,
+                                carry_room(mats[(size_t)j.r.matrix], j.r.nv));
         }
         if (st == DSPMM_STATUS_SUCCESS) {
             for (size_t i = 0; i < jobs.size() && i < sch.items.size(); i++) sch.items[i].carry = jobs[i].carry;
@@ -381,15 +412,16 @@ struct dspmm_server_s {
             } else if (alone) {
                 const Job &j = jobs[0];
                 st = dspmm_spmm_ex(items[0].A, DENSE_ROW_MAJOR, j.r.nv, j.B, j.r.nv, cfg.btype, j.C,
-                                   j.r.nv, j.own, j.carry, j.szK,
+                                   j.r.nv, &j.own, j.carry, j.szK,
                                    reinterpret_cast<dspmm_stream_t>(sl.st));
             } else if (cfg.plain == 2) {
                 // the matrix's own AUTO configuration and workspace (requests
                 // run in order on one stream, so the handle's buffer is not shared
                 // by two launches at once)
                 const Job &j = jobs[0];
+                const dspmm_config c = own_config(mats[(size_t)j.r.matrix], j.r.nv);
                 st = dspmm_spmm_ex(items[0].A, DENSE_ROW_MAJOR, j.r.nv, j.B, j.r.nv, cfg.btype, j.C,
-                                   j.r.nv, own_config(mats[(size_t)j.r.matrix], j.r.nv), nullptr, 0,
+                                   j.r.nv, &c, nullptr, 0,
                                    reinterpret_cast<dspmm_stream_t>(sl.st));
             } else if (cfg.plain) {
                 const Job &j = jobs[0];
