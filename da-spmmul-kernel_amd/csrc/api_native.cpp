@@ -72,6 +72,15 @@ void compute_stats(dspmm_matrix_s *A) {
         for (int k = 0; k < 6 && len > 8 << k; k++) A->slots[k] += (len + (8 << k) - 1) / (8 << k);
     }
     A->mean = A->nr ? s / A->nr : 0.0;
+    const double least = std::max(128.0, 4 * A->mean);
+    int longs = 0, pairs = 0, before = 0;
+    for (int r = 0; r < A->nr && A->max_len >= least; r++) {
+        const int len = rp[(size_t)r + 1] - rp[(size_t)r];
+        longs += len >= least;
+        pairs += len >= least && before >= least;
+        before = len;
+    }
+    A->clustered = pairs > longs / 2;
     const double var = A->nr ? std::max(0.0, s2 / A->nr - A->mean * A->mean) : 0.0;
     A->cv = A->mean > 0 ? std::sqrt(var) / A->mean : 0.0;
 }
@@ -558,19 +567,80 @@ void fit_tile(int nv, bool bf16, dspmm_config &c) {
     complete_nb(full, nv, bf16);
     while (nnz_tiled_lds_bytes(full.lanes, c.tile_nnz) > kMaxTileLds) c.tile_nnz /= 2;
 }
+// The tile of 16 nonzeros per lane, at vectors that divide nv: its order of
+// summation is the one that AUTO's may not fall behind in accuracy.
+int plain_tile(int nv, bool bf16) {
+    const int vw = choose_vw(nv, nv, nv, nullptr, nullptr, bf16 ? 2 : 4, bf16 ? 8 : 4);
+    return default_tile(std::min(64, pow2_ceil(div_up(nv, vw))));
+}
+// The longest chain of additions in a row of n nonzeros cut at S (k_split_combine
+// adds the chunks in up to 64 / nv parts).
+int64_t tile_chain(int64_t n, int S, int nv) {
+    if (n <= S) return n;
+    const int64_t parts = 64 / std::min(64, pow2_ceil(nv)), chunks = (n + S - 1) / S;
+    return S + (chunks + parts - 1) / parts + parts;
+}
 void single_tile(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, int cap, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
     const int64_t slabs = div_up(nv, full.vec * full.lanes), g = 64 / full.lanes;
-    c.tile_nnz = cap > 0 ? cap : full.lanes <= 4 ? 16 : full.lanes <= 32 ? 32 : 64;
+    c.tile_nnz = std::max(cap, full.lanes <= 4 ? 16 : full.lanes <= 32 ? 32 : 64);
     // a tile that just holds the longest row stays: smaller ones would split
     // rows and need the combine launch (32^3 stencil, BF16, nv = 11: 32 per tile
     // 10.5 us, 16 per tile 22)
-    while (c.tile_nnz > 8 && !(A->max_len <= c.tile_nnz && A->max_len > c.tile_nnz / 2) &&
+    const int least = A->mean > 160 ? 16 : 8;      // (2000 rows of 200, nv = 2: error 1.07 times in eights)
+    while (c.tile_nnz > least && !(A->max_len <= c.tile_nnz && A->max_len > c.tile_nnz / 2) &&
            A->nnz * slabs / (g * c.tile_nnz) < kTileWaves)
         c.tile_nnz /= 2;
+    // thousands of short chunks would be one long chain of the combine
+    const int plain = plain_tile(nv, bf16);
+    while (c.tile_nnz < plain &&
+           tile_chain(A->max_len, c.tile_nnz, nv) > 4 * tile_chain(A->max_len, plain, nv))
+        c.tile_nnz *= 2;
     fit_tile(nv, bf16, c);
     fit_carries(A, rm, nv, bf16, c);
+}
+
+// A lane group per row, for rows of like lengths: no tiles, no split rows.  False
+// where tiles are better.  Vectors as wide as the columns (or as BF16 allows), narrower
+// ones, to a quarter, where a wavefront's rows would overflow its window of pairs or
+// leave the GPU fewer than 1024 wavefronts.  BF16 B, us, tiles of 16 nonzeros per lane / this:
+// 60^3 stencil, nv = 2 145 / 25, nv = 8 111 / 22; 120000 rows of 20, nv = 48 121 / 47; 30000 of 27,
+// nv = 16 34 / 8; 2000 of 12, nv = 64 41 / 4.  Where the windows overflow all the same, rows wait
+// for one another's: 2000 of 100, nv = 2 9.0 in tiles of 8 / 28, 8000 of 100, nv = 8 12.7 / 20.7;
+// 30000 of 64, nv = 2 27.6 / 25.7.  Rows of more than kRowsMean want more than 32 columns and 3000
+// wavefronts, FP32: 8000 of 200, nv = 100 101 / 66; 8192 of 256, nv = 16 26 / 41, nv = 32 36 / 43.
+// Rows that 16 nonzeros per lane hold are summed in order, with the bits of such
+// tiles, longer ones in parts, which round no worse than they did cut.
+constexpr int kRowsLongest = 256;
+constexpr double kRowsMean = 110;
+bool row_groups(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, dspmm_config &c) {
+    if (A->max_len > kRowsLongest) return false;
+    const bool in_order = A->max_len <= plain_tile(nv, bf16);
+    if (rm && !bf16 && in_order) {                 // the reference class: windows of whole blocks
+        c = dspmm_config{};
+        c.variant = DSPMM_VARIANT_CSR_SCALAR;
+        return true;
+    }
+    // few nonzeros in few columns: tiles of 16 split them further (2000 rows of
+    // 64, nv = 8, either 7.3; 30000 of 27 the rows)
+    if (nv <= 8 && A->nnz < 300000) return false;
+    c = dspmm_config{};
+    c.vec = choose_vw_any(nv, bf16 ? 8 : 4);
+    const int least = std::max(1, c.vec / 4);
+    auto rows = [&]() {                        // of a wavefront
+        dspmm_config full = c;
+        complete_nb(full, nv, bf16);
+        return 64 / full.lanes;
+    };
+    while (c.vec > least && (A->mean * rows() > kRowSeqWindow || A->nr < 1024 * rows())) c.vec /= 2;
+    const bool overflow = A->mean * rows() > kRowSeqWindow;
+    if (overflow && rows() > 4 && (A->nr < 20000 || A->mean > 64)) return false;
+    if (A->mean > kRowsMean && (nv <= 32 || A->nr < 3000 * rows())) return false;
+    c.variant = in_order ? DSPMM_VARIANT_CSR_SCALAR : DSPMM_VARIANT_CSR_PARTS;
+    c.unroll = in_order ? 4 : 8;
+    c.tile_nnz = overflow ? 1 : 0;
+    return true;
 }
 
 // Whether one row outlasts the others of a row-per-group kernel.
@@ -587,7 +657,7 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
         return c;
     }
     const int64_t work = (int64_t)A->nnz * nv;
-    if (!rm && !bf16 && nv < 8 && (nv <= 3 || work < kInPlaceWork)) {
+    if (!rm && !bf16 && nv < 8 && (nv <= 3 || work < kInPlaceWork) && !A->clustered) {
         c.variant = DSPMM_VARIANT_CSR_VECTOR;
         return c;
     }
@@ -600,65 +670,49 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
     c.variant = DSPMM_VARIANT_NNZ_TILED;
     c.unroll = 4;
     const bool skew = skewed(A);
-    if ((bf16 || !rm) && nv < 8 && !skew && A->mean <= 48 && A->nr >= 512 * A->mean) {
-        // a lane per row, where enough wavefronts of them hide its gathers: 98^3
-        // stencil, nv = 2: 95, tiles 569; 38111 rows of 18, nv = 6: 13.6, 23; but
-        // 2131 rows of 25, nv = 6: 10.1, 8.3 and 24000 rows of 103, nv = 2: 231, 32;
-        // FP32 copies, 97096 rows of 34, nv = 6: 47, 77
-        c.variant = DSPMM_VARIANT_CSR_SCALAR;
-    } else if (nv <= 8) {
-        // four lanes and more per tile: 64^3 stencil, nv = 8, two values a
-        // lane and 32 per tile 43, eight a lane 132 (each gather instruction
-        // then reaches 64 rows of B)
-        c.vec = std::min(2, nv);
-        single_tile(A, rm, nv, bf16, skew ? 16 : 32, c);
-    } else if (skew) {
-        if (bf16 && nv > 32)
-            // few nonzeros: more lanes per tile before shorter tiles (11257 rows,
-            // the longest 1100, nv = 81: two values a lane 15.9, eight 19.7; 8729
-            // rows, the longest 2600, nv = 122: 18.6, 31.5)
-            for (c.vec = 8; c.vec > 2; c.vec /= 2) {
-                dspmm_config full = c;
-                complete_nb(full, nv, bf16);
-                if ((int64_t)A->nnz * div_up(nv, full.vec * full.lanes) / (64 / full.lanes * 32) >= kTileWaves)
-                    break;
-            }
-        single_tile(A, rm, nv, bf16, 0, c);
-    } else {
-        // rows of like lengths: a group per row, without tiles and split rows
-        // (4096 rows of 16, nv = 20 to 128: 4.7 to 5.5 / 8.7 to 12.3)
+    if (!rm && !bf16 && !skew && nv > 8 && nv <= 32 && work < kInPlaceWork && !A->clustered) {
+        // (overflowing windows: in place no worse than the copies)
         dspmm_config full{};
         complete_nb(full, nv, bf16);
-        const bool overflow = A->mean * (64 / full.lanes) > kRowSeqWindow;
-        if (overflow && nv <= 32 && (bf16 || !rm)) {
-            // long rows side by side would wait for one another's windows
-            // (20000 rows of 100, nv = 20: 32 / 66, sliced 38)
-            if (!bf16 && work < kInPlaceWork) {
-                c.variant = DSPMM_VARIANT_CSR_VECTOR;
-            } else if (bf16 && A->mean <= 64 && A->nnz >= 2000000) {
-                // sliced: 84200 rows of 48, nv = 28: 36, tiles 76 and more
-                c.variant = DSPMM_VARIANT_CSR_SCALAR;
-                c.tile_nnz = 1;
-            } else if (bf16) {
-                // 4120 rows of 91, nv = 12: 10.3, 128 per tile 31.4; 3368 rows of 70,
-                // nv = 30: 10.1, 31.1
-                c.vec = 4;
-                single_tile(A, rm, nv, bf16, A->max_len <= 32 ? 32 : 16, c);
-            } else {
-                c.unroll = 8;
-                c.tile_nnz = 128;
-                fit_tile(nv, bf16, c);
-                fit_carries(A, rm, nv, bf16, c);
-            }
-        } else {
-            c.variant = DSPMM_VARIANT_CSR_SCALAR;
-            c.unroll = bf16 || !rm ? 4 : 0;
-            if (overflow && c.unroll > 0) {
-                c.unroll = 16;
-                c.tile_nnz = 1;                // sliced windows: nv = 64, 32 / 43
-            }
+        if (A->mean * (64 / full.lanes) > kRowSeqWindow) {
+            c = dspmm_config{};
+            c.variant = DSPMM_VARIANT_CSR_VECTOR;
+            return c;
         }
     }
+    if (!skew) {
+        dspmm_config rows;
+        if (row_groups(A, rm, nv, bf16, rows)) return rows;
+    }
+    if (nv <= 8) {
+        // four lanes and more per tile: 64^3 stencil, nv = 8, two values a
+        // lane and 32 per tile 43, eight a lane 132 (each gather instruction
+        // then reaches 64 rows of B); 8000 rows of 100, nv = 2: one a lane 14.1, two 17.3
+        // (2 million nonzeros fill the GPU anyway: band of 256, 8192 rows, nv = 2: 19.5, 17.3)
+        c.vec = nv <= 3 && A->nnz < 2000000 ? 1 : 2;
+    } else if (bf16 && (nv > 32 || !skew)) {
+        // few nonzeros: more lanes per tile before shorter tiles (11257 rows,
+        // the longest 1100, nv = 81: two values a lane 15.9, eight 19.7; 8729
+        // rows, the longest 2600, nv = 122: 18.6, 31.5; 2000 rows of 100, nv = 24: four
+        // a lane 8.9, eight 11)
+        for (c.vec = choose_vw_any(nv, 8); c.vec > 2; c.vec /= 2) {
+            dspmm_config full = c;
+            complete_nb(full, nv, bf16);
+            const int S = full.lanes <= 4 ? 16 : 32;
+            if ((int64_t)A->nnz * div_up(nv, full.vec * full.lanes) / (64 / full.lanes * S) >= kTileWaves)
+                break;
+        }
+    }
+    // rows of like lengths with some beyond the groups': tiles that most of them
+    // fit; long rows: few chunks
+    int cap = 0;
+    if (!skew && A->mean <= 64 && A->max_len > kRowsLongest)
+        cap = std::min(plain_tile(nv, bf16), pow2_ceil((int)(2 * A->mean) + 1));
+    if (A->mean > 512) {
+        cap = std::min(plain_tile(nv, bf16), 128);
+        if (nv > 32) c.unroll = 8;             // (4096 rows of 2000, FP32, nv = 128: 79 / 92 in fours)
+    }
+    single_tile(A, rm, nv, bf16, cap, c);
     return c;
 }
 
@@ -668,33 +722,34 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
 void adjust_pick(dspmm_matrix_s *A, int nv, dspmm_config &c) {
     if (c.variant == DSPMM_VARIANT_RING) return;
     const bool skew = skewed(A);
-    int v = c.variant;
-    int unroll = 0;
+    dspmm_config p{};
+    p.variant = DSPMM_VARIANT_CSR_VECTOR;
     if (nv == 1) {
         // no products through LDS where many rows are summed by several lanes, off
         // the diagonal slices: 110136 rows of 30 15.9 / 18.2, 143583 of 23 13.2 /
         // 15.1; 107445 of 66 36.8 / 33.6, 12691 of 50 the same
         if (skew || A->mean <= 20 || A->mean > 64 || A->nnz < 2000000 ||
             column_reuse(A) >= kRowBlockMinReuse) return;
-        v = DSPMM_VARIANT_CSR_VECTOR;
     } else if (nv <= 8) {
-        v = DSPMM_VARIANT_CSR_VECTOR;          // skewed rows: 0.58 of the pick's time, at most 0.66
-        if (!skew && A->mean <= 32 && (int64_t)A->nnz * nv >= 16000000 && column_reuse(A) >= kRowBlockMinReuse) {
-            // neighbouring rows share B rows: 74^3 stencil, nv = 3: 32 / 55; 64^3, nv = 5: 26 / 36
-            // (78714 rows of 72 on 2463 columns, nv = 5: 98 / 52)
-            if (nv <= 3) v = DSPMM_VARIANT_CSR_SCALAR;
-            if (nv >= 5) { v = DSPMM_VARIANT_CSR_SCALAR; unroll = 4; }
+        // skewed rows: 0.58 of the pick's time, at most 0.66; but with the long rows
+        // side by side 262144 of a power law, nv = 8, 92 / 59
+        if (skew && A->clustered) return;
+        if (!skew && nv != 2 && nv != 4 && A->mean <= 32 && (int64_t)A->nnz * nv >= 16000000 &&
+            column_reuse(A) >= kRowBlockMinReuse) {
+            // neighbouring rows share B rows (60^3 stencil, vector kernel / in parts: nv = 3
+            // 28.6 / 21.5, nv = 5 30.6 / 25.7, nv = 2 16.7 / 21.5)
+            p.variant = DSPMM_VARIANT_CSR_PARTS;
+            p.vec = nv <= 3 ? 1 : 0;
         }
-    } else if (nv <= 32 && v == DSPMM_VARIANT_CSR_VECTOR && !skew && A->mean <= 32 && A->nnz >= 400000) {
-        // 65^3 stencil, nv = 15: 27 / 75; 58782 rows of 20, nv = 15: 20 / 24; below that many
-        // nonzeros, or with longer rows, no faster
-        v = DSPMM_VARIANT_CSR_SCALAR;
+    } else if (nv <= 32 && c.variant == DSPMM_VARIANT_CSR_VECTOR && !skew && A->mean <= 32 &&
+               A->nnz >= 400000 && (double)A->nc * nv >= 500000) {
+        // B beyond the vector kernel's reach of the L2s (60^3 stencil, nv = 12: 31 / 57; 120000
+        // rows of 20, nv = 16: 27 / 40; 30000 of 27, nv = 24 10.5 / 11.3, nv = 16 9.5 / 7.9)
+        p.variant = DSPMM_VARIANT_CSR_PARTS;
     } else {
         return;
     }
-    c = dspmm_config{};
-    c.variant = v;
-    c.unroll = unroll;
+    c = p;
 }
 
 // Row-major-only native kernels: on column-major operands they run on
@@ -704,6 +759,7 @@ bool rm_native(const dspmm_config &c, bool bf16) {
     case DSPMM_VARIANT_NNZ_TILED:
     case DSPMM_VARIANT_ROW_BLOCKED:
     case DSPMM_VARIANT_NNZ_CACHED:
+    case DSPMM_VARIANT_CSR_PARTS:
     case DSPMM_VARIANT_RING: return true;
     case DSPMM_VARIANT_CSR_SCALAR: return c.unroll > 0 || bf16;
     default: return false;
@@ -1064,17 +1120,23 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         a.mid_event = mid;
         return launch_spmv_tiled(a, st);
     }
+    case DSPMM_VARIANT_CSR_PARTS:
     case DSPMM_VARIANT_CSR_SCALAR:
     case DSPMM_VARIANT_CSR_VECTOR:
     case DSPMM_VARIANT_COO_SCALAR:
     case DSPMM_VARIANT_COO_VECTOR: {
-        if (cfg.variant == DSPMM_VARIANT_CSR_SCALAR && layout == DENSE_ROW_MAJOR &&
-            (bf16 || cfg.unroll > 0)) {
+        const bool parts = cfg.variant == DSPMM_VARIANT_CSR_PARTS;
+        if (parts && layout != DENSE_ROW_MAJOR) return DSPMM_STATUS_NOT_SUPPORTED;
+        // staged by whole blocks, which neighbouring rows' columns then share in L1
+        // (60^3 stencil, nv = 12: 31 us by wavefronts, 24 by blocks)
+        const bool staged = parts && !bf16 && cfg.unroll <= 0 && nv >= 5 && nv <= 32;
+        if ((parts && !staged) || (cfg.variant == DSPMM_VARIANT_CSR_SCALAR && layout == DENSE_ROW_MAJOR &&
+                      (bf16 || cfg.unroll > 0))) {
             dspmm_config c = cfg;
             if (cfg.tile_nnz != 0 && cfg.tile_nnz != 1) return DSPMM_STATUS_NOT_SUPPORTED;
             c.tile_nnz = 0;
-            c.unroll = cfg.unroll > 0 ? cfg.unroll : 4;
-            if (!row_seq_unroll_ok(c.unroll)) return DSPMM_STATUS_NOT_SUPPORTED;
+            c.unroll = cfg.unroll > 0 ? cfg.unroll : parts ? 8 : 4;
+            if (!row_seq_unroll_ok(c.unroll) || (parts && c.unroll != 8)) return DSPMM_STATUS_NOT_SUPPORTED;
             if (!launch) return DSPMM_STATUS_SUCCESS;
             complete_nb(c, nv, bf16);
             const Slab sl = make_slab(nv, c.vec);
@@ -1094,6 +1156,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
             a.nslabs = div_up(nv, a.slab_w);
             a.unroll = c.unroll;
             a.sliced = cfg.tile_nnz == 1;
+            a.parts = parts;
             a.bf16 = bf16;
             dspmm_status_t s = launch_row_seq(a, st);
             if (s == DSPMM_STATUS_SUCCESS && mid) s = hip_status(hipEventRecord(mid, st));
@@ -1103,6 +1166,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         const bool rm = layout == DENSE_ROW_MAJOR;
         int which = 0;
         switch (cfg.variant) {
+        case DSPMM_VARIANT_CSR_PARTS: which = K_CSR_PARTS_ROW; break;
         case DSPMM_VARIANT_CSR_SCALAR: which = rm ? K_SPMM_CSR_SCALAR_ROW : K_SPMM_CSR_SCALAR_COL; break;
         case DSPMM_VARIANT_CSR_VECTOR: which = rm ? K_SPMM_CSR_VECTOR_ROW : K_SPMM_CSR_VECTOR_COL; break;
         case DSPMM_VARIANT_COO_SCALAR: which = rm ? K_SPMM_COO_SCALAR_ROW : K_SPMM_COO_SCALAR_COL; break;
@@ -1146,7 +1210,7 @@ dspmm_status_t check_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const voi
 }
 
 dspmm_config resolve(dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_t bt,
-                     const dspmm_config *cfg, bool learned) {
+                     const dspmm_config *cfg, bool learned, bool adjust) {
     if (cfg && cfg->variant != DSPMM_VARIANT_AUTO) return *cfg;
     const auto key = std::make_tuple((int)layout, nv, (int)bt);
     auto it = A->tuned.find(key);
@@ -1161,7 +1225,7 @@ dspmm_config resolve(dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_
         // ring picks carry over (the ring takes either, with the vector width
         // left to the operands)
         if (bt == DSPMM_R_32F) {
-            adjust_pick(A, nv, c);
+            if (adjust) adjust_pick(A, nv, c);
             return c;
         }
         if (c.variant == DSPMM_VARIANT_RING) {
@@ -1836,7 +1900,7 @@ dspmm_status_t dspmm_matrix_set_config(dspmm_matrix_t A, DenseLayout layout, int
                                        dspmm_dtype_t btype, const dspmm_config *cfg) {
     if (!A || !cfg || nv < 1 || (layout != DENSE_ROW_MAJOR && layout != DENSE_COL_MAJOR) ||
         (btype != DSPMM_R_32F && btype != DSPMM_R_16BF) || cfg->variant < DSPMM_VARIANT_AUTO ||
-        cfg->variant > DSPMM_VARIANT_RING)
+        cfg->variant > DSPMM_VARIANT_CSR_PARTS)
         return DSPMM_STATUS_INVALID_VALUE;
     std::lock_guard<std::mutex> lk(A->mu);
     const auto key = std::make_tuple((int)layout, nv, (int)btype);

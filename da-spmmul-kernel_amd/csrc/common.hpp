@@ -157,6 +157,32 @@ __device__ __forceinline__ void store_g(float *p, const float (&r)[VW]) {
     }
 }
 
+// Sums of rows in parts (CSR_PARTS): the products of nonzeros p .. p + 7 (< p1),
+// values in sv and rows of B in b, four FMAs to a part, the parts to two sums in turn.
+template <int VW>
+__device__ __forceinline__ void add_parts(float (&even)[VW], float (&odd)[VW], const float (&b)[8][VW],
+                                          const float *sv, int p, int p1) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        float part[VW];
+#pragma unroll
+        for (int k = 0; k < VW; k++) part[k] = 0.f;
+#pragma unroll
+        for (int u = 4 * h; u < 4 * h + 4; u++) {
+            if (p + u < p1) {
+                const float a = sv[p + u];
+#pragma unroll
+                for (int k = 0; k < VW; k++) part[k] = __builtin_fmaf(a, b[u][k], part[k]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < VW; k++) {
+            if (h == 0) even[k] += part[k];
+            else odd[k] += part[k];
+        }
+    }
+}
+
 // First column of a lane's VW columns.  Where fewer than VW are left of the
 // row (nv >= VW), the last ones of the row: the lane shares columns with its
 // neighbour and both write the same values.

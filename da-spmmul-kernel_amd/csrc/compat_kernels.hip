@@ -376,6 +376,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream(int nr, int nv, int64_t l
 // LDS broadcast within its group.  Overwrites every row (empty rows -> 0).
 // Rows far longer than the block's others are summed by the whole block, the
 // longest ones by blocks of their own at the front of the grid (LongRow).
+// PARTS: a row's sum in parts (add_parts), by its own group however long it is.
 // SLICED: a block whose rows overflow one window, and one of whose rows is
 // at least 4 shares of a window long (kWin / rows per block), splits each
 // window into one slice per row that still has nonzeros (kWin / n for n
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream(int nr, int nv, int64_t l
 // the whole window once the others are done.  Both forms add each row's
 // products in nonzero order.
 // ===========================================================================
-template <int VW, int L, bool SLICED>
+template <int VW, int L, bool SLICED, bool PARTS = false>
 __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_t ldb, int64_t ldc,
                                                            const int *__restrict__ rowPtr,
                                                            const int *__restrict__ colIdx,
@@ -438,8 +439,24 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
     auto apart = [&](int len) {
         return is_long_row(len, be - bs, rlast - r0) || len >= scout_row;
     };
+    float odd[VW];
+#pragma unroll
+    for (int k = 0; k < VW; k++) odd[k] = 0.f;
+    auto add = [&](int p0, int p1, int w) {
+        if constexpr (PARTS) {
+            for (int p = p0 - w; p < p1 - w; p += 8) {
+                float b8[8][VW];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    load_g<float, VW>(b8[u], B + (int64_t)s_col[min(p + u, p1 - w - 1)] * ldb + col0);
+                add_parts<VW>(acc, odd, b8, s_val, p, p1 - w);
+            }
+        } else {
+            seq_accumulate<float, VW, 4>(acc, p0, p1, w, s_col, s_val, B, ldb, col0);
+        }
+    };
     int nlong = 0;
-    if (be - bs >= kLongRow) {                 // the same in every thread
+    if (!PARTS && be - bs >= kLongRow) {                 // the same in every thread
         if (threadIdx.x == 0) s_nlong = 0;
         __syncthreads();
         if (threadIdx.x % L == 0 && apart(end - start)) s_long[atomicAdd(&s_nlong, 1)] = r;
@@ -484,7 +501,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
             stage_window(s_col, s_val, colIdx, values, w, cnt);
             __syncthreads();
             const int p0 = max(start, w), p1 = min(end, w + cnt);
-            if (colok) seq_accumulate<float, VW, 4>(acc, p0, p1, w, s_col, s_val, B, ldb, col0);
+            if (colok) add(p0, p1, w);
         }
     } else if constexpr (SLICED) {
         const int lane = (int)threadIdx.x % kWave, wv = (int)threadIdx.x / kWave;
@@ -524,11 +541,14 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
             }
             __syncthreads();
             if (colok && cnt > 0)
-                seq_accumulate<float, VW, 4>(acc, rank << lsl, (rank << lsl) + cnt, 0, s_col, s_val,
-                                             B, ldb, col0);
+                add(rank << lsl, (rank << lsl) + cnt, 0);
             done += cnt;
             __syncthreads();                              // before the next window's tables
         }
+    }
+    if constexpr (PARTS) {
+#pragma unroll
+        for (int k = 0; k < VW; k++) acc[k] += odd[k];
     }
     if (r < nr && colok && mine) store_g<true, VW>(C + (int64_t)r * ldc + col0, acc);
 }
@@ -1277,6 +1297,28 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
     return launch_status();
 }
 
+// Sums in parts, 5 to 32 columns (the native API's CSR_PARTS on FP32): rows of like
+// lengths, so without scouts.
+dspmm_status_t csr_parts_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
+                            const int *colIdx, const float *values, const float *B, float *C,
+                            hipStream_t st) {
+    const Slab s = make_slab(nv, 4);
+    if (nv < 5 || s.lanes > 8) return DSPMM_STATUS_NOT_SUPPORTED;
+    const bool sliced = (double)nnz / std::max(1, nr) * (kBlock / s.lanes) > kWin / 2;
+    with_lanes(s.lanes, [&](auto l_c) {
+        constexpr int L_ = decltype(l_c)::value;
+        if constexpr (L_ >= 2 && L_ <= 8) {
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(div_up(nr, kBlock / L_)), dim3(kBlock), 0, st, nr, nv, ldb,
+                                   ldc, rowPtr, colIdx, values, B, C, s.width, 0, INT_MAX);
+            };
+            if (sliced) launch(k_csr_scalar_rm<4, L_, true, true>);
+            else launch(k_csr_scalar_rm<4, L_, false, true>);
+        }
+    });
+    return launch_status();
+}
+
 template <int VW, int L, int GT>
 void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                           const int *colIdx, const float *values, const float *B, float *C,
@@ -1539,6 +1581,8 @@ dspmm_status_t launch_compat(int which, int nr, int nc, int nnz, int nv, int64_t
     case K_SPMV_CSR_SCALAR:
     case K_SPMM_CSR_SCALAR_ROW:
         return csr_scalar_rm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
+    case K_CSR_PARTS_ROW:
+        return csr_parts_rm(nr, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st);
     case K_SPMV_CSR_VECTOR:
     case K_SPMM_CSR_VECTOR_ROW:
         return csr_vector_rm(nr, nc, nnz, nv, ldb, ldc, rowPtr, colIdx, values, B, C, st, hint);

@@ -79,7 +79,8 @@ enum CompatKernel {
     K_SPMM_CSR_VECTOR_COL,
     K_SPMM_COO_SCALAR_COL,
     K_SPMM_COO_VECTOR_COL,
-    K_COUNT
+    K_COUNT,
+    K_CSR_PARTS_ROW          // the native API's: csr_scalar_row with sums in parts
 };
 
 }  // namespace dspmm

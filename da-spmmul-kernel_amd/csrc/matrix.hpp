@@ -113,6 +113,7 @@ struct dspmm_matrix_s {
     std::vector<float> h_values;
     int max_len = 0;
     double mean = 0, cv = 0;
+    bool clustered = false;     // most long rows (128 nonzeros, 4 times the mean) follow one another
     int64_t slots[6] = {0};     // carry slots of nnz tiles of 8, 16, ... 256 nonzeros
     size_t base_bytes = 0;
     std::mutex mu;
@@ -195,9 +196,9 @@ void complete_nb(dspmm_config &c, int nv, bool bf16);
 // The configuration a call runs: cfg unless AUTO, else the tuned one cached
 // for (layout, nv, bt), else (with `learned`, row-major only) the
 // nearest-neighbour selector's pick -- with BF16 B only a B-row ring pick --
-// else the static heuristic.
+// else the static heuristic.  `adjust` off leaves a pick as it was measured (adjust_pick).
 dspmm_config resolve(dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_t bt,
-                     const dspmm_config *cfg, bool learned = true);
+                     const dspmm_config *cfg, bool learned = true, bool adjust = true);
 // The static default (no timing, no corpus).
 dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspmm_dtype_t bt);
 // Nearest-neighbour selection over the measured corpus (selector.cpp).

@@ -89,6 +89,7 @@ struct RowSeqLaunch {
     int nr = 0, nv = 0;
     int vw = 1, lanes = 1, slab_w = 1, nslabs = 1, unroll = 4;
     bool sliced = false;               // per-row slices of the staging windows
+    bool parts = false;                // sums in parts (unroll 8)
     bool bf16 = false;
 };
 bool row_seq_unroll_ok(int u);

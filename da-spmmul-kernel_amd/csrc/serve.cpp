@@ -245,11 +245,14 @@ struct dspmm_server_s {
                           reinterpret_cast<const void *>(256), cfg.btype, fr.f, false,
                           carry_room(m, nv)) != DSPMM_STATUS_SUCCESS)
             return nullptr;
+        {
+            // the selector's pick: what a lone call adjusts it to sums rows in
+            // another order, and a lone request has the bits of one in company
+            std::lock_guard<std::mutex> lk(m.h->mu);
+            fr.own = resolve(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, nullptr, true, false);
+        }
         // (the workspace query builds the kernel's plan: only where it may run)
-        fr.own_ok = fr.f.nsplits == 0 &&
-                    dspmm_spmm_ex_resolve(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, nullptr, &fr.own) ==
-                        DSPMM_STATUS_SUCCESS &&
-                    row_exact(m.h, nv, fr.own) &&
+        fr.own_ok = fr.f.nsplits == 0 && row_exact(m.h, nv, fr.own) &&
                     dspmm_spmm_ex_workspace_size(m.h, DENSE_ROW_MAJOR, nv, cfg.btype, &fr.own,
                                                  &fr.own_ws) == DSPMM_STATUS_SUCCESS;
         // the own kernel's plan (a ring plan, say) built now, at admission,

@@ -292,7 +292,7 @@ typedef enum dspmm_variant {
                                     columns share once; rows are summed like
                                     the host loop (row-exact); unroll = B rows
                                     in flight (4 or 8) */
-    DSPMM_VARIANT_RING = 9       /* row-major, nv a multiple of 4 (FP32) or 8
+    DSPMM_VARIANT_RING = 9,      /* row-major, nv a multiple of 4 (FP32) or 8
                                     (BF16) fitting one slab: B rows staged in a
                                     ring in LDS whose fills and evictions a host
                                     plan decides; a workgroup walks tiles of
@@ -303,6 +303,11 @@ typedef enum dspmm_variant {
                                     workgroups per CU in the fewest whole
                                     rounds); rows are summed like the host
                                     loop (row-exact) */
+    DSPMM_VARIANT_CSR_PARTS = 10 /* row-major: the kernel of CSR_SCALAR with an
+                                    unroll (0 or 8 here), a row's nonzeros summed
+                                    four at a time, these in turn in two sums:
+                                    rounds long rows better than their order
+                                    does, and is not row-exact */
 } dspmm_variant_t;
 
 typedef struct dspmm_config {

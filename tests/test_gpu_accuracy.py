@@ -138,3 +138,85 @@ def test_spmv_band(n):
     assert ms["band"] <= 1.5 * ms["scattered"] + 0.002
     h.close()
     t.close()
+
+
+def chunks(a, b, S):
+    """Chunks of S nonzeros, each in order with a rounded product, added in order."""
+    s = np.zeros(np.broadcast_shapes(a.shape, b.shape)[:-1], F)
+    prod = a * b
+    for c in range(0, a.shape[-1], S):
+        t = np.zeros_like(s)
+        for i in range(c, min(c + S, a.shape[-1])):
+            t = t + prod[..., i]
+        s = s + t
+    return s
+
+
+@pytest.mark.parametrize("bf16,layout,n,nv,S", [
+    (True, "row", 20, 8, 16), (True, "row", 100, 2, 16), (True, "row", 100, 16, 32), (True, "row", 100, 48, 128),
+    (True, "col", 100, 32, 64), (True, "row", 200, 12, 32), (True, "row", 250, 64, 128),
+    (False, "col", 100, 16, 64), (False, "col", 200, 48, 256), (False, "col", 250, 12, 64)])
+def test_auto(bf16, layout, n, nv, S):
+    """AUTO rounds no worse than tiles of S nonzeros in order do, 16 per lane."""
+    cols = min(nv, 16)
+    m = Rows(4000, n, 3000, nv)
+    d_B = D.DeviceArray.from_numpy(m.B if layout == "row" else np.ascontiguousarray(m.B.T))
+    if bf16:
+        d_B = D.to_bf16_device(d_B)
+        m.B = (((m.B.view(np.uint32) + 0x7fff + ((m.B.view(np.uint32) >> 16) & 1)) >> 16) << 16).view(F)
+    a, b = m.operands(nv, cols)
+    exact = m.exact(a, b)
+    out = D.DeviceArray.from_numpy(np.full((m.nr, nv) if layout == "row" else (nv, m.nr), np.nan, F))
+    h = D.Matrix(m.nr, m.nc, m.ptr, m.col.reshape(-1), m.val.reshape(-1))
+    h.spmm(d_B, out, nv, D.DENSE_ROW_MAJOR if layout == "row" else D.DENSE_COL_MAJOR,
+           btype=D.DSPMM_R_16BF if bf16 else D.DSPMM_R_32F)
+    D.synchronize()
+    got = error((out.numpy() if layout == "row" else out.numpy().T)[:, :cols], exact)
+    ref = error(chunks(a, b, S), exact)
+    note(f"{'bf16' if bf16 else 'fp32'} {layout} rows of {n}, nv={nv}: {got:.3g}, tiles of {S} {ref:.3g}")
+    assert got <= MARGIN * ref
+    h.close()
+
+
+@pytest.mark.parametrize("nv", [3, 5, 8, 12, 16, 32])
+def test_auto_stencil(nv):
+    """A 27-point stencil on 48^3, FP32: AUTO against sums over 8 lanes."""
+    g = np.arange(48 ** 3).reshape(48, 48, 48)
+    d = np.array([(x * 48 + y) * 48 + z for x in (-1, 0, 1) for y in (-1, 0, 1) for z in (-1, 0, 1)])
+    col = (g[1:-1, 1:-1, 1:-1].reshape(-1, 1) + d).astype(np.int32)
+    nr, nc = col.shape[0], 48 ** 3
+    rng = np.random.default_rng(nv)
+    val = rng.standard_normal(col.shape).astype(F)
+    B = rng.uniform(-1, 1, (nc, nv)).astype(F)
+    ptr = (np.arange(nr + 1) * 27).astype(np.int32)
+    h = D.Matrix(nr, nc, ptr, col.reshape(-1), val.reshape(-1))
+    out = D.DeviceArray.from_numpy(np.full((nr, nv), np.nan, F))
+    h.spmm(D.DeviceArray.from_numpy(B), out, nv)
+    D.synchronize()
+    pick = np.arange(0, nr, 7)
+    a, b = val[pick][:, None, :], np.ascontiguousarray(B[:, :8][col[pick]].transpose(0, 2, 1))
+    exact = (a.astype(np.float64) * b).sum(-1)
+    # (four threads to a row of more than 16 columns: in order, as always)
+    ref = error(over_lanes(a, b, 8) if nv <= 16 else chunks(a, b, 27), exact)
+    got = error(out.numpy()[pick][:, :8], exact)
+    note(f"stencil, nv={nv}: {got:.3g}, over the lanes {ref:.3g}")
+    assert got <= MARGIN * ref
+    h.close()
+
+
+def test_auto_clustered_rows():
+    """Long rows side by side: AUTO's first call on a power law sorted by length
+    within twice its tiles' time."""
+    rng = np.random.default_rng(1)
+    lens = np.sort(np.minimum(4000, (3 / rng.random(60000) ** 0.7).astype(int)))[::-1].copy()
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    h = D.Matrix(60000, 60000, ptr, rng.integers(0, 60000, ptr[-1]).astype(np.int32),
+                 rng.standard_normal(ptr[-1]).astype(F))
+    for nv in (3, 8):
+        B, out = D.DeviceArray.from_numpy(rng.uniform(-1, 1, (60000, nv)).astype(F)), D.DeviceArray.zeros(60000 * nv)
+        tiles = D.make_config(D.VARIANT_NNZ_TILED)
+        ms = [min(h.benchmark(B, out, nv, config=c, warmup=5, reps=20, per_call=False)[0] for _ in range(3))
+              for c in (None, tiles)]
+        note(f"nv={nv}: AUTO {ms[0]:.4f} ms, tiles {ms[1]:.4f} ms")
+        assert ms[0] <= 2 * ms[1] + 0.002
+    h.close()
