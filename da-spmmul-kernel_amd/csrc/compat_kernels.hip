@@ -929,21 +929,26 @@ __global__ __launch_bounds__(kBlock) void k_coo_spmv(int nnz, const int *__restr
 #pragma unroll
     for (int u = 0; u < U; u++)
         if (key[u] != INT_MAX) v[u] *= x[(int64_t)c[u] * ldx];
+    float carry = 0.f;                         // of a row that goes on into this chunk
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int klast = read_lane(key[u], kWave - 1);
         const int before = __shfl_up(key[u], 1);
         const bool begins = ln > 0 && before != key[u];
-        const bool single = __ballot(begins) == 0;   // one row in the whole chunk
+        const uint64_t heads = __ballot(begins);
+        const bool single = heads == 0;        // one row in the whole chunk
         float s[1] = {v[u]};
         if (single) s[0] = butterfly_sum<1, kWave>(s[0]);
         else segmented_scan<1, 1>(s, segment_id(begins));
+        // added to the chunk's sum, not to its first product: rows of 64 and more
+        // round like chunks added one by one
+        if (u > 0 && (single || ln < __builtin_ctzll(heads))) s[0] += carry;
         int next = __shfl_down(key[u], 1);
         if (ln == kWave - 1) next = INT_MAX;
-        if (u + 1 < U) {                       // a row that goes on: its sum joins the next chunk
+        if (u + 1 < U) {                       // a row that goes on: its sum joins the next chunk's
             const int nk = read_lane(key[u + 1 < U ? u + 1 : u], 0);
             const float t = __shfl(s[0], kWave - 1);
-            if (nk == klast && ln == 0) v[u + 1 < U ? u + 1 : u] += t;
+            carry = nk == klast ? t : 0.f;
             if (ln == kWave - 1) next = nk;
         }
         if (key[u] != INT_MAX && next != key[u] &&

@@ -220,3 +220,41 @@ def test_auto_clustered_rows():
         note(f"nv={nv}: AUTO {ms[0]:.4f} ms, tiles {ms[1]:.4f} ms")
         assert ms[0] <= 2 * ms[1] + 0.002
     h.close()
+
+
+def scanned(prod, row, nr):
+    """Chunks of 64 products, each scanned by rows over 64 lanes (1, 2, 4, ...
+    apart), a row's chunks added in order."""
+    pad = -len(prod) % 64
+    s = np.concatenate([prod, np.zeros(pad, F)]).reshape(-1, 64)
+    key = np.concatenate([row, np.full(pad, nr)]).reshape(-1, 64)
+    d = 1
+    while d < 64:
+        t = s.copy()
+        t[:, d:] += np.where(key[:, d:] == key[:, :-d], s[:, :-d], F(0))
+        s, d = t, 2 * d
+    tail = np.concatenate([key[:, 1:] != key[:, :-1], np.ones((len(key), 1), bool)], 1)
+    y = np.zeros(nr + 1, F)
+    np.add.at(y, key[tail], s[tail])
+    return y[:nr]
+
+
+@pytest.mark.parametrize("fn", ["spmv_coo_scalar", "spmv_coo_vector"])
+@pytest.mark.parametrize("n", [20, 64, 100, 300])
+def test_spmv_coo(fn, n):
+    """A row that goes on in the next chunk adds to that chunk's sum."""
+    nr, nc = 2000000 // n, 3000
+    rng = np.random.default_rng(n)
+    row = np.repeat(np.arange(nr, dtype=np.int32), n)
+    col = rng.integers(0, nc, nr * n).astype(np.int32)
+    val, x = rng.standard_normal(nr * n).astype(F), rng.uniform(-1, 1, nc).astype(F)
+    exact = (val.astype(np.float64) * x[col]).reshape(nr, n).sum(1)
+    ptr = (np.arange(nr + 1) * n).astype(np.int32)
+    d = [D.DeviceArray.from_numpy(v) for v in (ptr, row, col, val, x)]
+    out = D.DeviceArray.zeros(nr)
+    st = D.launch(fn, nr, nc, nr * n, 1, *d, out)
+    assert st == 0, D.status_string(st)
+    D.synchronize()
+    got, ref = error(out.numpy(), exact), error(scanned(val * x[col], row, nr), exact)
+    note(f"{fn} rows of {n}: {got:.3g}, chunk by chunk {ref:.3g}")
+    assert got <= MARGIN * ref
