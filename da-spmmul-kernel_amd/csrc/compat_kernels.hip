@@ -1324,6 +1324,8 @@ dspmm_status_t csr_parts_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, c
     return launch_status();
 }
 
+constexpr int kVecFewWaves = 2048;     // of launch_csr_vector_rm: 8 per CU
+
 template <int VW, int L, int GT>
 void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                           const int *colIdx, const float *values, const float *B, float *C,
@@ -1338,7 +1340,10 @@ void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t 
         // Four gathers in flight where a group has that many to make: with a B
         // that the L2s hold, only rows of more than 7 nonzeros per group gain (16384
         // rows of 32, nv = 64: 15.7 -> 13.4 us; 64^3 stencil, nv = 32: 98.7 -> 83.7;
-        // 32^3 stencil, nv = 64, 6.3 per group: 15.0, with four 16.5).
+        // 32^3 stencil, nv = 64, 6.3 per group: 15.0, with four 16.5).  One lane to
+        // a row of B reaches a line per lane and gather, and enough wavefronts to hide
+        // them want one at a time (rows of 600, nv = 2: 4800 rows 11.1 with four, 6.9;
+        // rows of 1000: 2400 rows 7.8, 6.3; 1200 rows 5.2, 6.1).
         const double per = (double)nnz / ((double)GT * std::max(1, nr));
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, nr, nv, ldb, ldc, rowPtr, colIdx,
@@ -1346,7 +1351,7 @@ void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t 
         };
         if (parts)
             launch(k_csr_vector_rm<VW, L, GT, 4, true>);
-        else if (per > 7 || (per > 2.5 && (int64_t)nc * nv >= (4 << 20)))
+        else if ((per > 7 && (L > 1 || (int64_t)blocks * (kBlock / kWave) < kVecFewWaves)) || (per > 2.5 && (int64_t)nc * nv >= (4 << 20)))
             launch(k_csr_vector_rm<VW, L, GT, 4, false>);
         else
             launch(k_csr_vector_rm<VW, L, GT, 1, false>);

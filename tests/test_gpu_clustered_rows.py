@@ -61,3 +61,21 @@ def test_long_rows_side_by_side(kind):
             t0 = min(r.problem().benchmark(RM, nv, alg, 3, 10) for _ in range(3))
             note(f"{kind} {name} nv={nv}: {1e3 * t:.1f} us, spread {1e3 * t0:.1f} us")
             assert t < 5 * t0 + 0.02, f"{kind} {name} nv={nv}: {t} ms against {t0} ms"
+
+
+@pytest.mark.parametrize("nv", [2, 4])
+def test_uniformly_long_rows(nv):
+    """Rows past the length from which the vector kernel may gather four at a
+    time: above a launch's 3 us no more per nonzero than rows short of it."""
+    ms = []
+    rng = np.random.default_rng(7)
+    for n in (440, 800):
+        col = np.sort(rng.integers(0, 20000, (4800, n)), axis=1).reshape(-1)
+        c = Case(f"rows of {n}", 4800, 20000, np.arange(4801) * n, col, rng.standard_normal(col.size).astype(np.float32),
+                 4, B=rng.uniform(-1, 1, 20000 * 4).astype(np.float32))
+        c.fill_output(np.nan)
+        ms.append(min(c.problem().benchmark(RM, nv, D.ALG_CSR_VECTOR, 5, 30) for _ in range(5)))
+        h32, c64, ab = c.ref(RM, nv)
+        assert_fp32(c.output(nv), c64, ab, c.rowlen_flat(RM, nv), c.name, h32)
+    note(f"nv={nv}: rows of 440 {ms[0]:.4f} ms, of 800 {ms[1]:.4f} ms")
+    assert ms[1] <= 1.05 * (0.003 + (ms[0] - 0.003) * 800 / 440)
