@@ -206,7 +206,7 @@ template <typename T>
 dspmm_status_t to_device(T **dst, const std::vector<T> &src) {
     *dst = nullptr;
     if (src.empty()) return DSPMM_STATUS_SUCCESS;
-    dspmm_status_t s = hip_status(hipMalloc((void **)dst, sizeof(T) * src.size()));
+    dspmm_status_t s = device_malloc((void **)dst, sizeof(T) * src.size());
     if (s != DSPMM_STATUS_SUCCESS) return s;
     return hip_status(hipMemcpy(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice));
 }
@@ -278,7 +278,7 @@ dspmm_status_t dspmm_batch_create(dspmm_batch_t *out, const dspmm_batch_item *it
     auto alloc_carry = [&]() -> dspmm_status_t {
         b->carry_bytes = sizeof(float) * (size_t)b->sch.carry_floats;
         if (b->carry_bytes == 0) return DSPMM_STATUS_SUCCESS;
-        return hip_status(hipMalloc((void **)&b->carry, b->carry_bytes));
+        return device_malloc((void **)&b->carry, b->carry_bytes);
     };
     st = alloc_carry();
     if (st == DSPMM_STATUS_ALLOC_FAILED) {         // the longest tiles have the fewest carries

@@ -60,8 +60,8 @@ bool is_col(int which) {
 //     back behind them, so that streams and threads never share one.  That
 //     costs a call 18 us, mostly the marker behind its work.
 // Free blocks beyond kScratchKept go back to the device at the next
-// synchronisation; dspmm_release_scratch, and dspmm_device_alloc where it finds
-// the memory short, give back the rest.
+// synchronisation; dspmm_release_scratch, and every allocation of the library that
+// finds the memory short (device_malloc), give back the rest.
 constexpr size_t kScratchCall = (size_t)256 << 20;   // the most that one call takes
 constexpr size_t kScratchKept = kScratchCall;
 constexpr size_t kScratchPool = 4 * kScratchCall;
@@ -260,6 +260,16 @@ int select_kernel(SPMV_SPMM_ALG alg, DenseLayout layout, int nv) {
 }
 
 }  // namespace
+
+dspmm_status_t device_malloc(void **ptr, size_t bytes) {
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory && release_scratch() == DSPMM_STATUS_SUCCESS) {
+        (void)hipGetLastError();
+        e = hipMalloc(ptr, bytes);
+    }
+    return hip_status(e);
+}
+
 }  // namespace dspmm
 
 using namespace dspmm;
@@ -325,12 +335,7 @@ dspmm_status_t dspmm_device_alloc(void **ptr, size_t bytes) {
     if (!ptr) return DSPMM_STATUS_INVALID_VALUE;
     *ptr = nullptr;
     if (bytes == 0) return DSPMM_STATUS_SUCCESS;
-    hipError_t e = hipMalloc(ptr, bytes);
-    if (e == hipErrorOutOfMemory && release_scratch() == DSPMM_STATUS_SUCCESS) {
-        (void)hipGetLastError();
-        e = hipMalloc(ptr, bytes);
-    }
-    return hip_status(e);
+    return device_malloc(ptr, bytes);
 }
 
 dspmm_status_t dspmm_release_scratch(void) { return release_scratch(); }

@@ -110,7 +110,7 @@ template <typename T>
 dspmm_status_t upload(T **dst, const T *src, size_t n, hipMemcpyKind kind, hipStream_t st) {
     *dst = nullptr;
     if (n == 0) return DSPMM_STATUS_SUCCESS;
-    dspmm_status_t s = hip_status(hipMalloc((void **)dst, n * sizeof(T)));
+    dspmm_status_t s = device_malloc((void **)dst, n * sizeof(T));
     if (s != DSPMM_STATUS_SUCCESS) return s;
     if (kind == hipMemcpyHostToDevice) return hip_status(hipMemcpy(*dst, src, n * sizeof(T), kind));
     return hip_status(hipMemcpyAsync(*dst, src, n * sizeof(T), kind, st));
@@ -334,7 +334,7 @@ dspmm_status_t get_diag_plan(dspmm_matrix_s *A, DiagPlan **out, bool build) {
             head.resize((size_t)kDiagMax, INT_MAX);
             head.insert(head.end(), p.h_off.begin(), p.h_off.end());
             p.bytes = diag_bytes(A);
-            dspmm_status_t s = hip_status(hipMalloc(&p.d_mem, p.bytes));
+            dspmm_status_t s = device_malloc((void **)&p.d_mem, p.bytes);
             if (s == DSPMM_STATUS_SUCCESS) {
                 p.d_vals = reinterpret_cast<float4 *>(p.d_mem);
                 p.d_didx = reinterpret_cast<uint32_t *>(p.d_vals + cells);
@@ -823,7 +823,7 @@ dspmm_status_t handle_buffer(void **buf, size_t *have, size_t need, RunMode mode
     (void)hipFree(*buf);
     *buf = nullptr;
     *have = 0;
-    dspmm_status_t s = hip_status(hipMalloc(buf, need));
+    dspmm_status_t s = device_malloc(buf, need);
     if (s != DSPMM_STATUS_SUCCESS) return s;
     *have = need;
     *out = *buf;

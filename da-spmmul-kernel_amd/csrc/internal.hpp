@@ -11,6 +11,10 @@ namespace dspmm {
 // Records `e` as this thread's last HIP error and maps it to a status.
 dspmm_status_t hip_status(hipError_t e);
 // Status of the most recent launch on this thread.
+// hipMalloc, which where it finds the memory short gives back the free scratch of
+// column-major products first.
+dspmm_status_t device_malloc(void **ptr, size_t bytes);
+
 inline dspmm_status_t launch_status() { return hip_status(hipGetLastError()); }
 
 inline hipStream_t as_hip(dspmm_stream_t s) { return reinterpret_cast<hipStream_t>(s); }

@@ -55,7 +55,7 @@ class Arena {
     dspmm_status_t init(size_t bytes) {
         const size_t size = round_up(bytes, 256);
         if (size == 0) return DSPMM_STATUS_SUCCESS;
-        dspmm_status_t s = hip_status(hipMalloc((void **)&base_, size));
+        dspmm_status_t s = device_malloc((void **)&base_, size);
         if (s == DSPMM_STATUS_SUCCESS) ff_.reset(size);
         return s;
     }
@@ -577,7 +577,7 @@ dspmm_status_t dspmm_server_create(dspmm_server_t *out, const dspmm_server_confi
         const size_t bi = sizeof(ItemDesc) * (size_t)items_cap, bs = sizeof(int4) * (size_t)s->seg_cap,
                      bx = sizeof(int) * (2 * kNumXcd + 1), bp = sizeof(int) * ((size_t)items_cap + 1);
         sl.stage_bytes = round_up(bi, 256) + round_up(bs, 256) + round_up(bx, 256) + bp;
-        if (st == DSPMM_STATUS_SUCCESS) st = hip_status(hipMalloc((void **)&sl.d_sched, sl.stage_bytes));
+        if (st == DSPMM_STATUS_SUCCESS) st = device_malloc((void **)&sl.d_sched, sl.stage_bytes);
         if (st == DSPMM_STATUS_SUCCESS) st = hip_status(hipHostMalloc((void **)&sl.h_stage, sl.stage_bytes));
     }
     if (st != DSPMM_STATUS_SUCCESS) {

@@ -14,7 +14,7 @@
  *     with ld = nc (input) and ld = nr (output);
  *   - all pointers are caller-owned device memory; launchers are
  *     asynchronous on `stream`.  They allocate nothing, except that a
- *     column-major SpMM of some size takes up to 256 MiB of scratch in stream
+ *     column-major SpMM of some size takes up to 256 MiB of scratch a call in stream
  *     order (dspmm_release_scratch); where there is none, and on a stream that
  *     is being captured, it runs without.
  * Output semantics (spmvspmm_benchmark.cu:141-157):
@@ -142,7 +142,9 @@ DSPMM_API dspmm_status_t dspmm_spmm(SPMV_SPMM_ALG alg, DenseLayout layout,
 DSPMM_API dspmm_status_t dspmm_device_alloc(void **ptr, size_t bytes);
 DSPMM_API dspmm_status_t dspmm_device_free(void *ptr);
 /* Gives back the scratch that column-major SpMMs keep on the current device
- * between calls (at most 256 MiB).  Waits for the default stream. */
+ * between calls (the default stream's block and as much free for the others, at
+ * most 256 MiB each).  Waits for the default stream.  Allocations of this
+ * library that find the memory short do so by themselves. */
 DSPMM_API dspmm_status_t dspmm_release_scratch(void);
 /* Synchronous copies (like CUArray::sync_device / sync_host). */
 DSPMM_API dspmm_status_t dspmm_memcpy_h2d(void *dst, const void *src, size_t bytes);

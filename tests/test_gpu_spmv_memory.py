@@ -84,3 +84,42 @@ def test_autotuner_without_diagonals():
     table = m.autotune_table(d_x, d_y, 1, reps=1)
     assert sorted(c.tile_nnz for c, _ in table if c.variant == D.VARIANT_SPMV_TILED) == [512, 1024, 2048, 4096]
     m.close()
+
+
+def test_a_matrix_takes_the_scratch_back():
+    """Column-major products keep scratch; a matrix that needs the memory gets it."""
+    a, w = W.c3_matrix(90), W.gen_csr(W.GEN_FIXED, 300000, 300000, seed=2, p0=4)
+    nv = 64
+    d = [D.DeviceArray.from_numpy(v) for v in (w.rowPtr, np.zeros(1, np.int32), w.colIdx, w.values)]
+    B, out = D.DeviceArray.zeros(w.nc * nv), D.DeviceArray.zeros(w.nr * nv)
+    assert D.lib().dspmm_release_scratch() == 0
+    D.synchronize()
+    free = D.device_info()["free_mem"]
+    assert D.launch("spmm_csr_scalar_col", w.nr, w.nc, w.nnz, nv, *d, B, out) == 0
+    D.synchronize()
+    kept = free - D.device_info()["free_mem"]
+    assert kept >= 128 << 20
+    x = np.random.default_rng(1).uniform(-1, 1, a.nc).astype(np.float32)
+    d_x, d_y = D.DeviceArray.from_numpy(x), D.DeviceArray.from_numpy(np.full(a.nr, np.nan, np.float32))
+    taken = []
+    try:
+        step = 64 << 30
+        while step >= 16 << 20:
+            if D.device_info()["free_mem"] < LEFT + step:
+                step //= 2
+                continue
+            taken.append(D.DeviceArray(step, np.uint8, (step,)))
+        left = D.device_info()["free_mem"]
+        note(f"scratch {kept >> 20} MiB, free {left >> 20} MiB, matrix {8 * a.nnz >> 20} MiB")
+        assert left < 8 * a.nnz
+        m = D.Matrix(a.nr, a.nc, a.rowPtr, a.colIdx, a.values)
+        m.spmm(d_x, d_y, 1, config=D.make_config(D.VARIANT_SPMV_TILED, tile_nnz=1024))
+        D.synchronize()
+        m.close()
+    finally:
+        for t in taken:
+            t.free()
+    h32 = O.spmm_host32(RM, a.nr, a.nc, 1, a.rowPtr, a.colIdx, a.values, x).reshape(-1)
+    c64, ab = O.spmm_fp64(RM, a.nr, a.nc, 1, a.rowPtr, a.colIdx, a.values, x)
+    assert_fp32(d_y.numpy(), c64.reshape(-1), ab.reshape(-1), np.diff(a.rowPtr).astype(np.float64),
+                "tiles", h32)
