@@ -36,7 +36,7 @@ __device__ __forceinline__ void seq_accumulate(float (&acc)[VW], int p0, int p1,
                                                const TB *__restrict__ B, int64_t ldb,
                                                int col0) {
     int p = p0;
-    for (; p + UNR <= p1; p += UNR) {
+    for (; p1 - p >= UNR; p += UNR) {
         float b[UNR][VW];
 #pragma unroll
         for (int u = 0; u < UNR; u++)
@@ -130,8 +130,8 @@ __device__ __forceinline__ bool is_long_row(int len, int block_nnz, int block_ro
 // groups multiply P nonzeros into LDS (P products of L * VW columns, two
 // steps' gathers in flight) and thread t < L * VW adds column t's products in
 // order; the (column, value) pairs go through LDS in chunks, loaded a chunk
-// ahead.  `base` is the first of the L * VW columns.  Returns column t's sum.  Every thread calls it (barriers
-// inside).
+// ahead.  `base` is the first of the L * VW columns.  Returns column t's sum.
+// Every thread calls it (barriers inside).
 template <int VW, int L, int U>
 struct LongRow {
     static constexpr int W = L * VW;
@@ -205,7 +205,7 @@ struct LongRow {
             __syncthreads();
             const int m = min(P, n - k * P);
             if (t < W) {                       // H products read ahead of the H being added
-                                constexpr int H = 8;
+                constexpr int H = 8;
                 const float *pr = prod + t;
                 float x[H], y[H];
 #pragma unroll
@@ -245,10 +245,10 @@ struct LongRow {
 
 // ===========================================================================
 // Row-balanced, sequential reduction, row-major, for few columns
-// (spmv_csr_scalar; spmm_csr_scalar_row with L * VW <= 8 and few
-// rows, or with 4).  A wavefront owns
-// G consecutive rows, at most 64 / (L * VW).  In windows of PW of their pairs,
-// every lane gathers B for its share of the window at once, the next window's
+// (spmv_csr_scalar; spmm_csr_scalar_row with L * VW <= 8 and few rows, or with
+// 4).  A wavefront owns G consecutive rows, at most 64 / (L * VW).  In windows
+// of PW of their pairs (counted from the window's start: nnz may be close to
+// INT_MAX), every lane gathers B for its share of the window at once, the next window's
 // while this one is added, and the products go to the wavefront's LDS region,
 // one column after another; then lane (row, column) adds its row's products
 // in nonzero order.  However long a row is, all 64 lanes gather for it.
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream(int nr, int nv, int64_t l
     auto gather = [&](int w) {
 #pragma unroll
         for (int k = 0; k < E; k++) {
-            const int p = min(w + ln / L + k * (kWave / L), e1 - 1);
+            const int p = w + min(ln / L + k * (kWave / L), e1 - 1 - w);
             cc[k] = colIdx[p];
             vv[k] = values[p];
         }
@@ -305,19 +305,20 @@ __global__ __launch_bounds__(kBlock) void k_csr_stream(int nr, int nv, int64_t l
     };
     float acc = 0.f;
     if (e0 < e1) gather(e0);
-    for (int w = e0; w < e1; w += PW) {
+    for (int w = e0; w < e1; w = e1 - w > PW ? w + PW : e1) {
+        const int left = e1 - w;
         wave_lds_sync();                       // the last window's products have been read
 #pragma unroll
         for (int k = 0; k < E; k++) {
             const int i = ln / L + k * (kWave / L);
 #pragma unroll
             for (int q = 0; q < VW; q++)       // +0 past the end: a sum that began at +0 keeps its bits
-                sp[(gl + q) * LD + i] = w + i < e1 ? vv[k] * b[k][q] : 0.f;
+                sp[(gl + q) * LD + i] = i < left ? vv[k] * b[k][q] : 0.f;
         }
-        if (w + PW < e1) gather(w + PW);
+        if (left > PW) gather(w + PW);
         wave_lds_sync();
         const int p0 = max(start, w) - w;
-        int n = min(end, w + PW) - w - p0;
+        int n = min(end - w, PW) - p0;
         // Long rows (of this window): 64 products at a time in the lanes of one
         // register per column, and each lane adds its product to the sum that
         // its lower neighbour hands up: 63 steps put the row's sum in order in
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
         }
     }
     if (!slice) {
-        for (int w = bs; w < be; w += kWin) {
+        for (int w = bs; w < be; w = be - w > kWin ? w + kWin : be) {
             for (int i = 0; i < nlong; i++) {  // no window starts inside a row that is done
                 const int q = s_long[i];
                 if (w >= rowPtr[q] && w < rowPtr[q + 1]) { w = rowPtr[q + 1]; i = -1; }
@@ -584,7 +585,7 @@ __device__ __forceinline__ void strided_accumulate(float (&acc)[VW], int p0, int
                                                    const float *__restrict__ values,
                                                    const float *__restrict__ Bc, int64_t ldb) {
     if constexpr (U == 1) {
-        for (int p = p0; p < e; p += stride) {
+        for (unsigned p = p0; p < (unsigned)e; p += stride) {
             const int c = colIdx[p];
             const float a = values[p];
             float b[VW];
@@ -987,7 +988,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_cm(int nr, int nv, int64_
 #pragma unroll
     for (int t = 0; t < T; t++) acc[t] = 0.f;
     const float *Bj = B + (int64_t)j0 * ldb;
-    for (int w = bs; w < be; w += kWin) {
+    for (int w = bs; w < be; w = be - w > kWin ? w + kWin : be) {
         const int cnt = min(kWin, be - w);
         __syncthreads();
         stage_window(s_col, s_val, colIdx, values, w, cnt);
@@ -1032,7 +1033,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_vector_cm(int nr, int nv, int64_
     int s = 0, e = 0;
     if (r < nr) { s = rowPtr[r]; e = rowPtr[r + 1]; }
     auto add = [&](int p0, int pe, int stride) {
-        for (int p = p0; p < pe; p += stride) {
+        for (unsigned p = p0; p < (unsigned)pe; p += stride) {
             const int c = colIdx[p];
             const float a = values[p];
 #pragma unroll

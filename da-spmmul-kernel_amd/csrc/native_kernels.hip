@@ -1202,7 +1202,7 @@ __global__ __launch_bounds__(kBlock) void k_row_seq(RowSeqLaunch g, int lg) {
         // pass each (a single window when they fit)
         int *sc = s_col[wv];
         float *sv = s_val[wv];
-        for (int w = e0; w < e1; w += kRsWin) {
+        for (int w = e0; w < e1; w = e1 - w > kRsWin ? w + kRsWin : e1) {
             const int cnt = min(kRsWin, e1 - w);
             wave_lds_sync();
             for (int i = lane; i < cnt; i += kWave) {
