@@ -78,12 +78,6 @@ __device__ __forceinline__ void store_vec_nt(float *p, const float (&r)[VW]) {
     }
 }
 
-template <int VW>
-__device__ __forceinline__ void atomic_add_vec(float *p, const float (&r)[VW]) {
-#pragma unroll
-    for (int k = 0; k < VW; k++) unsafeAtomicAdd(p + k, r[k]);
-}
-
 // ---- dense BF16 vectors along N (FP32 widening is a 16-bit shift) -------
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }

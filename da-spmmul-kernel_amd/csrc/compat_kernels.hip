@@ -1259,6 +1259,10 @@ int stream_rows(int W, int nnz, int nr) {
 // 9.9 / 8.7, 100000 of 20 12.4 / 12.5; power law of 60916 27 / 42, 16384 rows of 32 6.2 / 14.8.
 constexpr int kGroupRows8 = 98304;
 
+// The slabs that make_slab gives to vectors as wide as the columns allow.
+template <int VW, int L>
+constexpr bool kSlabShape = VW == 4 || (VW == 2 && L <= 2) || (VW == 1 && L == 1);
+
 dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                              const int *colIdx, const float *values, const float *B, float *C,
                              hipStream_t st) {
@@ -1267,7 +1271,7 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
         with_vw(s.vw, [&](auto vw_c) {
             with_lanes(s.lanes, [&](auto l_c) {
                 constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-                if constexpr (VW_ * L_ <= 8) {
+                if constexpr (VW_ * L_ <= 8 && kSlabShape<VW_, L_>) {
                     const int g = stream_rows(VW_ * L_, nnz, nr);
                     hipLaunchKernelGGL((k_csr_stream<VW_, L_, false>), dim3(div_up(nr, (int64_t)g * (kBlock / kWave))),
                                        dim3(kBlock), 0, st, nr, nv, ldb, ldc, rowPtr, colIdx, values,
@@ -1284,7 +1288,7 @@ dspmm_status_t csr_scalar_rm(int nr, int nnz, int nv, int64_t ldb, int64_t ldc, 
     with_vw(s.vw, [&](auto vw_c) {
         with_lanes(s.lanes, [&](auto l_c) {
             constexpr int VW_ = decltype(vw_c)::value, L_ = decltype(l_c)::value;
-            if constexpr (VW_ * L_ >= 8) {
+            if constexpr (VW_ * L_ >= 8 && kSlabShape<VW_, L_>) {
                 const int blocks = div_up(nr, kBlock / L_);
                 const int64_t others = (int64_t)blocks * s.count;
                 const Scouts sc = scouts_for(nr, nnz, nv, s.width, kScoutRow, others, others < kScoutBlocks);
@@ -1331,7 +1335,7 @@ template <int VW, int L, int GT>
 void launch_csr_vector_rm(int nr, int nc, int nnz, int nv, int64_t ldb, int64_t ldc, const int *rowPtr,
                           const int *colIdx, const float *values, const float *B, float *C,
                           hipStream_t st, const Slab &s, bool parts) {
-    if constexpr (GT * L <= kWave) {
+    if constexpr (GT * L <= kWave && kSlabShape<VW, L>) {
         // Scouts where a long row's wavefront would set the kernel's time.
         Scouts sc;
         const int blocks = div_up(nr, kBlock / (GT * L));
