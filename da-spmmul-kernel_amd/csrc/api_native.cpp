@@ -552,14 +552,16 @@ bool longer_tiles(int nv, bool bf16, dspmm_config &c) {
     }
     return true;
 }
-// Longer tiles while the carries of split rows exceed what dspmm_spmm_ex_noalloc
-// has for them (and the handle would keep).  Power law, BF16 B, 262144 rows, nv = 256:
-// 64 per tile 79 MB of carries, 128 39 MB; 1000000 rows, nv = 128: 64 per tile 150 MB, 256 38.
-void fit_carries(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, dspmm_config &c) {
-    const size_t copies = rm ? 0 : transposed_bytes(A, nv, bf16);
-    const size_t most = DSPMM_NOALLOC_SCRATCH_BYTES;
-    const size_t left = copies < most ? most - copies : most;
-    while (carry_bytes(A, c.tile_nnz, nv) > left && longer_tiles(nv, bf16, c)) {}
+// AUTO's tiles within dspmm_spmm_ex_noalloc's scratch: grown, where they need
+// more, until their carries (and the transposed copies) fit.
+dspmm_config noalloc_tiles(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, dspmm_config c) {
+    if (c.variant != DSPMM_VARIANT_NNZ_TILED) return c;
+    complete_nb(c, nv, bf16);
+    const size_t copies = rm || nv == 1 ? 0 : transposed_bytes(A, nv, bf16);
+    const dspmm_config as_is = c;
+    while (copies + carry_bytes(A, c.tile_nnz, nv) > DSPMM_NOALLOC_SCRATCH_BYTES)
+        if (!longer_tiles(nv, bf16, c)) return as_is;
+    return c;
 }
 // Halves the tile until the launch's LDS fits.
 void fit_tile(int nv, bool bf16, dspmm_config &c) {
@@ -580,7 +582,7 @@ int64_t tile_chain(int64_t n, int S, int nv) {
     const int64_t parts = 64 / std::min(64, pow2_ceil(nv)), chunks = (n + S - 1) / S;
     return S + (chunks + parts - 1) / parts + parts;
 }
-void single_tile(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, int cap, dspmm_config &c) {
+void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
     const int64_t slabs = div_up(nv, full.vec * full.lanes), g = 64 / full.lanes;
@@ -598,7 +600,6 @@ void single_tile(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, int cap, d
            tile_chain(A->max_len, c.tile_nnz, nv) > 4 * tile_chain(A->max_len, plain, nv))
         c.tile_nnz *= 2;
     fit_tile(nv, bf16, c);
-    fit_carries(A, rm, nv, bf16, c);
 }
 
 // A lane group per row, for rows of like lengths: no tiles, no split rows.  False
@@ -712,7 +713,7 @@ dspmm_config heuristic(const dspmm_matrix_s *A, DenseLayout layout, int nv, dspm
         cap = std::min(plain_tile(nv, bf16), 128);
         if (nv > 32) c.unroll = 8;             // (4096 rows of 2000, FP32, nv = 128: 79 / 92 in fours)
     }
-    single_tile(A, rm, nv, bf16, cap, c);
+    single_tile(A, nv, bf16, cap, c);
     return c;
 }
 
@@ -1431,17 +1432,28 @@ dspmm_status_t dspmm_matrix_prepare(dspmm_matrix_t A, DenseLayout layout, int nv
     if (auto_cfg && !A->tuned.count(key)) A->prepared[key] = c;
     const RunMode mode = (flags & DSPMM_PREPARE_HANDLE_BUFFERS) ? kRunPrepare : kRunPlans;
     float *Cw = const_cast<float *>(C);
+    // the no-alloc call's own tiles, where they are others
+    auto noalloc_plan = [&](const dspmm_config &k) {
+        const bool bf16 = btype == DSPMM_R_16BF;
+        dspmm_config full = k;
+        complete_nb(full, nv, bf16);
+        const dspmm_config n = noalloc_tiles(A, layout == DENSE_ROW_MAJOR, nv, bf16, k);
+        if (k.variant == DSPMM_VARIANT_NNZ_TILED && n.tile_nnz != full.tile_nnz)
+            st = run_ex(A, layout, nv, B, ldb, btype, Cw, ldc, n, nullptr, 0, nullptr, nullptr, kRunPlans);
+    };
     st = run_ex(A, layout, nv, B, ldb, btype, Cw, ldc, c, nullptr, 0, nullptr, nullptr, mode);
     if (auto_cfg && (st != DSPMM_STATUS_SUCCESS || c.variant == DSPMM_VARIANT_NNZ_CACHED ||
                      c.variant == DSPMM_VARIANT_RING)) {
         // the static default AUTO falls back to when the pick cannot run: the
         // kernels that stage B in LDS refuse operands by their alignment, the
         // others take any once they take these sizes
-        const dspmm_status_t sh = run_ex(A, layout, nv, B, ldb, btype, Cw, ldc,
-                                         heuristic(A, layout, nv, btype), nullptr, 0, nullptr,
+        const dspmm_config h = heuristic(A, layout, nv, btype);
+        const dspmm_status_t sh = run_ex(A, layout, nv, B, ldb, btype, Cw, ldc, h, nullptr, 0, nullptr,
                                          nullptr, mode);
+        if (sh == DSPMM_STATUS_SUCCESS) noalloc_plan(h);
         if (st == DSPMM_STATUS_NOT_SUPPORTED) st = sh;
     }
+    if (auto_cfg && st == DSPMM_STATUS_SUCCESS && !A->tuned.count(key)) noalloc_plan(c);
     return st;
 }
 
@@ -1500,11 +1512,19 @@ dspmm_status_t dspmm_spmm_ex(dspmm_matrix_t A, DenseLayout layout, int nv, const
     auto run = [&](const dspmm_config &rc) -> dspmm_status_t {
         dspmm_status_t s = run_ex(A, layout, nv, B, ldb, btype, C, ldc, rc, workspace, workspace_bytes,
                                   as_hip(stream));
-        if (s != DSPMM_STATUS_WORKSPACE_TOO_SMALL || !workspace || !auto_cfg || tuned ||
-            rc.variant != DSPMM_VARIANT_NNZ_TILED)
+        if (s != (workspace ? DSPMM_STATUS_WORKSPACE_TOO_SMALL : DSPMM_STATUS_ALLOC_FAILED) || !auto_cfg ||
+            tuned || rc.variant != DSPMM_VARIANT_NNZ_TILED)
             return s;
         // AUTO's own tiles: longer ones need fewer carries
         const bool bf16 = btype == DSPMM_R_16BF;
+        if (!workspace) {
+            dspmm_config l = rc;
+            while (s == DSPMM_STATUS_ALLOC_FAILED && longer_tiles(nv, bf16, l)) {
+                (void)hipGetLastError();
+                s = run_ex(A, layout, nv, B, ldb, btype, C, ldc, l, nullptr, 0, as_hip(stream));
+            }
+            return s;
+        }
         const size_t copies = layout == DENSE_COL_MAJOR && nv > 1 ? transposed_bytes(A, nv, bf16) : 0;
         dspmm_config l = rc;
         while (longer_tiles(nv, bf16, l))
@@ -1531,6 +1551,7 @@ dspmm_status_t dspmm_spmm_ex_noalloc(dspmm_matrix_t A, DenseLayout layout, int n
     if (st != DSPMM_STATUS_SUCCESS) return st;
     std::lock_guard<std::mutex> lk(A->mu);
     const bool auto_cfg = !cfg || cfg->variant == DSPMM_VARIANT_AUTO;
+    bool own_tiles = false;
     dspmm_config c{};
     if (auto_cfg) {
         // only a configuration already resolved (tuned, or picked by
@@ -1543,15 +1564,19 @@ dspmm_status_t dspmm_spmm_ex_noalloc(dspmm_matrix_t A, DenseLayout layout, int n
             auto ip = A->prepared.find(key);
             if (ip == A->prepared.end()) return DSPMM_STATUS_NOT_PREPARED;
             c = ip->second;
+            own_tiles = true;
         }
     } else {
         c = *cfg;
     }
     const hipStream_t hs = as_hip(stream);
+    const bool rm = layout == DENSE_ROW_MAJOR, bf16 = btype == DSPMM_R_16BF;
+    if (own_tiles) c = noalloc_tiles(A, rm, nv, bf16, c);
     st = run_ex(A, layout, nv, B, ldb, btype, C, ldc, c, ws, DSPMM_NOALLOC_SCRATCH_BYTES, hs,
                 nullptr, kRunNoAlloc);
     if (st == DSPMM_STATUS_NOT_SUPPORTED && auto_cfg)
-        st = run_ex(A, layout, nv, B, ldb, btype, C, ldc, heuristic(A, layout, nv, btype), ws,
+        st = run_ex(A, layout, nv, B, ldb, btype, C, ldc,
+                    noalloc_tiles(A, rm, nv, bf16, heuristic(A, layout, nv, btype)), ws,
                     DSPMM_NOALLOC_SCRATCH_BYTES, hs, nullptr, kRunNoAlloc);
     return st;
 }

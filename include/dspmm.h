@@ -353,7 +353,8 @@ DSPMM_API dspmm_status_t dspmm_spmm_ex(dspmm_matrix_t A, DenseLayout layout, int
  * AUTO's pick must already exist: call dspmm_matrix_prepare with the same
  * arguments first (else DSPMM_STATUS_NOT_PREPARED).  A call whose scratch
  * would exceed DSPMM_NOALLOC_SCRATCH_BYTES returns
- * DSPMM_STATUS_WORKSPACE_TOO_SMALL.  Every call on one GPU shares that
+ * DSPMM_STATUS_WORKSPACE_TOO_SMALL; before that, AUTO's nnz tiles grow, which
+ * leaves fewer split rows than dspmm_spmm_ex's have.  Every call on one GPU shares that
  * GPU's array (each call writes what it reads): calls that overlap in time
  * on one GPU race and must be serialised by the caller. */
 #define DSPMM_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
@@ -370,8 +371,10 @@ DSPMM_API dspmm_status_t dspmm_spmm_ex_workspace_size(dspmm_matrix_t A, DenseLay
                                                       size_t *bytes);
 /* Builds everything a later dspmm_spmm_ex call with these arguments needs
  * -- the tile plan of the configuration it resolves to and, for AUTO, the
- * plan of the static default it falls back to; the row array of the COO
- * classes -- and fixes AUTO's pick for (layout, nv, btype).  With
+ * plans of dspmm_spmm_ex_noalloc's longer tiles, where it takes them, and of
+ * the static default, where the pick is NNZ_CACHED or RING (which refuse some
+ * operands) or did not run; the row array of the COO classes -- and fixes
+ * AUTO's pick for (layout, nv, btype).  With
  * DSPMM_PREPARE_HANDLE_BUFFERS it also sizes the handle's own split-row and
  * transposed-copy buffers, for calls that pass no workspace.  Afterwards
  * such a call allocates nothing, copies nothing to the host and never

@@ -100,3 +100,20 @@ def test_small_arena(alone, nv, btype):
     h32 = O.spmm_host32(RM, a.nr, a.nc, nv, a.rowPtr, a.colIdx, a.values, Br).reshape(-1)
     c64, ab = O.spmm_fp64(RM, a.nr, a.nc, nv, a.rowPtr, a.colIdx, a.values, Br)
     assert_fp32(got[0], c64.reshape(-1), ab.reshape(-1), np.repeat(lens.astype(np.float64), nv), "served", h32)
+
+
+def test_auto_keeps_short_tiles():
+    """What no-alloc calls have for carries does not bound AUTO's: a product with
+    room is no slower than with the tile of 16 nonzeros per lane."""
+    a = W.gen_csr(W.GEN_ZIPF, 1000000, 1000000, 29, 1.6, 4, 2000, W.VAL_NORMAL)
+    m = D.Matrix(a.nr, a.nc, a.rowPtr, a.colIdx, a.values)
+    nv, bt = 64, D.DSPMM_R_16BF
+    d_B = D.to_bf16_device(D.DeviceArray.from_numpy(
+        np.random.default_rng(4).uniform(-1, 1, (a.nc, nv)).astype(np.float32)))
+    d_C = D.DeviceArray.zeros(a.nr * nv)
+    need = m.workspace_size(nv, btype=bt)
+    ms = [min(m.benchmark(d_B, d_C, nv, btype=bt, config=c, warmup=2, reps=5, per_call=False)[0] for _ in range(3))
+          for c in (None, D.make_config(D.VARIANT_NNZ_TILED))]
+    note(f"{a.nnz} nonzeros, workspace {need / MIB:.0f} MiB: AUTO {ms[0]:.3f} ms, 16 per lane {ms[1]:.3f} ms")
+    assert need > 64 * MIB and ms[0] <= 1.05 * ms[1]
+    m.close()
