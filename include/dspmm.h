@@ -331,7 +331,7 @@ typedef struct dspmm_config {
 /* C = A * B, overwriting C (nv columns; ldb/ldc in elements, >= nv for
  * row-major, >= nc / nr for column-major).  btype selects FP32 or BF16 B
  * storage; accumulation is always FP32.  cfg may be NULL (auto).  The
- * row-major kernels (NNZ_TILED, ROW_BLOCKED, NNZ_CACHED and the
+ * row-major kernels (NNZ_TILED, ROW_BLOCKED, NNZ_CACHED, CSR_PARTS and the
  * row-sequential CSR_SCALAR) take column-major operands through transposed
  * copies of B and C (results equal the row-major call's bit for bit); the
  * reference classes run column-major natively, FP32 only.  `workspace` may

@@ -125,3 +125,29 @@ def test_a_matrix_takes_the_scratch_back():
     c64, ab = O.spmm_fp64(RM, a.nr, a.nc, 1, a.rowPtr, a.colIdx, a.values, x)
     assert_fp32(d_y.numpy(), c64.reshape(-1), ab.reshape(-1), np.diff(a.rowPtr).astype(np.float64),
                 "tiles", h32)
+
+
+@pytest.mark.parametrize("nr,n,slices", [(64, 8, True), (63, 16, True), (128, 32, True), (1, 40, False), (65, 8, False),
+                                         (64, 33, False)])
+def test_which_bands_go_in_slices(nr, n, slices):
+    """One slice and two, and what keeps a band out of them: padding, long rows.
+    The path shows in the plan's bytes."""
+    col = (np.arange(nr)[:, None] + 2 * np.arange(n)).astype(np.int32)
+    rng = np.random.default_rng(n)
+    val = rng.uniform(-1, 1, (nr, n)).astype(np.float32)
+    x = rng.uniform(-1, 1, nr + 2 * n).astype(np.float32)
+    rp = (np.arange(nr + 1) * n).astype(np.int32)
+    m = D.Matrix(nr, x.size, rp, col.reshape(-1), val.reshape(-1))
+    d_x, d_y = D.DeviceArray.from_numpy(x), D.DeviceArray.from_numpy(np.full(nr, np.nan, np.float32))
+    before = m.describe()["hbm_bytes"]
+    m.spmm(d_x, d_y, 1)
+    D.synchronize()
+    grown = m.describe()["hbm_bytes"] - before
+    assert (grown >= 5 * nr * n) == slices, f"plan of {grown} bytes"
+    h32 = O.spmm_host32(RM, nr, x.size, 1, rp, col.reshape(-1), val.reshape(-1), x).reshape(-1)
+    c64, ab = O.spmm_fp64(RM, nr, x.size, 1, rp, col.reshape(-1), val.reshape(-1), x)
+    if n <= 16:
+        assert np.array_equal(d_y.numpy(), h32)
+    else:
+        assert_fp32(d_y.numpy(), c64.reshape(-1), ab.reshape(-1), np.full(nr, n, np.float64), "band", h32)
+    m.close()
