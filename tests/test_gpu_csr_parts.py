@@ -1,6 +1,8 @@
 """CSR_PARTS: a row's products four at a time, these in two sums in turn.  The
 edges of both kernels (by wavefronts, by blocks) against 64 bits, whole
 numbers exactly, and what the variant refuses."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -76,4 +78,28 @@ def test_refused():
     for cfg in (dict(unroll=4), dict(unroll=3), dict(tile_nnz=2, unroll=8)):
         with pytest.raises(D.DspmmError):
             m.spmm(d_B, d_C, 8, config=D.make_config(D.VARIANT_CSR_PARTS, **cfg))
+    m.close()
+
+
+@pytest.mark.parametrize("layout", [RM, CM])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_without_allocation(layout, bf16):
+    """Prepared, it runs in the no-alloc call too, with the same bits."""
+    nr, nc, nv = 1500, 900, 24
+    ptr, col, val = rows(np.random.default_rng(2).integers(0, 90, nr), nc)
+    m = D.Matrix(nr, nc, ptr, col, val)
+    bt = D.DSPMM_R_16BF if bf16 else D.DSPMM_R_32F
+    d_B = D.DeviceArray.from_numpy(np.random.default_rng(3).uniform(-1, 1, nc * nv).astype(np.float32))
+    d_B = D.to_bf16_device(d_B) if bf16 else d_B
+    out = [D.DeviceArray.from_numpy(np.full(nr * nv, np.nan, np.float32)) for _ in range(2)]
+    cfg = D.make_config(D.VARIANT_CSR_PARTS)
+    m.spmm(d_B, out[0], nv, layout, btype=bt, config=cfg)
+    m.prepare(d_B, out[1], nv, layout, btype=bt, config=cfg)
+    ld = (nv, nv) if layout == RM else (nc, nr)
+    st = D.lib().dspmm_spmm_ex_noalloc(m.handle, layout, nv, d_B.ptr, ld[0], bt, out[1].ptr, ld[1],
+                                       C.byref(cfg), None)
+    assert st == 0, D.status_string(st)
+    D.synchronize()
+    a, b = out[0].numpy(), out[1].numpy()
+    assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
     m.close()
