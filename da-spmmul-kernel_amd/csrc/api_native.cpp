@@ -530,13 +530,10 @@ constexpr int64_t kTransposedMinWork = 1 << 20;
 // never pay: 157000 rows of 35, nv = 3 69 / 134; 90^3 stencil, nv = 2 65 / 474.
 constexpr int64_t kInPlaceWork = 5500000;
 
-// Fills the tile size of a single nnz-tiled launch: at most `cap`, and small
-// enough that the launch has kTileWaves wavefronts (a wavefront owns 64 /
-// lanes tiles).  Power law, 262144 rows, BF16 B: nv = 32 and 16 per tile
-// 74 us, 64 142; nv = 128 and 32 per tile 160 us, 256 442 (3100 wavefronts
-// of long serial tiles).  A batch sizes its items' tiles by other rules: they
-// share the GPU.
+// Wavefronts that a single nnz-tiled launch asks of its tiles.
 constexpr int kTileWaves = 2048;
+
+// The next longer tile; false if there is none.
 bool longer_tiles(int nv, bool bf16, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
@@ -552,6 +549,7 @@ bool longer_tiles(int nv, bool bf16, dspmm_config &c) {
     }
     return true;
 }
+
 // AUTO's tiles within dspmm_spmm_ex_noalloc's scratch: grown, where they need
 // more, until their carries (and the transposed copies) fit.
 dspmm_config noalloc_tiles(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, dspmm_config c) {
@@ -563,18 +561,21 @@ dspmm_config noalloc_tiles(const dspmm_matrix_s *A, bool rm, int nv, bool bf16, 
         if (!longer_tiles(nv, bf16, c)) return as_is;
     return c;
 }
+
 // Halves the tile until the launch's LDS fits.
 void fit_tile(int nv, bool bf16, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
     while (nnz_tiled_lds_bytes(full.lanes, c.tile_nnz) > kMaxTileLds) c.tile_nnz /= 2;
 }
+
 // The tile of 16 nonzeros per lane, at vectors that divide nv: its order of
 // summation is the one that AUTO's may not fall behind in accuracy.
 int plain_tile(int nv, bool bf16) {
     const int vw = choose_vw(nv, nv, nv, nullptr, nullptr, bf16 ? 2 : 4, bf16 ? 8 : 4);
     return default_tile(std::min(64, pow2_ceil(div_up(nv, vw))));
 }
+
 // The longest chain of additions in a row of n nonzeros cut at S (k_split_combine
 // adds the chunks in up to 64 / nv parts).
 int64_t tile_chain(int64_t n, int S, int nv) {
@@ -582,6 +583,13 @@ int64_t tile_chain(int64_t n, int S, int nv) {
     const int64_t parts = 64 / std::min(64, pow2_ceil(nv)), chunks = (n + S - 1) / S;
     return S + (chunks + parts - 1) / parts + parts;
 }
+
+// Fills the tile size of a single nnz-tiled launch: `cap` if longer than what the
+// lanes have, and small enough that the launch has kTileWaves wavefronts (a wavefront
+// owns 64 / lanes tiles).  Power law, 262144 rows, BF16 B: nv = 32 and 16 per tile
+// 74 us, 64 142; nv = 128 and 32 per tile 160 us, 256 442 (3100 wavefronts
+// of long serial tiles).  A batch sizes its items' tiles by other rules: they
+// share the GPU.
 void single_tile(const dspmm_matrix_s *A, int nv, bool bf16, int cap, dspmm_config &c) {
     dspmm_config full = c;
     complete_nb(full, nv, bf16);
@@ -1132,7 +1140,7 @@ dspmm_status_t run_ex(dspmm_matrix_s *A, DenseLayout layout, int nv, const void 
         // (60^3 stencil, nv = 12: 31 us by wavefronts, 24 by blocks)
         const bool staged = parts && !bf16 && cfg.unroll <= 0 && nv >= 5 && nv <= 32;
         if ((parts && !staged) || (cfg.variant == DSPMM_VARIANT_CSR_SCALAR && layout == DENSE_ROW_MAJOR &&
-                      (bf16 || cfg.unroll > 0))) {
+                                   (bf16 || cfg.unroll > 0))) {
             dspmm_config c = cfg;
             if (cfg.tile_nnz != 0 && cfg.tile_nnz != 1) return DSPMM_STATUS_NOT_SUPPORTED;
             c.tile_nnz = 0;

@@ -457,7 +457,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_scalar_rm(int nr, int nv, int64_
         }
     };
     int nlong = 0;
-    if (!PARTS && be - bs >= kLongRow) {                 // the same in every thread
+    if (!PARTS && be - bs >= kLongRow) {       // the same in every thread
         if (threadIdx.x == 0) s_nlong = 0;
         __syncthreads();
         if (threadIdx.x % L == 0 && apart(end - start)) s_long[atomicAdd(&s_nlong, 1)] = r;
