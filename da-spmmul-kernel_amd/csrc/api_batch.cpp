@@ -47,6 +47,7 @@ constexpr int kBatchSlab = 64;
 // 96 mixed items of 16 columns 142 / 165; per 60 KB (128 items of mixed widths) 1059 / 1462.
 constexpr double kBatchSplit = 2048;
 constexpr double kBatchSplitAll = 10000;
+constexpr double kBatchLongMean = 128;         // 8 + n / 8 additions are more than 16 + n / 16
 
 // Bytes that an item moves, roughly.
 static double item_cost(const dspmm_matrix_s *A, int nv, bool bf16) {
@@ -74,7 +75,13 @@ struct ItemTiles {
 static ItemTiles item_tiles(const dspmm_matrix_s *A, int nv, bool bf16) {
     ItemTiles t;
     t.brief = t.whole = item_config(A, nv, bf16, 0);
-    t.brief.tile_nnz = std::max(8, std::min(kBatchTile, (bf16 ? kBatchPairsBf16 : kBatchPairs) * t.brief.lanes / kWave));
+    // up to two columns the combine adds a row's chunks one after the other: long
+    // rows' many chunks of 8 are a longer chain than half as many of 16 (rows of 256,
+    // nv = 2: error 1.24e-7 of the result's norm / 1.12e-7)
+    const bool longer = nv <= 2 && !bf16 && A->mean > kBatchLongMean;
+    if (longer) t.brief = item_config(A, nv, bf16, 1);
+    t.brief.tile_nnz = std::max(longer ? 16 : 8,
+                                std::min(kBatchTile, (bf16 ? kBatchPairsBf16 : kBatchPairs) * t.brief.lanes / kWave));
     const int least = choose_vw(nv, nv, nv, nullptr, nullptr, bf16 ? 2 : 4, bf16 ? 8 : 4);
     while (default_tile(t.whole.lanes) < A->max_len && t.whole.vec > least)
         t.whole = item_config(A, nv, bf16, t.whole.vec / 2);

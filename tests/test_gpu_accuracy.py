@@ -258,3 +258,39 @@ def test_spmv_coo(fn, n):
     got, ref = error(out.numpy(), exact), error(scanned(val * x[col], row, nr), exact)
     note(f"{fn} rows of {n}: {got:.3g}, chunk by chunk {ref:.3g}")
     assert got <= MARGIN * ref
+
+
+@pytest.mark.parametrize("bf16,nv", [(False, 1), (False, 2), (False, 4), (True, 1), (True, 8)])
+def test_batch_long_rows(bf16, nv):
+    """A narrow item of a batch: no worse than chunks of 16 added in order, in
+    as many parts as lanes of a wavefront share a column."""
+    m = Rows(4000, 256, 3000, nv)
+    d_B = D.DeviceArray.from_numpy(m.B)
+    if bf16:
+        d_B = D.to_bf16_device(d_B)
+        m.B = (((m.B.view(np.uint32) + 0x7fff + ((m.B.view(np.uint32) >> 16) & 1)) >> 16) << 16).view(F)
+    a, b = m.operands(nv, nv)
+    exact = m.exact(a, b)
+    out = D.DeviceArray.from_numpy(np.full((m.nr, nv), np.nan, F))
+    h = D.Matrix(m.nr, m.nc, m.ptr, m.col.reshape(-1), m.val.reshape(-1))
+    batch = D.Batch([(h, nv, d_B, out)], btype=D.DSPMM_R_16BF if bf16 else D.DSPMM_R_32F)
+    batch.run()
+    D.synchronize()
+    prod, parts, each = a * b, 64 // max(1, nv), []
+    for c in range(0, 256, 16):
+        t = np.zeros(prod.shape[:-1], F)
+        for i in range(c, c + 16):
+            t = t + prod[..., i]
+        each.append(t)
+    per = -(-len(each) // parts)
+    ref = np.zeros_like(each[0])
+    for p in range(0, len(each), per):
+        t = np.zeros_like(ref)
+        for c in each[p:p + per]:
+            t = t + c
+        ref = ref + t
+    got, ref = error(out.numpy(), exact), error(ref, exact)
+    note(f"{'bf16' if bf16 else 'fp32'} batch, rows of 256, nv={nv}: {got:.3g}, chunks of 16 {ref:.3g}")
+    assert got <= MARGIN * ref
+    batch.close()
+    h.close()
